@@ -54,7 +54,8 @@ struct PathBuffers {
     DeviceArray<float4> sampleRad;
     DeviceArray<float4> nrcQuery, nrcRecord, nrcTarget;  // neural cache queries, training records, targets
     DeviceArray<uint8_t> sortKey;                         // material class of every queued ray
-    DeviceArray<uint32_t> sortPerm, sortCount, sortOffset;  // shading order, per-block counts, their scan
+    DeviceArray<uint32_t> sortPerm;                       // shading order
+    DeviceArray<uint64_t> sortCount, sortOffset;          // rays of each class per block, their scan
     DeviceArray<uint8_t> sortScratch;                     // rocPRIM scan temporary storage
     // denoiser features per path (only while feature images or debug views are on):
     // state bit 0 = resolved, bit 1 = followed a specular hit at depth 0;

@@ -45,23 +45,37 @@ constexpr uint64_t kMaxChunk = 1ull << 27;
 constexpr int kBlock = 256;
 
 // counters[] layout
-constexpr int kCntQueue0 = 0, kCntQueue1 = 1, kCntShadow = 2, kCntShadowEnv = 3, kCntNrcQuery = 4, kCntDropped = 5,
-              kCntNrcRecord = 6, kCntNrcTrain = 7,
+constexpr int kCntNrcQuery = 4, kCntDropped = 5, kCntNrcRecord = 6, kCntNrcTrain = 7,
               kCntStats = 8;  // 64-bit stats at counters+8: [0] ext rays, [1] shadow rays, [2] nodes, [3] triangles,
                               // [4] rays of the fused tail, [5..7] [0], [2], [3] as they stood when the tail began
 // queue length of every depth (the first kDepthHist depths) and the fused tail's claim counter
 constexpr int kCntDepthHist = 24, kDepthHist = 32, kCntTailFetch = kCntDepthHist + kDepthHist;
-// Work claims of the persistent traversal kernels. The batch space of a queue
-// is split into kFetchParts interleaved partitions, each with its own counter
-// on its own 256-byte line: device-scope atomics from the 8 XCDs then spread
-// over 8 addresses instead of serialising on one. A wave claims kFetchBatch
-// rays per atomic.
-constexpr int kFetchParts = 8;
-constexpr uint32_t kFetchStride = 64;  // uint32 slots between partition counters
-constexpr uint32_t kFetchBatch = 64;
-constexpr int kCntFetchExt = 64, kCntFetchShadow = kCntFetchExt + kFetchParts * kFetchStride,
-              kCntFetchShadowEnv = kCntFetchShadow + kFetchParts * kFetchStride;
-constexpr uint32_t kCounterWords = kCntFetchShadowEnv + kFetchParts * kFetchStride;
+// A queue is kQueueParts parts, each with its own length and its own claim
+// counter on a 256-byte line of their own. A block of kShade reads and appends
+// to part blockIdx % kQueueParts, which is also the XCD it runs on (workgroups
+// go to the 8 XCDs in turn), so an append is an atomic on a line that one XCD
+// alone is using. One length for the whole queue is what bounded the shading
+// kernels of scenes whose paths go on: all wavefronts added to one address, at
+// about 11.4 ns each whatever they shaded (1024x1024, 16 spp Cornell box: 21.2 ms
+// of shading per frame, 5.9 with parts).
+constexpr int kQueueParts = 8;
+constexpr uint32_t kPartStride = 64;  // uint32 slots between the counters of two parts
+constexpr uint32_t kFetchBatch = 64;  // shadow rays a wavefront claims per atomic
+constexpr int kPartWords = kQueueParts * (int)kPartStride;
+constexpr int kCntFetchExt = 64, kCntFetchShadow = kCntFetchExt + kPartWords,
+              kCntFetchShadowEnv = kCntFetchShadow + kPartWords, kCntQueue0 = kCntFetchShadowEnv + kPartWords,
+              kCntQueue1 = kCntQueue0 + kPartWords, kCntShadow = kCntQueue1 + kPartWords,
+              kCntShadowEnv = kCntShadow + kPartWords;
+constexpr uint32_t kCounterWords = kCntShadowEnv + kPartWords;
+
+// Blocks of a queue of up to n paths, a whole number for every part: block b of
+// the slots is block b / kQueueParts of part b % kQueueParts. Slots are dealt in
+// blocks and not in eighths of the queue, whose parts would lie a power of two
+// apart and meet in the same memory channels (shading of the 1080p spectral
+// workload 27.2 against 26.0 ms); strips of 64 blocks instead of one changed nothing.
+__host__ __device__ inline uint32_t queueBlocks(uint64_t n) {
+    return (uint32_t)((n + (uint64_t)kBlock * kQueueParts - 1u) / ((uint64_t)kBlock * kQueueParts)) * kQueueParts;
+}
 
 struct FrameParams {
     SceneData sd;
@@ -120,8 +134,20 @@ struct PathView {
 struct QueueView {
     float4* o;
     float4* d;
-    uint32_t* count;
+    uint32_t* count;  // length of part p at count[p * kPartStride]
 };
+
+// Rays in all parts of a queue.
+DEV uint32_t queueTotal(const uint32_t* count) {
+    uint32_t n = 0;
+#pragma unroll
+    for (int p = 0; p < kQueueParts; p++) n += count[p * kPartStride];
+    return n;
+}
+// Slot of entry j of a part. The primary ray of path i is in slot i.
+DEV uint32_t queueSlot(uint32_t part, uint32_t j) {
+    return (j / kBlock) * (kBlock * kQueueParts) + part * kBlock + j % kBlock;
+}
 
 struct ShadowView {
     float4 *o, *d, *a, *b;
@@ -153,14 +179,21 @@ DEV uint32_t waveAppend(bool pred, uint32_t* counter) {
     return pred ? base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull)) : 0xFFFFFFFFu;
 }
 
-// First ray of the next batch of this wave's partition, or >= n once the
-// partition is exhausted. Wave-uniform; every lane must call it.
-DEV uint32_t claimBatch(uint32_t* fetchBase, uint32_t part, uint32_t n) {
-    uint32_t k = 0;
-    if ((threadIdx.x & 63u) == 0u) k = atomicAdd(&fetchBase[part * kFetchStride], 1u);
-    k = (uint32_t)__shfl((int)k, 0);
-    uint64_t first = ((uint64_t)k * kFetchParts + part) * kFetchBatch;
-    return first >= n ? n : (uint32_t)first;
+// First of the next `claim` rays of a part of partLen rays, or partLen or more
+// once the part is used up. Wave-uniform; every lane must be active. `look`:
+// read the counter first, for the parts that a wavefront turns to when its own
+// is used up: at the end of a launch every wavefront asks every part, and an
+// atomic on a used-up part waits in line with those of all the others. (Looking before
+// every claim was slower by far: 6.9 against 2.5 ms of shadow rays in the
+// 1024x1024 Cornell box, the line being in other hands whenever it is read.)
+DEV uint32_t claimRays(uint32_t* counter, uint32_t partLen, uint32_t claim, bool look) {
+    uint32_t base = 0;
+    if (look) {
+        base = __builtin_amdgcn_readfirstlane(__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (base >= partLen) return base;
+    }
+    if ((threadIdx.x & 63u) == 0u) base = atomicAdd(counter, claim);
+    return __builtin_amdgcn_readfirstlane(base);
 }
 
 // ------------------------------------------------------------ lights --
@@ -443,24 +476,43 @@ DEV F3 cameraOrigin(const SceneData& sd) {
     return F3{org.x, org.y, org.z};
 }
 
-__global__ void kPrepDepth(uint32_t* counters, int cur, int nxt, uint32_t depth) {
+// Before each depth: the rays about to be traced and the shadow rays of the
+// depth before are counted, and the counters this depth appends to and claims
+// from start at 0.
+__global__ __launch_bounds__(64) void kPrepDepth(uint32_t* counters, int cur, int nxt, uint32_t depth) {
     const uint32_t t = threadIdx.x;
     if (t == 0) {
         unsigned long long* stats = reinterpret_cast<unsigned long long*>(counters + kCntStats);
-        stats[0] += counters[cur];
-        if (depth < (uint32_t)kDepthHist) counters[kCntDepthHist + depth] = counters[cur];
-        counters[nxt] = 0u;
-        counters[kCntShadow] = 0u;
-        counters[kCntShadowEnv] = 0u;
+        const uint32_t n = queueTotal(counters + cur);
+        stats[0] += n;
+        stats[1] += queueTotal(counters + kCntShadow) + queueTotal(counters + kCntShadowEnv);
+        if (depth < (uint32_t)kDepthHist) counters[kCntDepthHist + depth] = n;
         counters[kCntTailFetch] = 0u;
     }
-    if (t < 3u * kFetchParts) counters[kCntFetchExt + t * kFetchStride] = 0u;
+    __syncthreads();
+    if (t < (uint32_t)kQueueParts) {
+        counters[nxt + t * kPartStride] = 0u;
+        counters[kCntShadow + t * kPartStride] = 0u;
+        counters[kCntShadowEnv + t * kPartStride] = 0u;
+    }
+    if (t < 3u * kQueueParts) counters[kCntFetchExt + t * kPartStride] = 0u;
 }
-__global__ void kPrepShadow(uint32_t* counters) {
+// After the last depth: its shadow rays.
+__global__ void kCountShadow(uint32_t* counters) {
     unsigned long long* stats = reinterpret_cast<unsigned long long*>(counters + kCntStats);
-    stats[1] += counters[kCntShadow] + counters[kCntShadowEnv];
+    stats[1] += queueTotal(counters + kCntShadow) + queueTotal(counters + kCntShadowEnv);
 }
-__global__ void kSetCount(uint32_t* counters, int slot, uint32_t value) { counters[slot] = value; }
+// Part lengths of the queue of a chunk's n primary rays; no shadow rays yet.
+__global__ __launch_bounds__(64) void kBeginQueue(uint32_t* counters, uint32_t n) {
+    const uint32_t p = threadIdx.x;
+    if (p >= (uint32_t)kQueueParts) return;
+    constexpr uint32_t kRound = kBlock * kQueueParts;
+    const uint32_t last = n % kRound;  // paths of the last, partial round of blocks
+    const uint32_t len = n / kRound * kBlock + min(last > p * kBlock ? last - p * kBlock : 0u, (uint32_t)kBlock);
+    counters[kCntQueue0 + p * kPartStride] = len;
+    counters[kCntShadow + p * kPartStride] = 0u;
+    counters[kCntShadowEnv + p * kPartStride] = 0u;
+}
 // The ray and traversal totals as they stand before the depth the fused tail takes over.
 __global__ void kTailSnapshot(uint32_t* counters) {
     unsigned long long* stats = reinterpret_cast<unsigned long long*>(counters + kCntStats);
@@ -471,21 +523,28 @@ __global__ void kTailSnapshot(uint32_t* counters) {
 
 // Closest-hit traversal, persistent with lane refill. Every loop iteration
 // advances each busy lane by one node or leaf visit; once kRefillLanes lanes of
-// a wavefront are idle, the wavefront claims that many new rays with one atomic,
-// so lanes do not wait for the slowest ray of a batch. The queue is split into
-// kFetchParts contiguous partitions, each with its own claim counter (its own
-// 256-byte line); a wavefront starts in the partition of its block and moves on
-// to the next partition once one is exhausted.
+// a wavefront are idle they take new rays, so lanes do not wait for the slowest
+// ray of a batch. A wavefront claims the rays in runs of up to kClaimMax (about a
+// quarter of its share of a short queue) and hands them out itself; one atomic per
+// refill made the wavefronts of a scene of few triangles wait for the claim
+// counters (1024x1024 Cornell box, 16 spp: 4.54 ms of traversal, 3.15 in runs). A
+// wavefront starts in the queue part of its block's XCD and moves on to the next part
+// once one is used up. What bounds it in scenes of many triangles is the latency of
+// the node loads: letting lanes with a leaf wait until 8, 16 or 24 of them could test
+// their triangles together halved the leaf steps and still took 23.2, 23.0 and 24.2
+// against 22.0 ms per 1080p spectral frame.
 // COUNT adds the number of BVH nodes visited and triangles tested to the frame statistics.
 constexpr uint32_t kRefillLanes = 16;
+constexpr uint32_t kClaimMax = 256;
 constexpr uint32_t kNoRay = 0xFFFFFFFFu;
 
 // ALPHA: some mesh runs the alpha test (the opaque variant keeps six waves per SIMD);
 // TEXA: some material has textures, so the test may read a texture's alpha.
 template <bool COUNT, bool ALPHA, bool TEXA = false>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEXA ? 4 : 6))) void kExtend(SceneView sv, const float4* ro, const float4* rd, float4* hits,
-                                                      uint32_t* counters, int countSlot, uint32_t* gstack,
-                                                      uint32_t alphaSalt, uint32_t pathBase, float4 camO) {
+                                                      uint32_t* counters, const uint32_t* count,
+                                                      uint32_t* gstack, uint32_t alphaSalt, uint32_t pathBase,
+                                                      float4 camO) {
     // camO.w != 0: the queue holds primary rays without stored origins; camO.xyz is theirs
     uint32_t nodeVisits = 0, triTests = 0;
     __shared__ uint32_t lds[kLdsStackWords];
@@ -494,23 +553,29 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
     st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
     st.dropped = 0;
     st.sp = 0;
-    const uint32_t n = counters[countSlot];
+    const uint32_t n = queueTotal(count);
     if (n == 0u || sv.nodeCount == 0u) {
         // empty queue, or no geometry: every ray misses
-        for (uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x; i < n; i += gridDim.x * kTraceBlock)
-            hits[i] = make_float4(rd[i].w, __uint_as_float(kNoHit), 0.0f, 0.0f);
+        for (uint32_t p = 0; p < (uint32_t)kQueueParts; p++)
+            for (uint32_t j = blockIdx.x * kTraceBlock + threadIdx.x; j < count[p * kPartStride];
+                 j += gridDim.x * kTraceBlock) {
+                const uint32_t i = queueSlot(p, j);
+                hits[i] = make_float4(rd[i].w, __uint_as_float(kNoHit), 0.0f, 0.0f);
+            }
         return;
     }
     // Wavefronts beyond one per 64 queued rays leave at once: every ray still
-    // has a wavefront to claim it (each wavefront drains all partitions), and a
-    // short queue does not pay kFetchParts contended claims in every resident
+    // has a wavefront to claim it (each wavefront drains all parts), and a
+    // short queue does not pay kQueueParts contended claims in every resident
     // wavefront (about 100 us per launch with the full grid).
     if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lanesBelow = (1ull << lane) - 1ull;
-    const uint32_t partSize = (n + kFetchParts - 1u) / kFetchParts;
-    uint32_t part = blockIdx.x % kFetchParts;
-    uint32_t partsTried = 0;  // partitions found exhausted by this wavefront
+    uint32_t part = blockIdx.x % kQueueParts;
+    uint32_t partsTried = 0;  // parts found exhausted by this wavefront
+    // rays [poolNext, poolEnd) of part poolPart are this wavefront's to hand out
+    uint32_t poolNext = 0, poolEnd = 0, poolPart = part;
+    const uint32_t claim = min(max(n / (gridDim.x * (kTraceBlock / 64u) * 4u), 64u), kClaimMax);
     uint32_t rayId = kNoRay, alphaKey = 0u;
     TraversalRay r;
     ClosestState cs;
@@ -522,15 +587,24 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
     while (true) {
         const uint64_t idleMask = __ballot(rayId == kNoRay);
         const uint32_t idle = (uint32_t)__popcll(idleMask);
-        if (partsTried < kFetchParts && (idle >= kRefillLanes || idle == 64u)) {
-            // claim `idle` rays of the current partition; lanes beyond its end stay idle
-            uint32_t base = 0;
-            if (lane == 0u) base = atomicAdd(&counters[kCntFetchExt + part * kFetchStride], idle);
-            base = (uint32_t)__shfl((int)base, 0);
-            const uint32_t begin = part * partSize, end = min(n, begin + partSize);
+        if (idle >= kRefillLanes && (partsTried < kQueueParts || poolNext < poolEnd)) {
+            if (poolNext >= poolEnd) {
+                const uint32_t partLen = __builtin_amdgcn_readfirstlane(count[part * kPartStride]);
+                const uint32_t base = claimRays(&counters[kCntFetchExt + part * kPartStride], partLen, claim,
+                                                partsTried > 0u);
+                poolPart = part;
+                poolNext = base;
+                poolEnd = min(base + claim, partLen);
+                if (base + claim >= partLen) {  // this part is used up
+                    part = (part + 1u) % kQueueParts;
+                    partsTried++;
+                }
+            }
+            const uint32_t first = poolNext;
+            poolNext = min(poolNext + idle, max(poolNext, poolEnd));
             if (rayId == kNoRay) {
-                const uint32_t k = begin + base + (uint32_t)__popcll(idleMask & lanesBelow);
-                if (base < partSize && k < end) {
+                const uint32_t j = first + (uint32_t)__popcll(idleMask & lanesBelow), k = queueSlot(poolPart, j);
+                if (j < poolEnd) {
                     float4 a = camO.w != 0.0f ? make_float4(camO.x, camO.y, camO.z, __uint_as_float(k)) : ro[k];
                     float4 b = rd[k];
                     r = makeTraversalRay(xyz(a), xyz(b));
@@ -543,10 +617,6 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
                     }
                 }
             }
-            if (base + idle >= partSize) {  // wave-uniform: this partition is used up
-                part = (part + 1u) % kFetchParts;
-                partsTried++;
-            }
         }
         if (rayId != kNoRay) {
             if (!closestStep<ALPHA, TEXA>(sv, r, kRayTMin, cs, st, alphaKey, COUNT ? &nodeVisits : nullptr,
@@ -554,11 +624,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
                 hits[rayId] = make_float4(cs.h.t, __uint_as_float(cs.h.tri), cs.h.u, cs.h.v);
                 rayId = kNoRay;
             }
-        } else if (partsTried >= kFetchParts) {
-            // nothing left to claim; this lane is done, but the wavefront keeps
-            // iterating until every lane has finished its ray
         }
-        if (partsTried >= kFetchParts && __ballot(rayId != kNoRay) == 0ull) break;
+        // nothing left to claim: the wavefront goes on until every lane has finished its ray
+        if (partsTried >= kQueueParts && poolNext >= poolEnd && __ballot(rayId != kNoRay) == 0ull) break;
     }
     if (st.dropped) atomicAdd(&counters[kCntDropped], st.dropped);
     if (COUNT) {
@@ -582,28 +650,27 @@ DEV uint32_t classifyOccluder(const SceneView& sv, uint32_t tri) {
 // or not.
 template <int MODE>
 __global__ __launch_bounds__(kTraceBlock) void kShadow(SceneView sv, PathView pv, ShadowView sh, uint32_t* counters,
-                                                      int countSlot, int fetchSlot, uint32_t envPass,
+                                                      int fetchSlot, uint32_t envPass,
                                                       uint32_t* gstack, uint32_t alphaSalt, uint32_t pathBase) {
     __shared__ uint32_t lds[kLdsStackWords];
     TraversalStack st;
     st.lds = lds + threadIdx.x;
     st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
     st.dropped = 0;
-    const uint32_t n = counters[countSlot];
-    if (n == 0u) return;
-    // A wavefront claims batches of its block's partition only, and partition p
-    // holds batches p, p + kFetchParts, ...: keep the wavefronts whose rank within
-    // their partition is below that partition's batch count (rank 0 always), so
-    // short queues do not pay a contended claim in every resident wavefront.
-    const uint32_t rank = (blockIdx.x / kFetchParts) * (kTraceBlock / 64u) + (threadIdx.x >> 6);
-    if ((uint64_t)rank * kFetchBatch * kFetchParts >= n) return;
+    const uint32_t n = queueTotal(sh.count);
+    // wavefronts beyond one per batch leave at once (see kExtend)
+    if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * (uint64_t)kFetchBatch >= n) return;
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t part = blockIdx.x % kFetchParts;
-    while (true) {
-        const uint32_t base = claimBatch(counters + fetchSlot, part, n);
-        if (base >= n) break;
-        uint32_t i = base + lane;
-        if (i >= n) continue;
+    uint32_t part = blockIdx.x % kQueueParts, partsTried = 0;
+    while (partsTried < (uint32_t)kQueueParts) {
+        // a batch of the current part, or the next part once that one is used up
+        const uint32_t partLen = sh.count[part * kPartStride];
+        const uint32_t base = claimRays(&counters[fetchSlot + part * kPartStride], partLen, kFetchBatch, partsTried > 0u), j = base + lane, i = queueSlot(part, j);
+        if (base + kFetchBatch >= partLen) {
+            part = (part + 1u) % kQueueParts;
+            partsTried++;
+        }
+        if (j >= partLen) continue;
         float4 o = sh.o[i], d = sh.d[i];
         uint32_t q = __float_as_uint(o.w);
         TraversalRay r = makeTraversalRay(xyz(o), xyz(d));
@@ -699,12 +766,13 @@ __global__ __launch_bounds__(kBlock) void kNrcTargets(const float4* record, cons
 // layer does not fit the three-wave budget of the hero kernel.
 // One path vertex: the ray (ro, rdir) of path q = bits of ro.w, at `depth`,
 // and its hit h. Leaves the continuation ray in nextO / nextD with cont set, or
-// cont false when the path ends here. Shadow and cache records are appended to
-// their queues by whichever lanes of the wave reach the append.
+// cont false when the path ends here. Shadow records go to the part `part` (one
+// for the wave) of their queues, cache records to theirs, by whichever lanes
+// of the wave reach the append.
 template <int MODE, bool NRC, bool TEX, bool SHEEN>
 DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv, const PathView& pv, float4 ro,
-                     float4 rdir, Hit h, const ShadowView& sh, const ShadowView& she, uint32_t* counters,
-                     const NrcView& nv, bool& cont, F3& nextO, F3& nextD) {
+                     float4 rdir, Hit h, const ShadowView& sh, const ShadowView& she, uint32_t part,
+                     uint32_t* counters, const NrcView& nv, bool& cont, F3& nextO, F3& nextD) {
     bool shadowEmit = false, envEmit = false;
     F3 shO = f3(0.0f), shD = f3(0.0f), seO = f3(0.0f), seD = f3(0.0f);
     float shT = 0.0f;
@@ -980,14 +1048,14 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
         // so they are not held in registers through BSDF sampling (waveAppend works
         // on whichever lanes are still active).
         {
-            const uint32_t sslot = waveAppend(shadowEmit, &counters[kCntShadow]);
+            const uint32_t sslot = queueSlot(part, waveAppend(shadowEmit, &sh.count[part * kPartStride]));
             if (shadowEmit) {
                 sh.o[sslot] = make_float4(shO.x, shO.y, shO.z, __uint_as_float(q));
                 sh.d[sslot] = make_float4(shD.x, shD.y, shD.z, shT);
                 sh.a[sslot] = st4(shA);
                 sh.b[sslot] = st4(shB);
             }
-            const uint32_t eslot = waveAppend(envEmit, &counters[kCntShadowEnv]);
+            const uint32_t eslot = queueSlot(part, waveAppend(envEmit, &she.count[part * kPartStride]));
             if (envEmit) {
                 she.o[eslot] = make_float4(seO.x, seO.y, seO.z, __uint_as_float(q));
                 she.d[eslot] = make_float4(seD.x, seD.y, seD.z, kRayTMax);
@@ -1123,28 +1191,34 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
 template <int MODE, bool NRC = false, bool TEX = false, bool SHEEN = false>
 __global__ __launch_bounds__(kBlock, SHEEN ? 2 : 3) void kShade(FrameParams fp, SceneView sv, PathView pv, QueueView in,
                                                  const float4* hits, QueueView out, ShadowView sh, ShadowView she,
-                                                 uint32_t* counters, int inSlot, int outSlot, NrcView nv,
-                                                 const uint32_t* __restrict__ order) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t n = counters[inSlot];
+                                                 uint32_t* counters, NrcView nv, const uint32_t* __restrict__ order) {
+    const uint32_t part = blockIdx.x % kQueueParts;
     bool cont = false;
     F3 nextO = f3(0.0f), nextD = f3(0.0f);
     uint32_t q = 0;
-    if (i < n) {
-        const uint32_t j = order ? order[i] : i;  // shading order (sorted by material class) or queue order
-        // depth 0 of a compact frame: the ray's origin is the camera's, its path index its queue slot
+    const uint32_t j = (blockIdx.x / kQueueParts) * kBlock + threadIdx.x;
+    uint32_t slot = queueSlot(part, j);
+    bool valid = j < in.count[part * kPartStride];
+    if (order) {  // sorted by material class: the queue's rays, dense over the grid
+        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+        valid = i < queueTotal(in.count);
+        if (valid) slot = order[i];
+    }
+    if (valid) {
+        // depth 0 of a compact frame: the ray's origin is the camera's
         F3 co = f3(0.0f);
         if (fp.compactPrimary && fp.depth == 0u) co = cameraOrigin(fp.sd);
-        const float4 ro = fp.compactPrimary && fp.depth == 0u ? make_float4(co.x, co.y, co.z, __uint_as_float(j)) : in.o[j];
-        const float4 rdir = in.d[j], hh = hits[j];
+        const float4 ro = fp.compactPrimary && fp.depth == 0u ? make_float4(co.x, co.y, co.z, __uint_as_float(slot))
+                                                              : in.o[slot];
+        const float4 rdir = in.d[slot], hh = hits[slot];
         q = __float_as_uint(ro.w);
         shadeVertex<MODE, NRC, TEX, SHEEN>(fp, fp.depth, sv, pv, ro, rdir, Hit{hh.x, __float_as_uint(hh.y), hh.z, hh.w},
-                                           sh, she, counters, nv, cont, nextO, nextD);
+                                           sh, she, part, counters, nv, cont, nextO, nextD);
     }
-    uint32_t slot = waveAppend(cont, &counters[outSlot]);
+    const uint32_t next = queueSlot(part, waveAppend(cont, &out.count[part * kPartStride]));
     if (cont) {
-        out.o[slot] = make_float4(nextO.x, nextO.y, nextO.z, __uint_as_float(q));
-        out.d[slot] = make_float4(nextD.x, nextD.y, nextD.z, kRayTMax);
+        out.o[next] = make_float4(nextO.x, nextO.y, nextO.z, __uint_as_float(q));
+        out.d[next] = make_float4(nextD.x, nextD.y, nextD.z, kRayTMax);
     }
 }
 
@@ -1162,15 +1236,14 @@ __global__ __launch_bounds__(kBlock, SHEEN ? 2 : 3) void kShade(FrameParams fp, 
 constexpr uint32_t kTailShadeLanes = 48;  // of 32, 48, 56 and 64 lanes, 48 and 56 measured fastest
 template <int MODE>
 __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneView sv, PathView pv, QueueView in,
-                                                        uint32_t* counters, int countSlot, uint32_t startDepth,
-                                                        uint32_t* gstack) {
+                                                        uint32_t* counters, uint32_t startDepth, uint32_t* gstack) {
     __shared__ uint32_t lds[kLdsStackWords];
     TraversalStack st;
     st.lds = lds + threadIdx.x;
     st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
     st.dropped = 0;
     st.sp = 0;
-    const uint32_t n = counters[countSlot];
+    const uint32_t n = queueTotal(in.count);
     // wavefronts beyond one per 64 queued paths leave at once
     if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
     constexpr uint32_t kIdle = 0u, kTrace = 1u, kReady = 2u;
@@ -1209,8 +1282,11 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
             base = (uint32_t)__shfl((int)base, 0);
             if (base + idle >= n) exhausted = true;
             if (state == kIdle) {
-                const uint32_t k = base + (uint32_t)__popcll(idleMask & lanesBelow);
-                if (k < n) {
+                uint32_t k = base + (uint32_t)__popcll(idleMask & lanesBelow);
+                if (k < n) {  // ray k of the queue's parts one after the other
+                    uint32_t p = 0;
+                    while (k >= in.count[p * kPartStride]) k -= in.count[p++ * kPartStride];
+                    k = queueSlot(p, k);
                     ro = in.o[k];
                     rd = in.d[k];
                     depth = startDepth;
@@ -1225,7 +1301,7 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
                 bool cont = false;
                 F3 nextO = f3(0.0f), nextD = f3(0.0f);
                 shadeVertex<MODE, false, false, false>(fp, depth, sv, pv, ro, rd, cs.h, ShadowView{}, ShadowView{},
-                                                       counters, NrcView{}, cont, nextO, nextD);
+                                                       0u, counters, NrcView{}, cont, nextO, nextD);
                 if (cont) {
                     ro = make_float4(nextO.x, nextO.y, nextO.z, ro.w);
                     rd = make_float4(nextD.x, nextD.y, nextD.z, kRayTMax);
@@ -1438,10 +1514,10 @@ __global__ void kFeatInit(uint32_t* state, uint32_t count) {
 // vertex that is not a specular hit to follow, and sample 0 counts bounces.
 template <int MODE, bool TEX>
 __global__ __launch_bounds__(kBlock) void kFeatures(FrameParams fp, SceneView sv, PathView pv, QueueView in,
-                                                    const float4* hits, const uint32_t* counters, int inSlot,
-                                                    FeatureView fv) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= counters[inSlot]) return;
+                                                    const float4* hits, FeatureView fv) {
+    const uint32_t part = blockIdx.x % kQueueParts, j = (blockIdx.x / kQueueParts) * kBlock + threadIdx.x;
+    if (j >= in.count[part * kPartStride]) return;
+    const uint32_t i = queueSlot(part, j);
     const float4 oq = in.o[i], dq = in.d[i], hh = hits[i];
     const uint32_t q = __float_as_uint(oq.w);
     if (fp.nrc && q >= fp.nrcRenderPaths) return;  // training paths of the neural cache
@@ -1809,8 +1885,7 @@ __global__ __launch_bounds__(kBlock) void kAdjointInit(uint32_t count, PathView 
 // those of kShade<kModeRgb> followed by the shadow passes.
 __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, SceneView sv, PathView pv, QueueView in,
                                                             const float4* hits, QueueView out, uint32_t* counters,
-                                                            int inSlot, int outSlot, uint32_t* gstack,
-                                                            AdjointView av) {
+                                                            uint32_t* gstack, AdjointView av) {
     __shared__ uint32_t lds[kLdsStackWords];
     extern __shared__ float gradLds[];
     GradSink sink{av.ldsMaterials ? gradLds : nullptr, &av};
@@ -1823,15 +1898,17 @@ __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, Sce
     st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
     st.dropped = 0;
     st.sp = 0;
-    const uint32_t n = counters[inSlot];
+    // the grid is a multiple of kQueueParts blocks: a block stays in the part of its XCD
+    const uint32_t part = blockIdx.x % kQueueParts, partLen = in.count[part * kPartStride];
+    const uint32_t stride = gridDim.x / kQueueParts * kTraceBlock;
     const uint32_t lane = threadIdx.x & 63u;
     const SceneData& sd = fp.sd;
-    for (uint32_t base = blockIdx.x * kTraceBlock + (threadIdx.x & ~63u); base < n; base += gridDim.x * kTraceBlock) {
-        const uint32_t i = base + lane;
+    for (uint32_t base = blockIdx.x / kQueueParts * kTraceBlock + (threadIdx.x & ~63u); base < partLen; base += stride) {
+        const uint32_t j = base + lane, i = queueSlot(part, j);
         bool cont = false;
         F3 nextO = f3(0.0f), nextD = f3(0.0f);
         uint32_t q = 0;
-        if (i < n) do {
+        if (j < partLen) do {
             float4 ro = in.o[i], rdir = in.d[i];
             q = __float_as_uint(ro.w);
             F3 o = xyz(ro), d = xyz(rdir);
@@ -2030,7 +2107,7 @@ __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, Sce
             if (newFlags & kFAbsorption) pv.sigma[q] = st4(sigma);
             pv.rad[q] = make_float4(lrem.x, lrem.y, lrem.z, 0.0f);
         } while (false);
-        uint32_t slot = waveAppend(cont, &counters[outSlot]);
+        const uint32_t slot = queueSlot(part, waveAppend(cont, &out.count[part * kPartStride]));
         if (cont) {
             out.o[slot] = make_float4(nextO.x, nextO.y, nextO.z, __uint_as_float(q));
             out.d[slot] = make_float4(nextD.x, nextD.y, nextD.z, kRayTMax);
@@ -2069,50 +2146,46 @@ __global__ __launch_bounds__(kBlock) void kBuildTriClass(SceneView sv, uint32_t 
 
 // Sorting the hits of a depth by material class before shading (waves then
 // run one family of BSDF lobes instead of both): class of every queued ray
-// (misses count as class 0) and the number of class-0 rays of every block.
-__global__ __launch_bounds__(kBlock) void kClassCount(const uint32_t* count, const float4* hits, const uint8_t* triClass,
-                                                     uint8_t* key, uint32_t* blockCount0) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t n = *count;
-    uint32_t c = 1u;
-    if (i < n) {
-        const uint32_t tri = __float_as_uint(hits[i].y);
+// (misses count as class 0) and the class-0 and class-1 rays of every block, in
+// the low and high half of a word.
+__global__ __launch_bounds__(kBlock) void kClassCount(QueueView in, const float4* hits,
+                                                     const uint8_t* triClass, uint8_t* key, uint64_t* blockCount) {
+    const uint32_t part = blockIdx.x % kQueueParts, j = (blockIdx.x / kQueueParts) * kBlock + threadIdx.x;
+    const uint32_t slot = queueSlot(part, j);
+    const bool valid = j < in.count[part * kPartStride];
+    uint32_t c = 0u;
+    if (valid) {
+        const uint32_t tri = __float_as_uint(hits[slot].y);
         c = tri == kNoHit ? 0u : triClass[tri];
-        key[i] = (uint8_t)c;
+        key[slot] = (uint8_t)c;
     }
-    const int zeros = __syncthreads_count(i < n && c == 0u);
-    if (threadIdx.x == 0) blockCount0[blockIdx.x] = (uint32_t)zeros;
+    const int zeros = __syncthreads_count(valid && c == 0u), ones = __syncthreads_count(valid && c != 0u);
+    if (threadIdx.x == 0) blockCount[blockIdx.x] = (uint64_t)(uint32_t)zeros | (uint64_t)(uint32_t)ones << 32;
 }
 
-// Stable partition: class-0 rays first, then class 1, each in queue order.
-// offset0 = exclusive scan of blockCount0; every block but the last is full.
-__global__ __launch_bounds__(kBlock) void kClassScatter(const uint32_t* count, const uint8_t* key,
-                                                       const uint32_t* blockCount0, const uint32_t* offset0,
+// Stable partition: class-0 rays first, then class 1, each in the order of the
+// queue's blocks. offset = exclusive scan of blockCount.
+__global__ __launch_bounds__(kBlock) void kClassScatter(QueueView in, const uint8_t* key,
+                                                       const uint64_t* blockCount, const uint64_t* offset,
                                                        uint32_t blocks, uint32_t* perm) {
-    __shared__ uint32_t waveZeros[kBlock / 64];
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t n = *count;
-    const uint32_t blockStart = blockIdx.x * kBlock;
-    if (blockStart >= n) return;  // uniform per block
-    const bool valid = i < n;
-    const uint32_t c = valid ? key[i] : 1u;
-    const unsigned long long zmask = __ballot(valid && c == 0u);
+    __shared__ uint32_t waveCount[2][kBlock / 64];
+    const uint32_t part = blockIdx.x % kQueueParts, j = (blockIdx.x / kQueueParts) * kBlock + threadIdx.x;
+    const uint32_t slot = queueSlot(part, j);
+    const bool valid = j < in.count[part * kPartStride];
+    const uint32_t c = valid && key[slot] ? 1u : 0u;
+    const unsigned long long mask0 = __ballot(valid && c == 0u), mask1 = __ballot(valid && c != 0u);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    if (lane == 0) waveZeros[wave] = (uint32_t)__popcll(zmask);
-    __syncthreads();
-    uint32_t before = 0;
-    for (uint32_t w = 0; w < wave; w++) before += waveZeros[w];
-    const uint32_t rank0 = before + (uint32_t)__popcll(zmask & ((1ull << lane) - 1ull));
-    if (!valid) return;
-    const uint32_t total0 = offset0[blocks - 1] + blockCount0[blocks - 1];
-    uint32_t pos;
-    if (c == 0u) {
-        pos = offset0[blockIdx.x] + rank0;
-    } else {
-        const uint32_t rank1 = (i - blockStart) - rank0;  // class-1 rays before i in this block
-        pos = total0 + (blockStart - offset0[blockIdx.x]) + rank1;
+    if (lane == 0) {
+        waveCount[0][wave] = (uint32_t)__popcll(mask0);
+        waveCount[1][wave] = (uint32_t)__popcll(mask1);
     }
-    perm[pos] = i;
+    __syncthreads();
+    if (!valid) return;
+    uint32_t rank = (uint32_t)__popcll((c ? mask1 : mask0) & ((1ull << lane) - 1ull));
+    for (uint32_t w = 0; w < wave; w++) rank += waveCount[c][w];
+    const uint32_t total0 = (uint32_t)offset[blocks - 1] + (uint32_t)blockCount[blocks - 1];
+    const uint32_t pos = c ? total0 + (uint32_t)(offset[blockIdx.x] >> 32) : (uint32_t)offset[blockIdx.x];
+    perm[pos + rank] = slot;
 }
 
 // ------------------------------------------------------------- host side --
@@ -2151,9 +2224,9 @@ bool ensureTraversalScratch(mrt_context* ctx) {
     if (!ctx->counters.reserve(kCounterWords)) return false;
     if (ctx->traceGrid == 0) {
         // persistent traversal grid: enough resident blocks to fill every CU
-        // 8 blocks per CU; a multiple of kFetchParts so every claim partition has blocks
+        // 8 blocks per CU; a multiple of kQueueParts so every queue part has blocks
         ctx->traceGrid = (uint32_t)std::max(1, ctx->cuCount) * 8u;
-        static_assert(8 % kFetchParts == 0, "trace grid must cover every claim partition");
+        static_assert(8 % kQueueParts == 0, "trace grid must cover every queue part");
         // the fused tail: two blocks per CU (two waves per SIMD), within the trace grid's stacks
         ctx->tailGrid = (uint32_t)std::max(1, ctx->cuCount) * 2u;
     }
@@ -2163,14 +2236,15 @@ bool ensureTraversalScratch(mrt_context* ctx) {
 
 static bool ensurePaths(mrt_context* ctx, size_t n, int mode, bool lightShadows, bool envShadows) {
     PathBuffers& b = ctx->paths;
+    const size_t slots = (size_t)queueBlocks(n) * kBlock;  // of a queue of up to n paths
     bool ok = b.rng.reserve(n) && b.flags.reserve(n) && b.thr.reserve(n) && b.rad.reserve(n) && b.misc.reserve(n) &&
-              b.sigma.reserve(n) && b.hits.reserve(n) && b.sampleRad.reserve(n);
+              b.sigma.reserve(n) && b.hits.reserve(slots) && b.sampleRad.reserve(n);
     for (int qi = 0; qi < 2; qi++)
-        for (int j = 0; j < 2; j++) ok = ok && b.rays[qi][j].reserve(n);
+        for (int j = 0; j < 2; j++) ok = ok && b.rays[qi][j].reserve(slots);
     if (lightShadows)
-        for (int j = 0; j < 4; j++) ok = ok && b.shadow[j].reserve(n);
+        for (int j = 0; j < 4; j++) ok = ok && b.shadow[j].reserve(slots);
     if (envShadows)
-        for (int j = 0; j < 3; j++) ok = ok && b.shadowEnv[j].reserve(n);
+        for (int j = 0; j < 3; j++) ok = ok && b.shadowEnv[j].reserve(slots);
     if (mode != kModeRgb) ok = ok && b.lam.reserve(n);
     if (mode == kModeHero)
         ok = ok && b.radXYZ.reserve(n) && b.tpp.reserve(n) && b.ptpp.reserve(n) && b.pbtp.reserve(n);
@@ -2218,32 +2292,30 @@ static void queueViews(mrt_context* ctx, QueueView qv[2]) {
     for (int qi = 0; qi < 2; qi++) {
         qv[qi].o = b.rays[qi][0].ptr;
         qv[qi].d = b.rays[qi][1].ptr;
-        qv[qi].count = ctx->counters.ptr + qi;
+        qv[qi].count = ctx->counters.ptr + (qi ? kCntQueue1 : kCntQueue0);
     }
 }
 
 // kExtend in the variant the scene needs: counting statistics or not, alpha test or not.
 static void launchExtend(mrt_context* ctx, bool countTraversal, const SceneView& sv, const QueueView& q, float4* hits,
-                         uint32_t* cnt, int slot, uint32_t salt, uint32_t pathBase,
+                         uint32_t* cnt, uint32_t salt, uint32_t pathBase,
                          float4 camO = make_float4(0.0f, 0.0f, 0.0f, 0.0f)) {
     hipStream_t s = ctx->stream;
     const bool alpha = sv.triAlpha != nullptr;
     const dim3 grid(ctx->traceGrid), block(kTraceBlock);
     uint32_t* stack = ctx->traversalStack.ptr;
     if (countTraversal && alpha)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<true, true, true>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, slot, stack,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<true, true, true>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, q.count, stack,
                            salt, pathBase, camO);
     else if (countTraversal)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<true, false>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, slot, stack,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<true, false>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, q.count, stack,
                            salt, pathBase, camO);
     else if (alpha && sv.texels)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<false, true, true>), grid, block, 0, s, sv, q.o, q.d, hits, cnt,
-                           slot, stack, salt, pathBase, camO);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<false, true, true>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, q.count, stack, salt, pathBase, camO);
     else if (alpha)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<false, true, false>), grid, block, 0, s, sv, q.o, q.d, hits, cnt,
-                           slot, stack, salt, pathBase, camO);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<false, true, false>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, q.count, stack, salt, pathBase, camO);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<false, false>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, slot,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kExtend<false, false>), grid, block, 0, s, sv, q.o, q.d, hits, cnt, q.count,
                            stack, salt, pathBase, camO);
 }
 
@@ -2251,21 +2323,21 @@ static void launchExtend(mrt_context* ctx, bool countTraversal, const SceneView&
 template <int MODE, bool SHEEN>
 static void launchShade(hipStream_t s, bool tex, const NrcRun* nrc, const FrameParams& fp, const SceneView& sv,
                         const PathView& pv, QueueView in, const float4* hits, QueueView out, ShadowView shv,
-                        ShadowView shev, uint32_t* cnt, int cur, int nxt, const uint32_t* order) {
-    const dim3 grid(blocksFor(fp.count)), block(kBlock);
+                        ShadowView shev, uint32_t* cnt, const uint32_t* order) {
+    const dim3 grid(queueBlocks(fp.count)), block(kBlock);
     constexpr int NM = MODE == kModeSingle ? kModeRgb : MODE;  // the cache runs in RGB and hero modes
     if (MODE != kModeSingle && nrc && tex)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kShade<NM, true, true, SHEEN>), grid, block, 0, s, fp, sv, pv, in, hits,
-                           out, shv, shev, cnt, cur, nxt, nrc->view, order);
+                           out, shv, shev, cnt, nrc->view, order);
     else if (MODE != kModeSingle && nrc)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kShade<NM, true, false, SHEEN>), grid, block, 0, s, fp, sv, pv, in, hits,
-                           out, shv, shev, cnt, cur, nxt, nrc->view, order);
+                           out, shv, shev, cnt, nrc->view, order);
     else if (tex)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kShade<MODE, false, true, SHEEN>), grid, block, 0, s, fp, sv, pv, in, hits,
-                           out, shv, shev, cnt, cur, nxt, NrcView{}, order);
+                           out, shv, shev, cnt, NrcView{}, order);
     else
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kShade<MODE, false, false, SHEEN>), grid, block, 0, s, fp, sv, pv, in,
-                           hits, out, shv, shev, cnt, cur, nxt, NrcView{}, order);
+                           hits, out, shv, shev, cnt, NrcView{}, order);
 }
 
 // tailDepth: the depth from which the fused tail kernel carries the paths left
@@ -2281,11 +2353,7 @@ static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool 
     SceneView sv = ctx->view();
     uint32_t* cnt = ctx->counters.ptr;
     QueueView qv[2];
-    for (int qi = 0; qi < 2; qi++) {
-        qv[qi].o = b.rays[qi][0].ptr;
-        qv[qi].d = b.rays[qi][1].ptr;
-        qv[qi].count = cnt + qi;
-    }
+    queueViews(ctx, qv);
     ShadowView shv{b.shadow[0].ptr, b.shadow[1].ptr, b.shadow[2].ptr, b.shadow[3].ptr, cnt + kCntShadow};
     ShadowView shev{b.shadowEnv[0].ptr, b.shadowEnv[1].ptr, b.shadowEnv[2].ptr, nullptr, cnt + kCntShadowEnv};
     fp.compactPrimary = fp.leanStart && !fv ? 1u : 0u;
@@ -2295,7 +2363,7 @@ static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool 
     else
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kGenerate<MODE, true>), dim3(blocksFor(fp.count)), dim3(kBlock), 0, s, fp, pv,
                            qv[0]);
-    hipLaunchKernelGGL(kSetCount, dim3(1), dim3(1), 0, s, cnt, kCntQueue0, fp.count);
+    hipLaunchKernelGGL(kBeginQueue, dim3(1), dim3(64), 0, s, cnt, fp.count);
     if (fv) hipLaunchKernelGGL(kFeatInit, dim3(blocksFor(fp.count)), dim3(kBlock), 0, s, fv->state, fp.count);
     int cur = 0;
     uint32_t maxDepth = fp.sd.rrMaxDepth;
@@ -2304,11 +2372,12 @@ static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool 
         fp.depth = depth;
         ev.depthNow = depth;
         if (tailDepth != 0u && depth == tailDepth) hipLaunchKernelGGL(kTailSnapshot, dim3(1), dim3(1), 0, s, cnt);
-        hipLaunchKernelGGL(kPrepDepth, dim3(1), dim3(64), 0, s, cnt, cur, nxt, depth);
+        hipLaunchKernelGGL(kPrepDepth, dim3(1), dim3(64), 0, s, cnt, cur ? kCntQueue1 : kCntQueue0,
+                           nxt ? kCntQueue1 : kCntQueue0, depth);
         if (tailDepth != 0u && depth == tailDepth && !countTraversal) {
             bool timed = ev.begin(s, 5);
             hipLaunchKernelGGL(HIP_KERNEL_NAME(kTail<MODE>), dim3(ctx->tailGrid), dim3(kTraceBlock), 0, s, fp, sv, pv,
-                               qv[cur], cnt, cur, depth, ctx->traversalStack.ptr);
+                               qv[cur], cnt, depth, ctx->traversalStack.ptr);
             if (timed) ev.end(s);
             break;
         }
@@ -2322,22 +2391,22 @@ static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool 
             for (int r = 0; r < 3; r++) org[r] = m[0][r] * 0.0f + m[1][r] * 0.0f + m[2][r] * 0.0f + m[3][r] * 1.0f;
             camO = make_float4(org[0], org[1], org[2], 1.0f);
         }
-        launchExtend(ctx, countTraversal, sv, qv[cur], b.hits.ptr, cnt, cur,
+        launchExtend(ctx, countTraversal, sv, qv[cur], b.hits.ptr, cnt,
                      alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 0u), pathBase, camO);
         if (timed) ev.end(s);
         timed = ev.begin(s, 1);
         const uint32_t* order = nullptr;
         if (sortShading) {
-            const uint32_t nb = blocksFor(fp.count);
-            hipLaunchKernelGGL(kClassCount, dim3(nb), dim3(kBlock), 0, s, cnt + cur, b.hits.ptr, ctx->triClass.ptr,
-                               b.sortKey.ptr, b.sortCount.ptr);
+            const uint32_t nb = queueBlocks(fp.count);
+            hipLaunchKernelGGL(kClassCount, dim3(nb), dim3(kBlock), 0, s, qv[cur], b.hits.ptr,
+                               ctx->triClass.ptr, b.sortKey.ptr, b.sortCount.ptr);
             size_t bytes = b.sortScratch.capacity;
-            if (!check(rocprim::exclusive_scan(b.sortScratch.ptr, bytes, b.sortCount.ptr, b.sortOffset.ptr, 0u, nb,
-                                               rocprim::plus<uint32_t>(), s),
+            if (!check(rocprim::exclusive_scan(b.sortScratch.ptr, bytes, b.sortCount.ptr, b.sortOffset.ptr,
+                                               (uint64_t)0, nb, rocprim::plus<uint64_t>(), s),
                        "shading sort scan"))
                 return false;
-            hipLaunchKernelGGL(kClassScatter, dim3(nb), dim3(kBlock), 0, s, cnt + cur, b.sortKey.ptr, b.sortCount.ptr,
-                               b.sortOffset.ptr, nb, b.sortPerm.ptr);
+            hipLaunchKernelGGL(kClassScatter, dim3(nb), dim3(kBlock), 0, s, qv[cur], b.sortKey.ptr,
+                               b.sortCount.ptr, b.sortOffset.ptr, nb, b.sortPerm.ptr);
             order = b.sortPerm.ptr;
         }
         // textured materials take a separate variant so that untextured scenes
@@ -2345,34 +2414,32 @@ static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool 
         const bool tex = sv.texels != nullptr;
         if (fv) {
             if (tex)
-                hipLaunchKernelGGL(HIP_KERNEL_NAME(kFeatures<MODE, true>), dim3(blocksFor(fp.count)), dim3(kBlock), 0,
-                                   s, fp, sv, pv, qv[cur], b.hits.ptr, cnt, cur, *fv);
+                hipLaunchKernelGGL(HIP_KERNEL_NAME(kFeatures<MODE, true>), dim3(queueBlocks(fp.count)), dim3(kBlock), 0, s,
+                                   fp, sv, pv, qv[cur], b.hits.ptr, *fv);
             else
-                hipLaunchKernelGGL(HIP_KERNEL_NAME(kFeatures<MODE, false>), dim3(blocksFor(fp.count)), dim3(kBlock),
-                                   0, s, fp, sv, pv, qv[cur], b.hits.ptr, cnt, cur, *fv);
+                hipLaunchKernelGGL(HIP_KERNEL_NAME(kFeatures<MODE, false>), dim3(queueBlocks(fp.count)), dim3(kBlock), 0, s,
+                                   fp, sv, pv, qv[cur], b.hits.ptr, *fv);
         }
         if (ctx->sheenEnabled)
-            launchShade<MODE, true>(s, tex, nrc, fp, sv, pv, qv[cur], b.hits.ptr, qv[nxt], shv, shev, cnt, cur, nxt,
-                                    order);
+            launchShade<MODE, true>(s, tex, nrc, fp, sv, pv, qv[cur], b.hits.ptr, qv[nxt], shv, shev, cnt, order);
         else
-            launchShade<MODE, false>(s, tex, nrc, fp, sv, pv, qv[cur], b.hits.ptr, qv[nxt], shv, shev, cnt, cur, nxt,
-                                     order);
+            launchShade<MODE, false>(s, tex, nrc, fp, sv, pv, qv[cur], b.hits.ptr, qv[nxt], shv, shev, cnt, order);
         if (timed) ev.end(s);
         if (fp.neeEnabled || fp.envNee) {  // otherwise no shadow record can exist
-            hipLaunchKernelGGL(kPrepShadow, dim3(1), dim3(1), 0, s, cnt);
             timed = ev.begin(s, 2);
             if (fp.neeEnabled)
                 hipLaunchKernelGGL(kShadow<MODE>, dim3(ctx->traceGrid), dim3(kTraceBlock), 0, s, sv, pv, shv, cnt,
-                                   kCntShadow, kCntFetchShadow, 0u, ctx->traversalStack.ptr,
+                                   kCntFetchShadow, 0u, ctx->traversalStack.ptr,
                                    alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 1u), pathBase);
             if (fp.envNee)
                 hipLaunchKernelGGL(kShadow<MODE>, dim3(ctx->traceGrid), dim3(kTraceBlock), 0, s, sv, pv, shev, cnt,
-                                   kCntShadowEnv, kCntFetchShadowEnv, 1u, ctx->traversalStack.ptr,
+                                   kCntFetchShadowEnv, 1u, ctx->traversalStack.ptr,
                                    alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 2u), pathBase);
             if (timed) ev.end(s);
         }
         cur = nxt;
     }
+    if (fp.neeEnabled || fp.envNee) hipLaunchKernelGGL(kCountShadow, dim3(1), dim3(1), 0, s, cnt);
     uint32_t imagePaths = fp.count;
     if (MODE != kModeSingle && nrc) {
         // the cache's estimate of what image paths would have gathered after their query vertex
@@ -2518,12 +2585,13 @@ static int setupFrame(mrt_context* ctx, const SceneData* scene, const mrt_render
     fs.sortShading = prm->materialSort != 0u && ctx->triCount > 0;
     if (fs.sortShading && chunk > 0) {
         PathBuffers& b = ctx->paths;
-        const uint32_t nb = blocksFor(chunk);
+        const size_t slots = (size_t)queueBlocks(chunk) * kBlock;
+        const uint32_t nb = blocksFor(slots);
         size_t scratch = 0;
-        if (!ensureTriClass(ctx) || !b.sortKey.reserve(chunk) || !b.sortPerm.reserve(chunk) ||
+        if (!ensureTriClass(ctx) || !b.sortKey.reserve(slots) || !b.sortPerm.reserve(slots) ||
             !b.sortCount.reserve(nb) || !b.sortOffset.reserve(nb) ||
-            !check(rocprim::exclusive_scan(nullptr, scratch, b.sortCount.ptr, b.sortOffset.ptr, 0u, nb,
-                                           rocprim::plus<uint32_t>(), ctx->stream),
+            !check(rocprim::exclusive_scan(nullptr, scratch, b.sortCount.ptr, b.sortOffset.ptr, (uint64_t)0, nb,
+                                           rocprim::plus<uint64_t>(), ctx->stream),
                    "shading sort scan size") ||
             !b.sortScratch.reserve(scratch))
             return -3;
@@ -2811,20 +2879,21 @@ extern "C" int mrt_render_backward(mrt_context* ctx, const SceneData* scene, con
         // replay with the same streams
         hipLaunchKernelGGL(HIP_KERNEL_NAME(kGenerate<kModeRgb, true>), dim3(blocksFor(fp.count)), dim3(kBlock), 0, s, fp,
                            pv, qv[0]);
-        hipLaunchKernelGGL(kSetCount, dim3(1), dim3(1), 0, s, cnt, kCntQueue0, fp.count);
+        hipLaunchKernelGGL(kBeginQueue, dim3(1), dim3(64), 0, s, cnt, fp.count);
         hipLaunchKernelGGL(kAdjointInit, dim3(blocksFor(fp.count)), dim3(kBlock), 0, s, fp.count, pv,
                            b.sampleRad.ptr);
         int cur = 0;
         for (uint32_t depth = 0; depth < fp.sd.rrMaxDepth; depth++) {
             int nxt = 1 - cur;
             fp.depth = depth;
-            hipLaunchKernelGGL(kPrepDepth, dim3(1), dim3(64), 0, s, cnt, cur, nxt, depth);
+            hipLaunchKernelGGL(kPrepDepth, dim3(1), dim3(64), 0, s, cnt, cur ? kCntQueue1 : kCntQueue0,
+                               nxt ? kCntQueue1 : kCntQueue0, depth);
             // the same alpha decisions as the primal pass: same salt, same path numbering
-            launchExtend(ctx, false, sv, qv[cur], b.hits.ptr, cnt, cur, alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 0u),
+            launchExtend(ctx, false, sv, qv[cur], b.hits.ptr, cnt, alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 0u),
                          (uint32_t)fp.pathBegin);
             hipLaunchKernelGGL(kShadeAdjoint, dim3(ctx->traceGrid), dim3(kTraceBlock),
                                av.ldsMaterials ? (uint32_t)gradLdsBytes : 0u, s, fp, sv, pv, qv[cur], b.hits.ptr,
-                               qv[nxt], cnt, cur, nxt, ctx->traversalStack.ptr, av);
+                               qv[nxt], cnt, ctx->traversalStack.ptr, av);
             cur = nxt;
         }
         if (!check(hipGetLastError(), "adjoint launch")) return -4;
