@@ -261,9 +261,10 @@ VKRT_Result VKRT_traceShadowRays(VKRT* vkrt, const float* rays, size_t count, ui
  * hipMalloc). deviceRays, deviceMesh, devicePrimitive and the optional
  * deviceT / deviceBarycentrics are device pointers on the context's GPU,
  * laid out as in VKRT_traceRays; results are bit-identical to it. The
- * traversal stacks and the overflow counter live in one fixed device array of
- * the library (about 61 MB per GPU, held until the process ends) shared by
- * every call on that GPU: calls that overlap on one GPU race. At most 2^30
+ * traversal stacks are the context's own once it has drawn a frame or answered
+ * a host query; until then, and for the count of a stack overflow, one fixed
+ * device array of the library (about 61 MB per GPU, held until the process
+ * ends) serves every call on that GPU: calls that overlap on one GPU race. At most 2^30
  * rays per call (VKRT_ERROR_INVALID_ARGUMENT beyond). The scene must already
  * be on the device (VKRT_ERROR_OPERATION_FAILED when it changed since the
  * last upload, as uploading allocates). Returns after the results are

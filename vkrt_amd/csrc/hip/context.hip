@@ -128,6 +128,8 @@ extern "C" void mrt_destroy(mrt_context* ctx) {
     b.sampleRad.release();
     ctx->counters.release();
     ctx->traversalStack.release();
+    ctx->queryRays.release();
+    ctx->queryOut.release();
     hipEventDestroy(ctx->evBegin);
     hipEventDestroy(ctx->evEnd);
     for (auto& e : ctx->evStage) hipEventDestroy(e);

@@ -413,55 +413,89 @@ DEV Hit traceClosest(const SceneView& s, const TraversalRay& r, float tmin, floa
     return cs.h;
 }
 
-// Any hit in (tmin, tmax): the first accepted intersection ends the search, as
-// RAY_FLAG_ACCEPT_FIRST_HIT_AND_END_SEARCH. Returns the global triangle id or kNoHit.
-DEV uint32_t traceAny(const SceneView& s, const TraversalRay& r, float tmin, float tmax, TraversalStack& st,
-                      uint32_t alphaKey) {
-    if (s.nodeCount == 0) return kNoHit;
+// Any-hit traversal state of one ray.
+struct AnyState {
+    uint32_t ref, steps;
+    uint32_t tri;  // the hit, once the traversal has finished: a global triangle id or kNoHit
+};
+DEV void anyBegin(AnyState& as, TraversalStack& st) {
+    as.ref = 0;
+    as.steps = 0;
+    as.tri = kNoHit;
     st.sp = 0;
-    uint32_t ref = 0;
-    for (uint32_t step = 0;; step++) {
-        if (step >= kMaxTraversalSteps) {
-            st.dropped++;
-            break;
+}
+
+// One node or leaf visit of an any-hit traversal in (tmin, tmax): the first
+// accepted intersection ends the search, as
+// RAY_FLAG_ACCEPT_FIRST_HIT_AND_END_SEARCH. Returns false once the traversal
+// has finished. ALPHA = false compiles the alpha test out.
+template <bool ALPHA = true>
+DEV bool anyStep(const SceneView& s, const TraversalRay& r, float tmin, float tmax, AnyState& as, TraversalStack& st,
+                 uint32_t alphaKey) {
+    if (as.steps++ >= kMaxTraversalSteps) {
+        st.dropped++;
+        return false;
+    }
+    if (!(as.ref & kLeafBit)) {
+        const Children c = boxes8(s.nodes + as.ref, r, tmin, tmax);
+        if (c.mask != 0u) {
+            // visit the lowest overlapping slot next, push the others
+            const uint32_t m = c.mask;
+            const int first = __ffs(m) - 1;
+            as.ref = first == 0 ? c.rLo.x : first == 1 ? c.rLo.y : first == 2 ? c.rLo.z : first == 3 ? c.rLo.w
+                   : first == 4 ? c.rHi.x : first == 5 ? c.rHi.y : first == 6 ? c.rHi.z : c.rHi.w;
+            const uint32_t rest = m & (m - 1u);
+            if (rest & 0x02u) st.push(c.rLo.y, 0.0f);
+            if (rest & 0x04u) st.push(c.rLo.z, 0.0f);
+            if (rest & 0x08u) st.push(c.rLo.w, 0.0f);
+            if (rest & 0x10u) st.push(c.rHi.x, 0.0f);
+            if (rest & 0x20u) st.push(c.rHi.y, 0.0f);
+            if (rest & 0x40u) st.push(c.rHi.z, 0.0f);
+            if (rest & 0x80u) st.push(c.rHi.w, 0.0f);
+            return true;
         }
-        bool popNext = true;
-        if (!(ref & kLeafBit)) {
-            const Children c = boxes8(s.nodes + ref, r, tmin, tmax);
-            if (c.mask != 0u) {
-                // visit the lowest overlapping slot next, push the others
-                const uint32_t m = c.mask;
-                const int first = __ffs(m) - 1;
-                ref = first == 0 ? c.rLo.x : first == 1 ? c.rLo.y : first == 2 ? c.rLo.z : first == 3 ? c.rLo.w
-                    : first == 4 ? c.rHi.x : first == 5 ? c.rHi.y : first == 6 ? c.rHi.z : c.rHi.w;
-                const uint32_t rest = m & (m - 1u);
-                if (rest & 0x02u) st.push(c.rLo.y, 0.0f);
-                if (rest & 0x04u) st.push(c.rLo.z, 0.0f);
-                if (rest & 0x08u) st.push(c.rLo.w, 0.0f);
-                if (rest & 0x10u) st.push(c.rHi.x, 0.0f);
-                if (rest & 0x20u) st.push(c.rHi.y, 0.0f);
-                if (rest & 0x40u) st.push(c.rHi.z, 0.0f);
-                if (rest & 0x80u) st.push(c.rHi.w, 0.0f);
-                popNext = false;
-            }
-        } else {
-            uint32_t first = leafFirst(ref), count = leafCount(ref);
-            for (uint32_t i = 0; i < count; i++) {
-                const TriRecord tr = s.tris[first + i];
-                float t, u, v;
-                if (intersectTriangle(tr, r.o, r.pre, tmin, tmax, t, u, v)) {
-                    const uint32_t tri = __float_as_uint(tr.v0.w);
-                    if (!s.triAlpha || alphaAccept(s, tri, u, v, alphaKey)) return tri;
+    } else {
+        uint32_t first = leafFirst(as.ref), count = leafCount(as.ref);
+        for (uint32_t i = 0; i < count; i++) {
+            const TriRecord tr = s.tris[first + i];
+            float t, u, v;
+            if (intersectTriangle(tr, r.o, r.pre, tmin, tmax, t, u, v)) {
+                const uint32_t tri = __float_as_uint(tr.v0.w);
+                if (!ALPHA || !s.triAlpha || alphaAccept(s, tri, u, v, alphaKey)) {
+                    as.tri = tri;
+                    return false;
                 }
             }
         }
-        if (popNext) {
-            if (st.sp == 0) break;
-            float d;
-            st.pop(ref, d);
-        }
     }
-    return kNoHit;
+    if (st.sp == 0) return false;
+    float d;
+    st.pop(as.ref, d);
+    return true;
 }
+
+// Any hit in (tmin, tmax): the global triangle id of the first accepted intersection, or kNoHit.
+DEV uint32_t traceAny(const SceneView& s, const TraversalRay& r, float tmin, float tmax, TraversalStack& st,
+                      uint32_t alphaKey) {
+    if (s.nodeCount == 0) return kNoHit;
+    AnyState as;
+    anyBegin(as, st);
+    while (anyStep<true>(s, r, tmin, tmax, as, st, alphaKey)) {
+    }
+    return as.tri;
+}
+
+constexpr uint32_t kVisOccluded = 0u, kVisVisible = 1u, kVisUnsupported = 2u;
+// src/shaders/entry/shadow/closest_hit.slang:4-8
+DEV uint32_t classifyOccluder(const SceneView& sv, uint32_t tri) {
+    if (tri == kNoHit) return kVisVisible;
+    const Material& m = sv.materials[sv.meshes[sv.triMesh[tri]].materialIndex];
+    return m.transmission > 0.0f ? kVisUnsupported : kVisOccluded;
+}
+
+// Lanes of a persistent traversal kernel take new rays once this many of the
+// wavefront's lanes are idle (groups of 8 and 32 measured slower).
+constexpr uint32_t kRefillLanes = 16;
+constexpr uint32_t kNoRay = 0xFFFFFFFFu;
 
 }  // namespace mrt

@@ -77,7 +77,7 @@ bool nrcTrainSteps(mrt_context* ctx, const float4* in, uint32_t stride, const fl
                    uint32_t capacity, uint32_t steps, uint32_t batch, float lr);
 float nrcReadLoss(mrt_context* ctx);
 
-// allocation-free ray query (render.hip): resolves its scratch array's device address
+// allocation-free ray query (query.hip): resolves its scratch array's device address
 bool noAllocScratchInit(mrt_context* ctx);
 
 }  // namespace mrt
@@ -151,6 +151,8 @@ struct mrt_context {
     mrt::PathBuffers paths;
     mrt::DeviceArray<uint32_t> counters;
     mrt::DeviceArray<uint32_t> traversalStack;
+    mrt::DeviceArray<float4> queryRays;    // one piece of a host ray query
+    mrt::DeviceArray<uint32_t> queryOut;
     uint32_t traceGrid = 0;
     uint32_t tailGrid = 0;
     // queue length of every depth in the last single-chunk frame, with the

@@ -35,8 +35,6 @@ constexpr uint32_t kFAbsorption = 8u;
 constexpr uint32_t kFPendingCollapse = 16u;
 constexpr uint32_t kFPrevEnvNee = 32u;  // the previous vertex sampled the environment for NEE
 
-constexpr uint32_t kVisOccluded = 0u, kVisVisible = 1u, kVisUnsupported = 2u;
-
 // Paths in flight per chunk. Large enough that the queues of late bounces
 // (after most paths have ended) still fill the chip: 2^27 paths keep about
 // 40 GB of path state and queues resident, well inside 288 GB of HBM (a
@@ -60,7 +58,6 @@ constexpr int kCntDepthHist = 24, kDepthHist = 32, kCntTailFetch = kCntDepthHist
 // of shading per frame, 5.9 with parts).
 constexpr int kQueueParts = 8;
 constexpr uint32_t kPartStride = 64;  // uint32 slots between the counters of two parts
-constexpr uint32_t kFetchBatch = 64;  // shadow rays a wavefront claims per atomic
 constexpr int kPartWords = kQueueParts * (int)kPartStride;
 constexpr int kCntFetchExt = 64, kCntFetchShadow = kCntFetchExt + kPartWords,
               kCntFetchShadowEnv = kCntFetchShadow + kPartWords, kCntQueue0 = kCntFetchShadowEnv + kPartWords,
@@ -534,9 +531,7 @@ __global__ void kTailSnapshot(uint32_t* counters) {
 // their triangles together halved the leaf steps and still took 23.2, 23.0 and 24.2
 // against 22.0 ms per 1080p spectral frame.
 // COUNT adds the number of BVH nodes visited and triangles tested to the frame statistics.
-constexpr uint32_t kRefillLanes = 16;
 constexpr uint32_t kClaimMax = 256;
-constexpr uint32_t kNoRay = 0xFFFFFFFFu;
 
 // ALPHA: some mesh runs the alpha test (the opaque variant keeps six waves per SIMD);
 // TEXA: some material has textures, so the test may read a texture's alpha.
@@ -636,64 +631,91 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
     }
 }
 
-DEV uint32_t classifyOccluder(const SceneView& sv, uint32_t tri) {
-    if (tri == kNoHit) return kVisVisible;
-    const Material& m = sv.materials[sv.meshes[sv.triMesh[tri]].materialIndex];
-    return m.transmission > 0.0f ? kVisUnsupported : kVisOccluded;
-}
-
-// Any-hit queries of one shadow queue. Each record carries the contribution if
-// the segment is visible (a) and if it is not (b); at most one record per path
-// is in a queue, so the radiance update needs no atomics. Light rays follow the
-// reference's classification (a transmissive first occluder clears prevNee,
+// Any-hit queries of one shadow queue, with lanes refilled as in kExtend. Each
+// record carries the contribution if the segment is visible (a) and if it is
+// not (b); at most one record per path is in a queue, so the radiance update
+// needs no atomics. Light rays follow the reference's classification (a
+// transmissive first occluder clears prevNee,
 // src/shaders/entry/shadow/closest_hit.slang:4-8); environment rays are visible
-// or not.
-template <int MODE>
-__global__ __launch_bounds__(kTraceBlock) void kShadow(SceneView sv, PathView pv, ShadowView sh, uint32_t* counters,
-                                                      int fetchSlot, uint32_t envPass,
-                                                      uint32_t* gstack, uint32_t alphaSalt, uint32_t pathBase) {
+// or not. ALPHA as in kExtend.
+template <int MODE, bool ALPHA>
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? 4 : 6))) void kShadow(
+    SceneView sv, PathView pv, ShadowView sh, uint32_t* counters, int fetchSlot, uint32_t envPass, uint32_t* gstack,
+    uint32_t alphaSalt, uint32_t pathBase) {
     __shared__ uint32_t lds[kLdsStackWords];
     TraversalStack st;
     st.lds = lds + threadIdx.x;
     st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
     st.dropped = 0;
+    st.sp = 0;
     const uint32_t n = queueTotal(sh.count);
-    // wavefronts beyond one per batch leave at once (see kExtend)
-    if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * (uint64_t)kFetchBatch >= n) return;
+    // wavefronts beyond one per 64 rays leave at once (see kExtend)
+    if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
     const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t lanesBelow = (1ull << lane) - 1ull;
     uint32_t part = blockIdx.x % kQueueParts, partsTried = 0;
-    while (partsTried < (uint32_t)kQueueParts) {
-        // a batch of the current part, or the next part once that one is used up
-        const uint32_t partLen = sh.count[part * kPartStride];
-        const uint32_t base = claimRays(&counters[fetchSlot + part * kPartStride], partLen, kFetchBatch, partsTried > 0u), j = base + lane, i = queueSlot(part, j);
-        if (base + kFetchBatch >= partLen) {
-            part = (part + 1u) % kQueueParts;
-            partsTried++;
+    uint32_t poolNext = 0, poolEnd = 0, poolPart = part;
+    const uint32_t claim = min(max(n / (gridDim.x * (kTraceBlock / 64u) * 4u), 64u), kClaimMax);
+    uint32_t rayId = kNoRay, path = 0u, alphaKey = 0u;
+    float tmax = 0.0f;
+    TraversalRay r;
+    AnyState as;
+    anyBegin(as, st);
+    while (true) {
+        const uint64_t idleMask = __ballot(rayId == kNoRay);
+        const uint32_t idle = (uint32_t)__popcll(idleMask);
+        if (idle >= kRefillLanes && (partsTried < kQueueParts || poolNext < poolEnd)) {
+            if (poolNext >= poolEnd) {
+                const uint32_t partLen = __builtin_amdgcn_readfirstlane(sh.count[part * kPartStride]);
+                const uint32_t base = claimRays(&counters[fetchSlot + part * kPartStride], partLen, claim, partsTried > 0u);
+                poolPart = part;
+                poolNext = base;
+                poolEnd = min(base + claim, partLen);
+                if (base + claim >= partLen) {  // this part is used up
+                    part = (part + 1u) % kQueueParts;
+                    partsTried++;
+                }
+            }
+            const uint32_t first = poolNext;
+            poolNext = min(poolNext + idle, max(poolNext, poolEnd));
+            if (rayId == kNoRay) {
+                const uint32_t j = first + (uint32_t)__popcll(idleMask & lanesBelow);
+                if (j < poolEnd) {
+                    rayId = queueSlot(poolPart, j);
+                    const float4 o = sh.o[rayId], d = sh.d[rayId];
+                    path = __float_as_uint(o.w);
+                    tmax = d.w;
+                    r = makeTraversalRay(xyz(o), xyz(d));
+                    if (ALPHA) alphaKey = alphaRayKey(alphaSalt, pathBase + path);
+                    anyBegin(as, st);
+                }
+            }
         }
-        if (j >= partLen) continue;
-        float4 o = sh.o[i], d = sh.d[i];
-        uint32_t q = __float_as_uint(o.w);
-        TraversalRay r = makeTraversalRay(xyz(o), xyz(d));
-        uint32_t tri = traceAny(sv, r, kRayTMin, d.w, st, alphaRayKey(alphaSalt, pathBase + q));
-        uint32_t vis = envPass ? (tri == kNoHit ? kVisVisible : kVisOccluded) : classifyOccluder(sv, tri);
-        if (vis != kVisVisible && envPass) continue;  // b is zero for environment rays
-        F4 c = ld4(vis == kVisVisible ? sh.a[i] : sh.b[i]);
-        uint32_t flags = pv.flags[q];
-        if (vis == kVisUnsupported) pv.flags[q] = flags & ~kFPrevNee;
-        if (MODE == kModeRgb) {
-            F4 rad = ld4(pv.rad[q]);
-            pv.rad[q] = st4(F3{rad.x, rad.y, rad.z} + F3{c.x, c.y, c.z}, 0.0f);
-        } else if (MODE == kModeSingle) {
-            F4 rad = ld4(pv.rad[q]);
-            rad.x += c.x;
-            pv.rad[q] = st4(rad);
-        } else if (flags & (kFHeroActive | kFPendingCollapse)) {
-            pv.rad[q] = st4(ld4(pv.rad[q]) + c);
-        } else {
-            F4 rx = ld4(pv.radXYZ[q]);
-            rx.w += c.x;
-            pv.radXYZ[q] = st4(rx);
+        if (rayId != kNoRay && !anyStep<ALPHA>(sv, r, kRayTMin, tmax, as, st, alphaKey)) {
+            const uint32_t vis =
+                envPass ? (as.tri == kNoHit ? kVisVisible : kVisOccluded) : classifyOccluder(sv, as.tri);
+            if (vis == kVisVisible || !envPass) {  // b is zero for environment rays
+                const F4 c = ld4(vis == kVisVisible ? sh.a[rayId] : sh.b[rayId]);
+                const uint32_t flags = pv.flags[path];
+                if (vis == kVisUnsupported) pv.flags[path] = flags & ~kFPrevNee;
+                if (MODE == kModeRgb) {
+                    F4 rad = ld4(pv.rad[path]);
+                    pv.rad[path] = st4(F3{rad.x, rad.y, rad.z} + F3{c.x, c.y, c.z}, 0.0f);
+                } else if (MODE == kModeSingle) {
+                    F4 rad = ld4(pv.rad[path]);
+                    rad.x += c.x;
+                    pv.rad[path] = st4(rad);
+                } else if (flags & (kFHeroActive | kFPendingCollapse)) {
+                    pv.rad[path] = st4(ld4(pv.rad[path]) + c);
+                } else {
+                    F4 rx = ld4(pv.radXYZ[path]);
+                    rx.w += c.x;
+                    pv.radXYZ[path] = st4(rx);
+                }
+            }
+            rayId = kNoRay;
         }
+        if (partsTried >= kQueueParts && poolNext >= poolEnd && __ballot(rayId != kNoRay) == 0ull) break;
     }
     if (st.dropped) atomicAdd(&counters[kCntDropped], st.dropped);
 }
@@ -1711,28 +1733,6 @@ __global__ void kFill4(float4* p, size_t n, float4 v) {
     if (i < n) p[i] = v;
 }
 
-__global__ __launch_bounds__(kTraceBlock) void kTraceQuery(SceneView sv, const float4* rays, uint32_t n,
-                                                          float4* out, uint32_t* gstack, uint32_t anyHit) {
-    __shared__ uint32_t lds[kLdsStackWords];
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
-    for (uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x; i < n; i += gridDim.x * kTraceBlock) {
-        float4 a = rays[2 * i], b = rays[2 * i + 1];
-        TraversalRay r = makeTraversalRay(xyz(a), xyz(b));
-        // a query ray has no path: its index is its key
-        const uint32_t key = alphaRayKey(alphaSalt(0u, 0ull, 0u, 3u), i);
-        if (anyHit) {
-            uint32_t vis = classifyOccluder(sv, traceAny(sv, r, a.w, b.w, st, key));
-            out[i] = make_float4(__uint_as_float(vis), 0.0f, 0.0f, 0.0f);
-        } else {
-            Hit h = traceClosest(sv, r, a.w, b.w, st, key);
-            out[i] = make_float4(h.t, __uint_as_float(h.tri), h.u, h.v);
-        }
-    }
-}
-
 __global__ __launch_bounds__(kTraceBlock) void kPrimary(SceneView sv, SceneData sd, uint32_t rngPolicy,
                                                        uint64_t rngSeed, uint32_t sampleIndex, uint32_t* outMesh,
                                                        uint32_t* outPrim, uint32_t* gstack) {
@@ -2319,6 +2319,18 @@ static void launchExtend(mrt_context* ctx, bool countTraversal, const SceneView&
                            stack, salt, pathBase, camO);
 }
 
+template <int MODE>
+static void launchShadow(mrt_context* ctx, const SceneView& sv, const PathView& pv, const ShadowView& sh, int fetchSlot,
+                         uint32_t envPass, uint32_t salt, uint32_t pathBase) {
+    const dim3 grid(ctx->traceGrid), block(kTraceBlock);
+    if (sv.triAlpha)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kShadow<MODE, true>), grid, block, 0, ctx->stream, sv, pv, sh,
+                           ctx->counters.ptr, fetchSlot, envPass, ctx->traversalStack.ptr, salt, pathBase);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(kShadow<MODE, false>), grid, block, 0, ctx->stream, sv, pv, sh,
+                           ctx->counters.ptr, fetchSlot, envPass, ctx->traversalStack.ptr, salt, pathBase);
+}
+
 // kShade variant for the scene: RGB with the neural cache, textured, sheen.
 template <int MODE, bool SHEEN>
 static void launchShade(hipStream_t s, bool tex, const NrcRun* nrc, const FrameParams& fp, const SceneView& sv,
@@ -2428,12 +2440,10 @@ static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool 
         if (fp.neeEnabled || fp.envNee) {  // otherwise no shadow record can exist
             timed = ev.begin(s, 2);
             if (fp.neeEnabled)
-                hipLaunchKernelGGL(kShadow<MODE>, dim3(ctx->traceGrid), dim3(kTraceBlock), 0, s, sv, pv, shv, cnt,
-                                   kCntFetchShadow, 0u, ctx->traversalStack.ptr,
-                                   alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 1u), pathBase);
+                launchShadow<MODE>(ctx, sv, pv, shv, kCntFetchShadow, 0u, alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 1u),
+                                   pathBase);
             if (fp.envNee)
-                hipLaunchKernelGGL(kShadow<MODE>, dim3(ctx->traceGrid), dim3(kTraceBlock), 0, s, sv, pv, shev, cnt,
-                                   kCntFetchShadowEnv, 1u, ctx->traversalStack.ptr,
+                launchShadow<MODE>(ctx, sv, pv, shev, kCntFetchShadowEnv, 1u,
                                    alphaSalt(fp.sd.frameNumber, fp.rngSeed, depth, 2u), pathBase);
             if (timed) ev.end(s);
         }
@@ -2946,169 +2956,6 @@ extern "C" int mrt_read_output(mrt_context* ctx, uint16_t* out, size_t count) {
     }
     hipStreamSynchronize(ctx->stream);
     return check(hipMemcpy(out, ctx->output.ptr, count * sizeof(uint16_t), hipMemcpyDeviceToHost), "read output") ? 0 : -2;
-}
-
-static uint32_t hostBits(float f) {
-    uint32_t u;
-    memcpy(&u, &f, sizeof(u));
-    return u;
-}
-
-static int runQuery(mrt_context* ctx, const float* rays, size_t count, uint32_t anyHit, std::vector<float4>& result) {
-    if (!check(hipSetDevice(ctx->device), "hipSetDevice")) return -2;
-    if (!ensureTraversalScratch(ctx)) return -3;
-    if (count > 0xFFFFFFFFull / 2) {
-        setError("too many rays");
-        return -1;
-    }
-    float4* dRays = nullptr;
-    float4* dOut = nullptr;
-    if (!check(hipMalloc(&dRays, count * 2 * sizeof(float4)), "hipMalloc rays")) return -3;
-    if (!check(hipMalloc(&dOut, count * sizeof(float4)), "hipMalloc out")) {
-        hipFree(dRays);
-        return -3;
-    }
-    int rc = 0;
-    if (check(hipMemcpy(dRays, rays, count * 8 * sizeof(float), hipMemcpyHostToDevice), "upload rays")) {
-        hipLaunchKernelGGL(kTraceQuery, dim3(ctx->traceGrid), dim3(kTraceBlock), 0, ctx->stream, ctx->view(), dRays,
-                           (uint32_t)count, dOut, ctx->traversalStack.ptr, anyHit);
-        result.resize(count);
-        if (!check(hipStreamSynchronize(ctx->stream), "trace query") ||
-            !check(hipMemcpy(result.data(), dOut, count * sizeof(float4), hipMemcpyDeviceToHost), "read hits"))
-            rc = -4;
-    } else {
-        rc = -4;
-    }
-    hipFree(dRays);
-    hipFree(dOut);
-    return rc;
-}
-
-// ------------------------------------------------------ allocation-free --
-// The allocation-free ray query keeps everything beyond its inputs and
-// outputs in one fixed device array: a header whose word 0 counts dropped
-// traversal-stack pushes, then the global traversal stacks of a persistent
-// grid of kNoAllocBlocks blocks (kTraceBlock lanes x kGlobalStackWords words
-// each): 64 + 256 * 256 * 232 words, about 61 MB, held on every device the
-// library runs on until the process ends.
-constexpr uint32_t kNoAllocBlocks = 256;
-constexpr size_t kNoAllocHeaderWords = 64;
-constexpr size_t kNoAllocScratchWords =
-    kNoAllocHeaderWords + (size_t)kNoAllocBlocks * kTraceBlock * (size_t)kGlobalStackWords;
-static __device__ __align__(256) uint32_t scratch[kNoAllocScratchWords];
-
-// Device address of scratch on the current device; called once per context
-// at creation with its device current (the array's name is not a device
-// address in host code).
-bool mrt::noAllocScratchInit(mrt_context* ctx) {
-    void* p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) {
-        (void)hipGetLastError();
-        ctx->noAllocScratch = nullptr;
-        return false;
-    }
-    ctx->noAllocScratch = static_cast<uint32_t*>(p);
-    return true;
-}
-
-__global__ void kClearWords(uint32_t* p, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
-}
-
-// kTraceQuery's closest-hit search (same keys, same stack) writing the
-// per-mesh answer directly: mesh, primitive within the mesh, t, barycentrics.
-__global__ __launch_bounds__(kTraceBlock) void kTraceQueryDirect(SceneView sv, const float4* rays, uint32_t n,
-                                                                const uint32_t* triMesh, const uint32_t* meshTriBase,
-                                                                uint32_t* outMesh, uint32_t* outPrim, float* outT,
-                                                                float* outBary, uint32_t* scratchWords) {
-    __shared__ uint32_t lds[kLdsStackWords];
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = scratchWords + kNoAllocHeaderWords + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
-    for (uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x; i < n; i += gridDim.x * kTraceBlock) {
-        const float4 a = rays[2 * (size_t)i], b = rays[2 * (size_t)i + 1];
-        const TraversalRay r = makeTraversalRay(xyz(a), xyz(b));
-        const Hit h = traceClosest(sv, r, a.w, b.w, st, alphaRayKey(alphaSalt(0u, 0ull, 0u, 3u), i));
-        const bool hit = h.tri != kNoHit && h.tri < sv.triCount;
-        const uint32_t mesh = hit ? triMesh[h.tri] : VKRT_INVALID_INDEX;
-        outMesh[i] = mesh;
-        outPrim[i] = hit ? h.tri - meshTriBase[mesh] : VKRT_INVALID_INDEX;
-        if (outT) outT[i] = hit ? h.t : 0.0f;
-        if (outBary) {
-            outBary[2 * (size_t)i] = hit ? h.u : 0.0f;
-            outBary[2 * (size_t)i + 1] = hit ? h.v : 0.0f;
-        }
-    }
-    if (st.dropped) atomicAdd(&scratchWords[0], st.dropped);
-}
-
-extern "C" int mrt_trace_rays_noalloc(mrt_context* ctx, const float* deviceRays, size_t count, uint32_t* deviceMesh,
-                                      uint32_t* devicePrim, float* deviceT, float* deviceBary) {
-    if (!ctx || !deviceRays || !deviceMesh || !devicePrim) return -1;
-    if (count > MRT_NOALLOC_MAX_RAYS) {
-        setError("allocation-free ray query: more rays than its maximum of 2^30 per call");
-        return -1;
-    }
-    if (!ctx->noAllocScratch) {
-        setError("allocation-free ray query: no device address for its scratch array");
-        return -2;
-    }
-    if (!check(hipSetDevice(ctx->device), "hipSetDevice")) return -2;
-    if (count == 0) return 0;
-    hipStream_t s = ctx->stream;
-    hipLaunchKernelGGL(kClearWords, dim3(1), dim3((uint32_t)kNoAllocHeaderWords), 0, s, ctx->noAllocScratch,
-                       (uint32_t)kNoAllocHeaderWords);
-    hipLaunchKernelGGL(kTraceQueryDirect, dim3(kNoAllocBlocks), dim3(kTraceBlock), 0, s, ctx->view(),
-                       reinterpret_cast<const float4*>(deviceRays), (uint32_t)count, ctx->triMesh.ptr,
-                       ctx->meshTriBase.ptr, deviceMesh, devicePrim, deviceT, deviceBary, ctx->noAllocScratch);
-    uint32_t dropped = 0;
-    if (!check(hipGetLastError(), "allocation-free ray query launch") ||
-        !check(hipStreamSynchronize(s), "allocation-free ray query") ||
-        !check(hipMemcpy(&dropped, ctx->noAllocScratch, sizeof(dropped), hipMemcpyDeviceToHost), "read counter"))
-        return -4;
-    if (dropped) {
-        setError("traversal stack overflow");
-        return -5;
-    }
-    return 0;
-}
-
-extern "C" int mrt_trace_rays(mrt_context* ctx, const float* rays, size_t count, uint32_t* outMesh, uint32_t* outPrim,
-                              float* outT, float* outBary) {
-    if (!ctx || !rays || !outMesh || !outPrim) return -1;
-    std::vector<float4> res;
-    int rc = runQuery(ctx, rays, count, 0u, res);
-    if (rc) return rc;
-    std::vector<uint32_t> triMesh(ctx->triMesh.count), triBase(ctx->meshTriBase.count);
-    if (!triMesh.empty()) hipMemcpy(triMesh.data(), ctx->triMesh.ptr, triMesh.size() * 4, hipMemcpyDeviceToHost);
-    if (!triBase.empty()) hipMemcpy(triBase.data(), ctx->meshTriBase.ptr, triBase.size() * 4, hipMemcpyDeviceToHost);
-    for (size_t i = 0; i < count; i++) {
-        uint32_t tri = hostBits(res[i].y);
-        if (tri == kNoHit || tri >= triMesh.size()) {
-            outMesh[i] = VKRT_INVALID_INDEX;
-            outPrim[i] = VKRT_INVALID_INDEX;
-        } else {
-            outMesh[i] = triMesh[tri];
-            outPrim[i] = tri - triBase[triMesh[tri]];
-        }
-        if (outT) outT[i] = tri == kNoHit ? 0.0f : res[i].x;
-        if (outBary) {
-            outBary[2 * i] = tri == kNoHit ? 0.0f : res[i].z;
-            outBary[2 * i + 1] = tri == kNoHit ? 0.0f : res[i].w;
-        }
-    }
-    return 0;
-}
-
-extern "C" int mrt_trace_shadow_rays(mrt_context* ctx, const float* rays, size_t count, uint32_t* outVisibility) {
-    if (!ctx || !rays || !outVisibility) return -1;
-    std::vector<float4> res;
-    int rc = runQuery(ctx, rays, count, 1u, res);
-    if (rc) return rc;
-    for (size_t i = 0; i < count; i++) outVisibility[i] = hostBits(res[i].x);
-    return 0;
 }
 
 extern "C" int mrt_primary_hits(mrt_context* ctx, const SceneData* scene, const mrt_render_params* prm,
