@@ -114,3 +114,54 @@ def test_statistics_frame_records_the_rays_before_the_tail():
     assert s.tailStartDepth == 0 and s.tailRays == 0
     assert 0 < s.raysBeforeTail < s.extensionRays
     assert 0 < s.nodeVisitsBeforeTail < s.nodeVisits and 0 < s.triangleTestsBeforeTail < s.triangleTests
+
+
+def shadowed_frames(scene, w, h, spp, mode, spectral, tail_rays, env, frames=2):
+    r = V.Renderer(w, h)
+    scenes.load(r, scene)
+    r.configure(spp=spp, max_depth=9, min_depth=4, mode=mode, spectral=spectral, rng=V.RNG_PCG32, seed=5,
+                env_importance=env)
+    r.set_fused_tail(tail_rays)
+    r.start(w, h, 0)
+    for _ in range(frames):
+        r.draw()
+    st, img = r.stats(), r.accumulation()
+    r.close()
+    return img, st
+
+
+def lit_glass_under_sky():
+    """A light, a sky, dispersive and absorbing glass: both kinds of shadow ray,
+    unsupported occluders and collapsed hero wavelengths."""
+    s = scenes.cornell_box()
+    glass = V.default_material(baseColor=(0.9, 0.95, 0.9), roughness=0.05, metallic=0.0, specular=0.5)
+    glass.transmission, glass.ior, glass.abbeNumber = 1.0, 1.5, 30.0
+    glass.absorptionCoefficient = 0.5
+    glass.attenuationColor[:] = (0.7, 0.9, 0.8)
+    s.materials.append(glass)
+    s.meshes[4].material = len(s.materials) - 1
+    s.environment = scenes.sky_environment(128, 64, sun_radiance=50.0)
+    return s
+
+
+@pytest.mark.parametrize("mode,spectral", [(V.RENDER_MODE_RGB, V.SPECTRAL_HERO),
+                                           (V.RENDER_MODE_SPECTRAL, V.SPECTRAL_SINGLE),
+                                           (V.RENDER_MODE_SPECTRAL, V.SPECTRAL_HERO)])
+@pytest.mark.parametrize("env", [False, True], ids=["light", "light and sky"])
+@pytest.mark.parametrize("w,h,spp", [(5, 3, 1), (65, 63, 1), (512, 513, 1), (96, 54, 64)])
+def test_fused_tail_with_shadow_rays_gives_the_same_frame(mode, spectral, env, w, h, spp):
+    """Whole frames (up to 2^18 paths; 512 x 513 is just above) and tails from a
+    later depth against the launches per depth, to the last bit."""
+    ref, off = shadowed_frames(lit_glass_under_sky(), w, h, spp, mode, spectral, 0, env)
+    assert off.tailLaunches == 0 and off.shadowRays > 0
+    paths = w * h * spp
+    for rays in (1 << 20, paths // 2):
+        if rays == 0:
+            continue
+        img, st = shadowed_frames(lit_glass_under_sky(), w, h, spp, mode, spectral, rays, env)
+        whole = paths <= min(rays, 1 << 18)
+        assert st.tailLaunches == (1 if whole or st.tailStartDepth else 0)
+        assert (st.tailLaunches == 1 and st.tailStartDepth == 0) == whole
+        assert st.extensionRays == off.extensionRays and st.shadowRays == off.shadowRays
+        assert st.raysBeforeTail + (st.tailRays if st.tailLaunches else 0) == st.extensionRays
+        assert np.array_equal(img, ref)

@@ -46,8 +46,7 @@ constexpr int kBlock = 256;
 constexpr int kCntNrcQuery = 4, kCntDropped = 5, kCntNrcRecord = 6, kCntNrcTrain = 7,
               kCntStats = 8;  // 64-bit stats at counters+8: [0] ext rays, [1] shadow rays, [2] nodes, [3] triangles,
                               // [4] rays of the fused tail, [5..7] [0], [2], [3] as they stood when the tail began
-// queue length of every depth (the first kDepthHist depths) and the fused tail's claim counter
-constexpr int kCntDepthHist = 24, kDepthHist = 32, kCntTailFetch = kCntDepthHist + kDepthHist;
+constexpr int kCntDepthHist = 24, kDepthHist = 32;  // queue length of every depth (the first kDepthHist depths)
 // A queue is kQueueParts parts, each with its own length and its own claim
 // counter on a 256-byte line of their own. A block of kShade reads and appends
 // to part blockIdx % kQueueParts, which is also the XCD it runs on (workgroups
@@ -176,22 +175,52 @@ DEV uint32_t waveAppend(bool pred, uint32_t* counter) {
     return pred ? base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull)) : 0xFFFFFFFFu;
 }
 
-// First of the next `claim` rays of a part of partLen rays, or partLen or more
-// once the part is used up. Wave-uniform; every lane must be active. `look`:
-// read the counter first, for the parts that a wavefront turns to when its own
-// is used up: at the end of a launch every wavefront asks every part, and an
-// atomic on a used-up part waits in line with those of all the others. (Looking before
-// every claim was slower by far: 6.9 against 2.5 ms of shadow rays in the
-// 1024x1024 Cornell box, the line being in other hands whenever it is read.)
-DEV uint32_t claimRays(uint32_t* counter, uint32_t partLen, uint32_t claim, bool look) {
-    uint32_t base = 0;
-    if (look) {
-        base = __builtin_amdgcn_readfirstlane(__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        if (base >= partLen) return base;
+// The rays a wavefront of a persistent kernel still has to hand out to its
+// lanes: it claims them in runs of up to kClaimMax (about a quarter of its share
+// of a short queue) from the part of its block's XCD, then from the other parts.
+// One atomic per refill of the lanes made the wavefronts wait for the claim
+// counters (1024x1024 Cornell box, 16 spp: 4.54 ms of closest hits, 3.15 in
+// runs). Wave-uniform; every lane must be active where it is used.
+constexpr uint32_t kClaimMax = 256;
+struct RayClaims {
+    uint32_t part, tried = 0;               // the part asked next, parts found used up
+    uint32_t next = 0, end = 0, from;       // entries [next, end) of part `from` are to be handed out
+    uint32_t claim;
+    // n: rays in the queue
+    DEV explicit RayClaims(uint32_t n)
+        : part(blockIdx.x % kQueueParts), from(part),
+          claim(min(max(n / (gridDim.x * (kTraceBlock / 64u) * 4u), 64u), kClaimMax)) {}
+    DEV bool empty() const { return tried >= (uint32_t)kQueueParts && next >= end; }
+    // Entry for the first of `idle` lanes; the lane of rank k gets first + k if that is below
+    // `end`, of part `from`. counters: one per part; count: the parts' lengths.
+    DEV uint32_t take(uint32_t* counters, const uint32_t* count, uint32_t idle) {
+        if (next >= end) {
+            const uint32_t len = __builtin_amdgcn_readfirstlane(count[part * kPartStride]);
+            uint32_t base = 0;
+            // At the end of a launch every wavefront asks every part; an atomic on a
+            // used-up part waits in line with those of all the others, so its counter is
+            // looked at first. (Looking before every claim was slower by far, 6.9 against
+            // 2.5 ms of shadow rays in that Cornell box: the line is in other hands whenever it is read.)
+            if (tried > 0u)
+                base = __builtin_amdgcn_readfirstlane(
+                    __hip_atomic_load(&counters[part * kPartStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            if (base < len) {
+                if ((threadIdx.x & 63u) == 0u) base = atomicAdd(&counters[part * kPartStride], claim);
+                base = __builtin_amdgcn_readfirstlane(base);
+            }
+            from = part;
+            next = base;
+            end = min(base + claim, len);
+            if (base + claim >= len) {
+                part = (part + 1u) % kQueueParts;
+                tried++;
+            }
+        }
+        const uint32_t first = next;
+        next = min(next + idle, max(next, end));
+        return first;
     }
-    if ((threadIdx.x & 63u) == 0u) base = atomicAdd(counter, claim);
-    return __builtin_amdgcn_readfirstlane(base);
-}
+};
 
 // ------------------------------------------------------------ lights --
 // src/shaders/sampling/discrete.slang:8-18
@@ -484,7 +513,6 @@ __global__ __launch_bounds__(64) void kPrepDepth(uint32_t* counters, int cur, in
         stats[0] += n;
         stats[1] += queueTotal(counters + kCntShadow) + queueTotal(counters + kCntShadowEnv);
         if (depth < (uint32_t)kDepthHist) counters[kCntDepthHist + depth] = n;
-        counters[kCntTailFetch] = 0u;
     }
     __syncthreads();
     if (t < (uint32_t)kQueueParts) {
@@ -520,18 +548,12 @@ __global__ void kTailSnapshot(uint32_t* counters) {
 
 // Closest-hit traversal, persistent with lane refill. Every loop iteration
 // advances each busy lane by one node or leaf visit; once kRefillLanes lanes of
-// a wavefront are idle they take new rays, so lanes do not wait for the slowest
-// ray of a batch. A wavefront claims the rays in runs of up to kClaimMax (about a
-// quarter of its share of a short queue) and hands them out itself; one atomic per
-// refill made the wavefronts of a scene of few triangles wait for the claim
-// counters (1024x1024 Cornell box, 16 spp: 4.54 ms of traversal, 3.15 in runs). A
-// wavefront starts in the queue part of its block's XCD and moves on to the next part
-// once one is used up. What bounds it in scenes of many triangles is the latency of
-// the node loads: letting lanes with a leaf wait until 8, 16 or 24 of them could test
-// their triangles together halved the leaf steps and still took 23.2, 23.0 and 24.2
-// against 22.0 ms per 1080p spectral frame.
+// a wavefront are idle they take new rays (RayClaims), so lanes do not wait for
+// the slowest ray of a batch. What bounds it in scenes of many triangles is the
+// latency of the node loads: letting lanes with a leaf wait until 8, 16 or 24 of
+// them could test their triangles together halved the leaf steps and still
+// took 23.2, 23.0 and 24.2 against 22.0 ms per 1080p spectral frame.
 // COUNT adds the number of BVH nodes visited and triangles tested to the frame statistics.
-constexpr uint32_t kClaimMax = 256;
 
 // ALPHA: some mesh runs the alpha test (the opaque variant keeps six waves per SIMD);
 // TEXA: some material has textures, so the test may read a texture's alpha.
@@ -566,11 +588,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
     if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lanesBelow = (1ull << lane) - 1ull;
-    uint32_t part = blockIdx.x % kQueueParts;
-    uint32_t partsTried = 0;  // parts found exhausted by this wavefront
-    // rays [poolNext, poolEnd) of part poolPart are this wavefront's to hand out
-    uint32_t poolNext = 0, poolEnd = 0, poolPart = part;
-    const uint32_t claim = min(max(n / (gridDim.x * (kTraceBlock / 64u) * 4u), 64u), kClaimMax);
+    RayClaims claims(n);
     uint32_t rayId = kNoRay, alphaKey = 0u;
     TraversalRay r;
     ClosestState cs;
@@ -582,24 +600,11 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
     while (true) {
         const uint64_t idleMask = __ballot(rayId == kNoRay);
         const uint32_t idle = (uint32_t)__popcll(idleMask);
-        if (idle >= kRefillLanes && (partsTried < kQueueParts || poolNext < poolEnd)) {
-            if (poolNext >= poolEnd) {
-                const uint32_t partLen = __builtin_amdgcn_readfirstlane(count[part * kPartStride]);
-                const uint32_t base = claimRays(&counters[kCntFetchExt + part * kPartStride], partLen, claim,
-                                                partsTried > 0u);
-                poolPart = part;
-                poolNext = base;
-                poolEnd = min(base + claim, partLen);
-                if (base + claim >= partLen) {  // this part is used up
-                    part = (part + 1u) % kQueueParts;
-                    partsTried++;
-                }
-            }
-            const uint32_t first = poolNext;
-            poolNext = min(poolNext + idle, max(poolNext, poolEnd));
+        if (idle >= kRefillLanes && !claims.empty()) {
+            const uint32_t first = claims.take(counters + kCntFetchExt, count, idle);
             if (rayId == kNoRay) {
-                const uint32_t j = first + (uint32_t)__popcll(idleMask & lanesBelow), k = queueSlot(poolPart, j);
-                if (j < poolEnd) {
+                const uint32_t j = first + (uint32_t)__popcll(idleMask & lanesBelow), k = queueSlot(claims.from, j);
+                if (j < claims.end) {
                     float4 a = camO.w != 0.0f ? make_float4(camO.x, camO.y, camO.z, __uint_as_float(k)) : ro[k];
                     float4 b = rd[k];
                     r = makeTraversalRay(xyz(a), xyz(b));
@@ -621,13 +626,34 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
             }
         }
         // nothing left to claim: the wavefront goes on until every lane has finished its ray
-        if (partsTried >= kQueueParts && poolNext >= poolEnd && __ballot(rayId != kNoRay) == 0ull) break;
+        if (claims.empty() && __ballot(rayId != kNoRay) == 0ull) break;
     }
     if (st.dropped) atomicAdd(&counters[kCntDropped], st.dropped);
     if (COUNT) {
         unsigned long long* stats = reinterpret_cast<unsigned long long*>(counters + kCntStats);
         atomicAdd(&stats[2], (unsigned long long)nodeVisits);
         atomicAdd(&stats[3], (unsigned long long)triTests);
+    }
+}
+
+// Adds the contribution c of a path's shadow ray once its visibility is known.
+template <int MODE>
+DEV void addShadowed(const PathView& pv, uint32_t path, uint32_t vis, F4 c) {
+    const uint32_t flags = pv.flags[path];
+    if (vis == kVisUnsupported) pv.flags[path] = flags & ~kFPrevNee;
+    if (MODE == kModeRgb) {
+        F4 rad = ld4(pv.rad[path]);
+        pv.rad[path] = st4(F3{rad.x, rad.y, rad.z} + F3{c.x, c.y, c.z}, 0.0f);
+    } else if (MODE == kModeSingle) {
+        F4 rad = ld4(pv.rad[path]);
+        rad.x += c.x;
+        pv.rad[path] = st4(rad);
+    } else if (flags & (kFHeroActive | kFPendingCollapse)) {
+        pv.rad[path] = st4(ld4(pv.rad[path]) + c);
+    } else {
+        F4 rx = ld4(pv.radXYZ[path]);
+        rx.w += c.x;
+        pv.radXYZ[path] = st4(rx);
     }
 }
 
@@ -653,9 +679,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
     if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lanesBelow = (1ull << lane) - 1ull;
-    uint32_t part = blockIdx.x % kQueueParts, partsTried = 0;
-    uint32_t poolNext = 0, poolEnd = 0, poolPart = part;
-    const uint32_t claim = min(max(n / (gridDim.x * (kTraceBlock / 64u) * 4u), 64u), kClaimMax);
+    RayClaims claims(n);
     uint32_t rayId = kNoRay, path = 0u, alphaKey = 0u;
     float tmax = 0.0f;
     TraversalRay r;
@@ -664,24 +688,12 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
     while (true) {
         const uint64_t idleMask = __ballot(rayId == kNoRay);
         const uint32_t idle = (uint32_t)__popcll(idleMask);
-        if (idle >= kRefillLanes && (partsTried < kQueueParts || poolNext < poolEnd)) {
-            if (poolNext >= poolEnd) {
-                const uint32_t partLen = __builtin_amdgcn_readfirstlane(sh.count[part * kPartStride]);
-                const uint32_t base = claimRays(&counters[fetchSlot + part * kPartStride], partLen, claim, partsTried > 0u);
-                poolPart = part;
-                poolNext = base;
-                poolEnd = min(base + claim, partLen);
-                if (base + claim >= partLen) {  // this part is used up
-                    part = (part + 1u) % kQueueParts;
-                    partsTried++;
-                }
-            }
-            const uint32_t first = poolNext;
-            poolNext = min(poolNext + idle, max(poolNext, poolEnd));
+        if (idle >= kRefillLanes && !claims.empty()) {
+            const uint32_t first = claims.take(counters + fetchSlot, sh.count, idle);
             if (rayId == kNoRay) {
                 const uint32_t j = first + (uint32_t)__popcll(idleMask & lanesBelow);
-                if (j < poolEnd) {
-                    rayId = queueSlot(poolPart, j);
+                if (j < claims.end) {
+                    rayId = queueSlot(claims.from, j);
                     const float4 o = sh.o[rayId], d = sh.d[rayId];
                     path = __float_as_uint(o.w);
                     tmax = d.w;
@@ -694,28 +706,11 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
         if (rayId != kNoRay && !anyStep<ALPHA>(sv, r, kRayTMin, tmax, as, st, alphaKey)) {
             const uint32_t vis =
                 envPass ? (as.tri == kNoHit ? kVisVisible : kVisOccluded) : classifyOccluder(sv, as.tri);
-            if (vis == kVisVisible || !envPass) {  // b is zero for environment rays
-                const F4 c = ld4(vis == kVisVisible ? sh.a[rayId] : sh.b[rayId]);
-                const uint32_t flags = pv.flags[path];
-                if (vis == kVisUnsupported) pv.flags[path] = flags & ~kFPrevNee;
-                if (MODE == kModeRgb) {
-                    F4 rad = ld4(pv.rad[path]);
-                    pv.rad[path] = st4(F3{rad.x, rad.y, rad.z} + F3{c.x, c.y, c.z}, 0.0f);
-                } else if (MODE == kModeSingle) {
-                    F4 rad = ld4(pv.rad[path]);
-                    rad.x += c.x;
-                    pv.rad[path] = st4(rad);
-                } else if (flags & (kFHeroActive | kFPendingCollapse)) {
-                    pv.rad[path] = st4(ld4(pv.rad[path]) + c);
-                } else {
-                    F4 rx = ld4(pv.radXYZ[path]);
-                    rx.w += c.x;
-                    pv.radXYZ[path] = st4(rx);
-                }
-            }
+            if (vis == kVisVisible || !envPass)  // b is zero for environment rays
+                addShadowed<MODE>(pv, path, vis, ld4(vis == kVisVisible ? sh.a[rayId] : sh.b[rayId]));
             rayId = kNoRay;
         }
-        if (partsTried >= kQueueParts && poolNext >= poolEnd && __ballot(rayId != kNoRay) == 0ull) break;
+        if (claims.empty() && __ballot(rayId != kNoRay) == 0ull) break;
     }
     if (st.dropped) atomicAdd(&counters[kCntDropped], st.dropped);
 }
@@ -790,12 +785,14 @@ __global__ __launch_bounds__(kBlock) void kNrcTargets(const float4* record, cons
 // and its hit h. Leaves the continuation ray in nextO / nextD with cont set, or
 // cont false when the path ends here. Shadow records go to the part `part` (one
 // for the wave) of their queues, cache records to theirs, by whichever lanes
-// of the wave reach the append.
-template <int MODE, bool NRC, bool TEX, bool SHEEN>
+// of the wave reach the append; FUSED: the path's shadow records are left in slot q
+// for the caller to trace. shadowEmit, envEmit: which records there are.
+template <int MODE, bool NRC, bool TEX, bool SHEEN, bool FUSED = false>
 DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv, const PathView& pv, float4 ro,
                      float4 rdir, Hit h, const ShadowView& sh, const ShadowView& she, uint32_t part,
-                     uint32_t* counters, const NrcView& nv, bool& cont, F3& nextO, F3& nextD) {
-    bool shadowEmit = false, envEmit = false;
+                     uint32_t* counters, const NrcView& nv, bool& cont, F3& nextO, F3& nextD, bool& shadowEmit,
+                     bool& envEmit) {
+    shadowEmit = envEmit = false;
     F3 shO = f3(0.0f), shD = f3(0.0f), seO = f3(0.0f), seD = f3(0.0f);
     float shT = 0.0f;
     F4 shA = f4(0.0f), shB = f4(0.0f), seA = f4(0.0f);
@@ -1070,14 +1067,16 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
         // so they are not held in registers through BSDF sampling (waveAppend works
         // on whichever lanes are still active).
         {
-            const uint32_t sslot = queueSlot(part, waveAppend(shadowEmit, &sh.count[part * kPartStride]));
+            const uint32_t sslot =
+                FUSED ? q : queueSlot(part, waveAppend(shadowEmit, &sh.count[part * kPartStride]));
             if (shadowEmit) {
                 sh.o[sslot] = make_float4(shO.x, shO.y, shO.z, __uint_as_float(q));
                 sh.d[sslot] = make_float4(shD.x, shD.y, shD.z, shT);
                 sh.a[sslot] = st4(shA);
                 sh.b[sslot] = st4(shB);
             }
-            const uint32_t eslot = queueSlot(part, waveAppend(envEmit, &she.count[part * kPartStride]));
+            const uint32_t eslot =
+                FUSED ? q : queueSlot(part, waveAppend(envEmit, &she.count[part * kPartStride]));
             if (envEmit) {
                 she.o[eslot] = make_float4(seO.x, seO.y, seO.z, __uint_as_float(q));
                 she.d[eslot] = make_float4(seD.x, seD.y, seD.z, kRayTMax);
@@ -1215,7 +1214,7 @@ __global__ __launch_bounds__(kBlock, SHEEN ? 2 : 3) void kShade(FrameParams fp, 
                                                  const float4* hits, QueueView out, ShadowView sh, ShadowView she,
                                                  uint32_t* counters, NrcView nv, const uint32_t* __restrict__ order) {
     const uint32_t part = blockIdx.x % kQueueParts;
-    bool cont = false;
+    bool cont = false, shadowEmit, envEmit;
     F3 nextO = f3(0.0f), nextD = f3(0.0f);
     uint32_t q = 0;
     const uint32_t j = (blockIdx.x / kQueueParts) * kBlock + threadIdx.x;
@@ -1235,7 +1234,7 @@ __global__ __launch_bounds__(kBlock, SHEEN ? 2 : 3) void kShade(FrameParams fp, 
         const float4 rdir = in.d[slot], hh = hits[slot];
         q = __float_as_uint(ro.w);
         shadeVertex<MODE, NRC, TEX, SHEEN>(fp, fp.depth, sv, pv, ro, rdir, Hit{hh.x, __float_as_uint(hh.y), hh.z, hh.w},
-                                           sh, she, part, counters, nv, cont, nextO, nextD);
+                                           sh, she, part, counters, nv, cont, nextO, nextD, shadowEmit, envEmit);
     }
     const uint32_t next = queueSlot(part, waveAppend(cont, &out.count[part * kPartStride]));
     if (cont) {
@@ -1246,19 +1245,22 @@ __global__ __launch_bounds__(kBlock, SHEEN ? 2 : 3) void kShade(FrameParams fp, 
 
 // The last depths of a chunk in one launch, once the queues have become short:
 // every lane takes a path of the queue at depth startDepth and carries it to
-// its end, tracing and shading vertex after vertex (the arithmetic of kExtend
-// and kShade, so the same image), instead of one launch per depth that waits
+// its end, tracing and shading vertex after vertex (the arithmetic of kExtend,
+// kShade and kShadow, so the same image), instead of launches per depth that each wait
 // for the slowest ray of that depth. A lane that has its hit waits until
 // kTailShadeLanes lanes of the wave have theirs, or no lane is still tracing,
-// and they shade together; idle lanes claim new paths in batches as in
-// kExtend. Used when no shadow rays, cache, features, material sort, alpha
-// test, material textures or sheen are active (the shading variant without
-// them), at two waves per SIMD: the shading body inside the lane loop needs
-// more registers than the three-wave budget of kShade.
+// and they shade together; idle lanes take new paths as in kExtend. NEE: the
+// vertex's shadow rays are traced next, light before environment, then its
+// continuation, so a path's radiance is summed in the same order. Used
+// when no cache, features, material sort, alpha test, material textures or
+// sheen are active (the shading variant without them), at two waves per SIMD:
+// the shading body inside the lane loop needs more registers than the
+// three-wave budget of kShade.
 constexpr uint32_t kTailShadeLanes = 48;  // of 32, 48, 56 and 64 lanes, 48 and 56 measured fastest
-template <int MODE>
+template <int MODE, bool NEE>
 __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneView sv, PathView pv, QueueView in,
-                                                        uint32_t* counters, uint32_t startDepth, uint32_t* gstack) {
+                                                        ShadowView sh, ShadowView she, uint32_t* counters,
+                                                        uint32_t startDepth, uint32_t* gstack) {
     __shared__ uint32_t lds[kLdsStackWords];
     TraversalStack st;
     st.lds = lds + threadIdx.x;
@@ -1268,19 +1270,19 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
     const uint32_t n = queueTotal(in.count);
     // wavefronts beyond one per 64 queued paths leave at once
     if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
-    constexpr uint32_t kIdle = 0u, kTrace = 1u, kReady = 2u;
+    constexpr uint32_t kIdle = 0u, kTrace = 1u, kReady = 2u, kLight = 3u, kEnv = 4u;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lanesBelow = (1ull << lane) - 1ull;
-    uint32_t state = kIdle, depth = 0u, traced = 0u;
-    bool exhausted = false;  // wave-uniform: the queue has been claimed to its end
+    uint32_t state = kIdle, depth = 0u, traced = 0u, shadowed = 0u;
+    RayClaims claims(n);
     float4 ro = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rd = ro;
+    bool cont = false, shadowEmit = false, envEmit = false;
+    float shadowT = 0.0f;
     TraversalRay r;
     ClosestState cs;
-    cs.ref = 0;
-    cs.steps = 0;
-    cs.h.t = 0.0f;
-    cs.h.tri = kNoHit;
-    cs.h.u = cs.h.v = 0.0f;
+    AnyState as;
+    closestBegin(cs, st, 0.0f);
+    anyBegin(as, st);
     // start the traversal of the lane's ray (ro, rd): a ray that misses the
     // scene's box (or a scene without geometry) has its miss at once
     auto beginRay = [&]() {
@@ -1295,21 +1297,42 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
             state = kReady;
         }
     };
+    // what a lane does after shading or after a shadow ray: the vertex's next
+    // shadow ray, or its continuation, or nothing more
+    auto beginNext = [&]() {
+        if (NEE && (shadowEmit || envEmit)) {
+            const uint32_t q = __float_as_uint(ro.w);
+            const bool light = shadowEmit;
+            const float4 o = light ? sh.o[q] : she.o[q], d = light ? sh.d[q] : she.d[q];
+            state = light ? kLight : kEnv;
+            envEmit = envEmit && light;
+            shadowEmit = false;
+            r = makeTraversalRay(xyz(o), xyz(d));
+            shadowT = d.w;
+            shadowed++;
+            anyBegin(as, st);
+        } else if (cont) {
+            depth++;
+            traced++;
+            beginRay();
+        } else {
+            state = kIdle;
+        }
+    };
     while (true) {
         const uint64_t idleMask = __ballot(state == kIdle);
         const uint32_t idle = (uint32_t)__popcll(idleMask);
-        if (!exhausted && (idle >= kRefillLanes || idle == 64u)) {
-            uint32_t base = 0;
-            if (lane == 0u) base = atomicAdd(&counters[kCntTailFetch], idle);
-            base = (uint32_t)__shfl((int)base, 0);
-            if (base + idle >= n) exhausted = true;
+        if (idle >= kRefillLanes && !claims.empty()) {
+            const uint32_t first = claims.take(counters + kCntFetchExt, in.count, idle);
             if (state == kIdle) {
-                uint32_t k = base + (uint32_t)__popcll(idleMask & lanesBelow);
-                if (k < n) {  // ray k of the queue's parts one after the other
-                    uint32_t p = 0;
-                    while (k >= in.count[p * kPartStride]) k -= in.count[p++ * kPartStride];
-                    k = queueSlot(p, k);
-                    ro = in.o[k];
+                const uint32_t j = first + (uint32_t)__popcll(idleMask & lanesBelow), k = queueSlot(claims.from, j);
+                if (j < claims.end) {
+                    if (fp.compactPrimary && startDepth == 0u) {  // primary rays without stored origins
+                        const F3 co = cameraOrigin(fp.sd);
+                        ro = make_float4(co.x, co.y, co.z, __uint_as_float(k));
+                    } else {
+                        ro = in.o[k];
+                    }
                     rd = in.d[k];
                     depth = startDepth;
                     beginRay();
@@ -1317,33 +1340,43 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
             }
         }
         if (state == kTrace && !closestStep<false, false>(sv, r, kRayTMin, cs, st, 0u)) state = kReady;
+        if (NEE && state >= kLight && !anyStep<false>(sv, r, kRayTMin, shadowT, as, st, 0u)) {
+            const uint32_t q = __float_as_uint(ro.w);
+            const bool light = state == kLight;
+            const uint32_t vis = light ? classifyOccluder(sv, as.tri) : (as.tri == kNoHit ? kVisVisible : kVisOccluded);
+            if (light || vis == kVisVisible)  // an occluded environment ray adds nothing
+                addShadowed<MODE>(pv, q, vis, ld4(light ? (vis == kVisVisible ? sh.a[q] : sh.b[q]) : she.a[q]));
+            beginNext();
+        }
         const uint32_t ready = (uint32_t)__popcll(__ballot(state == kReady));
-        if (ready >= kTailShadeLanes || (ready > 0u && __ballot(state == kTrace) == 0ull)) {
+        if (ready >= kTailShadeLanes || (ready > 0u && __ballot(state == kTrace || state >= kLight) == 0ull)) {
             if (state == kReady) {
-                bool cont = false;
+                cont = false;
                 F3 nextO = f3(0.0f), nextD = f3(0.0f);
-                shadeVertex<MODE, false, false, false>(fp, depth, sv, pv, ro, rd, cs.h, ShadowView{}, ShadowView{},
-                                                       0u, counters, NrcView{}, cont, nextO, nextD);
+                shadeVertex<MODE, false, false, false, NEE>(fp, depth, sv, pv, ro, rd, cs.h, sh, she, 0u, counters,
+                                                            NrcView{}, cont, nextO, nextD, shadowEmit, envEmit);
                 if (cont) {
                     ro = make_float4(nextO.x, nextO.y, nextO.z, ro.w);
                     rd = make_float4(nextD.x, nextD.y, nextD.z, kRayTMax);
-                    depth++;
-                    traced++;
-                    beginRay();
-                } else {
-                    state = kIdle;
                 }
+                beginNext();
             }
         }
-        if (exhausted && __ballot(state != kIdle) == 0ull) break;
+        if (claims.empty() && __ballot(state != kIdle) == 0ull) break;
     }
     if (st.dropped) atomicAdd(&counters[kCntDropped], st.dropped);
     // the continuation rays (the queue's own rays were counted when the depth began)
-    for (int off = 32; off > 0; off >>= 1) traced += (uint32_t)__shfl_down((int)traced, off);
-    if (lane == 0u && traced) {
+    for (int off = 32; off > 0; off >>= 1) {
+        traced += (uint32_t)__shfl_down((int)traced, off);
+        if (NEE) shadowed += (uint32_t)__shfl_down((int)shadowed, off);
+    }
+    if (lane == 0u) {
         unsigned long long* stats = reinterpret_cast<unsigned long long*>(counters + kCntStats);
-        atomicAdd(&stats[0], (unsigned long long)traced);
-        atomicAdd(&stats[4], (unsigned long long)traced);
+        if (traced) {
+            atomicAdd(&stats[0], (unsigned long long)traced);
+            atomicAdd(&stats[4], (unsigned long long)traced);
+        }
+        if (NEE && shadowed) atomicAdd(&stats[1], (unsigned long long)shadowed);
     }
 }
 
@@ -2352,13 +2385,19 @@ static void launchShade(hipStream_t s, bool tex, const NrcRun* nrc, const FrameP
                            hits, out, shv, shev, cnt, NrcView{}, order);
 }
 
-// tailDepth: the depth from which the fused tail kernel carries the paths left
-// (0: none). With traversal statistics the depths stay separate launches and
-// only the totals at that depth are recorded.
+constexpr uint32_t kNoTail = 0xFFFFFFFFu;
+// Frames with shadow rays of at most this many paths (two per lane of kTail's
+// grid) run as one kTail launch from depth 0: a 256x256 Cornell preview of 1
+// sample takes 0.36 ms so and 0.75 ms with three launches per depth, a 512x512
+// one 0.61 and 0.92; at 2^19 paths one launch was faster for a room under a
+// light (1.13 against 1.26 ms from depth 1) and slower under an open sky (1.6, 1.5).
+constexpr uint64_t kWholeFramePaths = 1u << 18;
+// tailDepth: the depth from which the fused tail kernel carries the paths left.
+// With traversal statistics the depths stay separate launches and only the totals at that depth are recorded.
 template <int MODE>
 static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool countTraversal,
                         const NrcRun* nrc = nullptr, bool keepSampleRad = false, bool sortShading = false,
-                        const FeatureView* fv = nullptr, uint32_t tailDepth = 0u) {
+                        const FeatureView* fv = nullptr, uint32_t tailDepth = kNoTail) {
     hipStream_t s = ctx->stream;
     PathBuffers& b = ctx->paths;
     PathView pv = pathView(ctx);
@@ -2383,13 +2422,18 @@ static bool launchChunk(mrt_context* ctx, FrameParams fp, StageEvents& ev, bool 
         int nxt = 1 - cur;
         fp.depth = depth;
         ev.depthNow = depth;
-        if (tailDepth != 0u && depth == tailDepth) hipLaunchKernelGGL(kTailSnapshot, dim3(1), dim3(1), 0, s, cnt);
+        const bool tail = tailDepth == depth;
+        if (tail) hipLaunchKernelGGL(kTailSnapshot, dim3(1), dim3(1), 0, s, cnt);
         hipLaunchKernelGGL(kPrepDepth, dim3(1), dim3(64), 0, s, cnt, cur ? kCntQueue1 : kCntQueue0,
                            nxt ? kCntQueue1 : kCntQueue0, depth);
-        if (tailDepth != 0u && depth == tailDepth && !countTraversal) {
+        if (tail && !countTraversal) {
             bool timed = ev.begin(s, 5);
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(kTail<MODE>), dim3(ctx->tailGrid), dim3(kTraceBlock), 0, s, fp, sv, pv,
-                               qv[cur], cnt, depth, ctx->traversalStack.ptr);
+            if (fp.neeEnabled || fp.envNee)
+                hipLaunchKernelGGL(HIP_KERNEL_NAME(kTail<MODE, true>), dim3(ctx->tailGrid), dim3(kTraceBlock), 0, s, fp, sv,
+                                   pv, qv[cur], shv, shev, cnt, depth, ctx->traversalStack.ptr);
+            else
+                hipLaunchKernelGGL(HIP_KERNEL_NAME(kTail<MODE, false>), dim3(ctx->tailGrid), dim3(kTraceBlock), 0, s, fp,
+                                   sv, pv, qv[cur], shv, shev, cnt, depth, ctx->traversalStack.ptr);
             if (timed) ev.end(s);
             break;
         }
@@ -2721,17 +2765,23 @@ extern "C" int mrt_render_frame(mrt_context* ctx, const SceneData* scene, const 
     const FeatureView* fv = featurePass ? &fview : nullptr;
     // The fused tail (kTail) takes over from the first depth whose queue held
     // at most prm->tailRays rays in the previous frame of the same size: a
-    // single-chunk frame whose shading variant is the plain one (no shadow
-    // rays, cache, features, material sort, alpha test, textures or sheen).
-    uint32_t tailDepth = 0u;
+    // single-chunk frame whose shading variant is the plain one (no cache,
+    // features, material sort, alpha test, textures or sheen). A vertex with a
+    // shadow ray is twice the work, so frames with them take over at half that
+    // (961x543 sky, 8 samples, both kinds of sampling: 4.85 ms without a tail, 3.37
+    // and 3.35 at 2^18 and 2^20 rays; 1024x1024 Cornell box, 16 samples: 11.23,
+    // 11.22 and 11.36), and those of at most kWholeFramePaths paths are all tail.
+    uint32_t tailDepth = kNoTail;
     const uint32_t maxDepth = scene->rrMaxDepth;
     const SceneView svNow = ctx->view();
+    const bool nee = fp.neeEnabled || fp.envNee;
     const bool tailAllowed = prm->tailRays > 0u && totalPaths == chunk && !fp.nrc && !fv && !fs.sortShading &&
-                             !fp.neeEnabled && !fp.envNee && svNow.triAlpha == nullptr && svNow.texels == nullptr &&
-                             !ctx->sheenEnabled;
-    if (tailAllowed && ctx->hintPaths == chunk && ctx->hintMaxDepth == maxDepth) {
+                             svNow.triAlpha == nullptr && svNow.texels == nullptr && !ctx->sheenEnabled;
+    if (tailAllowed && nee && chunk <= std::min<uint64_t>(prm->tailRays, kWholeFramePaths)) {
+        tailDepth = 0u;
+    } else if (tailAllowed && ctx->hintPaths == chunk && ctx->hintMaxDepth == maxDepth) {
         for (uint32_t d = 1; d < std::min<uint32_t>(maxDepth, kDepthHist); d++)
-            if (ctx->depthHint[d] <= prm->tailRays) {
+            if (ctx->depthHint[d] <= (nee ? prm->tailRays / 2u : prm->tailRays)) {
                 tailDepth = d;
                 break;
             }
@@ -2807,10 +2857,10 @@ extern "C" int mrt_render_frame(mrt_context* ctx, const SceneData* scene, const 
         stats->shadowLaunches = stageN[2];
         stats->nrcInferMs = stageMs[3];
         stats->nrcTrainMs = stageMs[4];
-        stats->raysBeforeTail = tailDepth ? st64[5] : st64[0];
-        stats->nodeVisitsBeforeTail = tailDepth ? st64[6] : st64[2];
-        stats->triangleTestsBeforeTail = tailDepth ? st64[7] : st64[3];
-        if (tailDepth && !countTraversal) {
+        stats->raysBeforeTail = tailDepth != kNoTail ? st64[5] : st64[0];
+        stats->nodeVisitsBeforeTail = tailDepth != kNoTail ? st64[6] : st64[2];
+        stats->triangleTestsBeforeTail = tailDepth != kNoTail ? st64[7] : st64[3];
+        if (tailDepth != kNoTail && !countTraversal) {
             stats->tailStartDepth = tailDepth;
             stats->tailLaunches = stageN[5];
             stats->tailMs = stageMs[5];
