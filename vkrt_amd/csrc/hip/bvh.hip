@@ -42,19 +42,45 @@ __device__ __forceinline__ float orderedToFloat(uint32_t u) {
     return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
 }
 
-// per-triangle box, centroid bounds reduced into ordered-int min/max
+// World-space triangles from the packed vertices and the meshes' transforms:
+// the arithmetic (and rounding) of the host's worldPoint, so that they are the
+// triangles an exported scene shows. Moving a mesh then sends 64 bytes per mesh
+// instead of re-packing and sending the scene.
+__global__ __launch_bounds__(kB) void kPlaceTriangles(const ShaderVertex* vertices, const uint32_t* indices,
+                                                     const MeshInfo* meshes, const uint32_t* triMesh,
+                                                     const uint32_t* meshTriBase, const float* transforms, uint32_t n,
+                                                     float* worldTris) {
+    const uint32_t i = blockIdx.x * kB + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t mi = triMesh[i];
+    const MeshInfo& mesh = meshes[mi];
+    const float* m = transforms + (size_t)mi * 16u;
+    const uint32_t* tri = indices + mesh.indexBase + (size_t)(i - meshTriBase[mi]) * 3u;
+    for (int c = 0; c < 3; c++) {
+        uint32_t vi = tri[c];
+        if (vi >= mesh.vertexCount) vi = 0u;
+        const float* v = vertices[mesh.vertexBase + vi].position;
+        const float x = v[0], y = v[1], z = v[2];
+        for (int r = 0; r < 3; r++)
+            worldTris[(size_t)i * 9u + 3u * c + r] = (m[r] * x) + (m[4 + r] * y) + (m[8 + r] * z) + m[12 + r];
+    }
+}
+
+// per-triangle box, centroid bounds reduced into ordered-int min/max. At most
+// kBoundsBlocks blocks: the six atomics that end a block all meet on one line, and one
+// block per 256 triangles made them the kernel (384,004 triangles: 108 us, now 40 us).
+constexpr uint32_t kBoundsBlocks = 512;
 __global__ __launch_bounds__(kB) void kTriBounds(const float* tris9, uint32_t n, Aabb* boxes, uint32_t* centroidBounds) {
-    uint32_t i = blockIdx.x * kB + threadIdx.x;
     float c[3] = {INFINITY, INFINITY, INFINITY}, C[3] = {-INFINITY, -INFINITY, -INFINITY};
-    if (i < n) {
+    for (uint32_t i = blockIdx.x * kB + threadIdx.x; i < n; i += gridDim.x * kB) {
         const float* t = tris9 + (size_t)i * 9u;
         Aabb b;
         for (int a = 0; a < 3; a++) {
             b.lo[a] = fminf(fminf(t[a], t[3 + a]), t[6 + a]);
             b.hi[a] = fmaxf(fmaxf(t[a], t[3 + a]), t[6 + a]);
             float m = 0.5f * (b.lo[a] + b.hi[a]);
-            c[a] = m;
-            C[a] = m;
+            c[a] = fminf(c[a], m);
+            C[a] = fmaxf(C[a], m);
         }
         boxes[i] = b;
     }
@@ -220,6 +246,96 @@ __global__ __launch_bounds__(kB) void kPlocMerge(uint32_t* clusters, uint32_t m,
     keep[i] = (mutual && i > j) ? 0u : 1u;
 }
 
+// The last passes in one workgroup: once kPlocSmall clusters are left, a pass
+// is a microsecond of work and its launches, compaction and the wait for its
+// count were some 65 us. The pairs and their order are those of the passes above.
+constexpr int kPlocSmall = 2048;
+constexpr int kPlocThreads = 1024;
+__global__ __launch_bounds__(kPlocThreads) void kPlocFinish(uint32_t* clusters, uint32_t mBegin, Aabb* boxes,
+                                                           uint32_t* counts, int2* children, uint32_t n,
+                                                           uint32_t* nodeCounter, uint32_t* left) {
+    __shared__ Aabb box[kPlocSmall];
+    __shared__ uint32_t id[kPlocSmall], cnt[kPlocSmall];
+    __shared__ int nn[kPlocSmall];
+    __shared__ uint32_t waveKept[kPlocThreads / 64], nodeNext;
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
+    int m = (int)mBegin;
+    for (int i = t; i < m; i += kPlocThreads) {
+        id[i] = clusters[i];
+        box[i] = boxes[id[i]];
+        cnt[i] = counts[id[i]];
+    }
+    if (t == 0) nodeNext = *nodeCounter;
+    __syncthreads();
+    while (m > 1) {
+        for (int i = t; i < m; i += kPlocThreads) {
+            const Aabb a = box[i];
+            float best = INFINITY;
+            int bj = -1;
+            for (int k = -kPlocRadius; k <= kPlocRadius; k++) {
+                const int j = i + k;
+                if (k == 0 || j < 0 || j >= m) continue;
+                const float c = halfArea(merge(a, box[j]));
+                if (bj < 0 || pairBefore(c, i, j, best, bj)) {
+                    best = c;
+                    bj = j;
+                }
+            }
+            nn[i] = bj;
+        }
+        __syncthreads();
+        // clusters 2t and 2t + 1, so that the survivors keep their order
+        Aabb b[2];
+        uint32_t newId[2], newCnt[2], kept = 0;
+        bool keep[2];
+        for (int e = 0; e < 2; e++) {
+            const int i = 2 * t + e, j = i < m ? nn[i] : -1;
+            const bool mutual = j >= 0 && nn[j] == i;
+            keep[e] = i < m && !(mutual && i > j);
+            if (!keep[e]) continue;
+            kept++;
+            b[e] = box[i];
+            newId[e] = id[i];
+            newCnt[e] = cnt[i];
+            if (mutual) {
+                newId[e] = atomicAdd(&nodeNext, 1u);
+                b[e] = merge(b[e], box[j]);
+                newCnt[e] += cnt[j];
+                children[newId[e] - n] = make_int2((int)id[i], (int)id[j]);
+                boxes[newId[e]] = b[e];
+                counts[newId[e]] = newCnt[e];
+            }
+        }
+        uint32_t before = kept;  // inclusive sum over the wave
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)before, off);
+            if (lane >= off) before += v;
+        }
+        if (lane == 63) waveKept[wave] = before;
+        before -= kept;
+        __syncthreads();
+        uint32_t total = 0;
+        for (int w = 0; w < kPlocThreads / 64; w++) {
+            if (w < wave) before += waveKept[w];
+            total += waveKept[w];
+        }
+        for (int e = 0; e < 2; e++) {
+            if (!keep[e]) continue;
+            id[before] = newId[e];
+            box[before] = b[e];
+            cnt[before] = newCnt[e];
+            before++;
+        }
+        __syncthreads();
+        if ((int)total >= m) break;  // no progress (uniform): the host reports it
+        m = (int)total;
+    }
+    if (t == 0) {
+        clusters[0] = id[0];
+        *left = (uint32_t)m;
+    }
+}
+
 // ------------------------------------------------------------- collapse --
 struct CollapseItem {
     uint32_t node;   // binary node: leaf (< n) or merged node (>= n)
@@ -237,74 +353,86 @@ __device__ __forceinline__ void writeTriangle(const float* tris9, uint32_t t, Tr
     *out = r;
 }
 
+// One level of the collapse: eight lanes per wide node, lane k holding child k
+// and opening it when it is the largest box among the eight (the lowest lane
+// among equals). A lane per node kept its children in indexed arrays, which
+// live in scratch memory, and read them one after the other.
 __global__ __launch_bounds__(kB) void kCollapse(const CollapseItem* in, const uint32_t* inCount, CollapseItem* out,
                                                uint32_t* outCount, uint32_t* nodeAlloc, uint32_t n,
                                                const int2* children, const uint32_t* counts, const Aabb* boxes,
                                                const uint32_t* sortedTri, const float* tris9, TriRecord* triOut,
                                                BvhNode* nodes, uint32_t nodeCapacity, uint32_t* overflow,
                                                uint32_t leafMax) {
-    uint32_t w = blockIdx.x * kB + threadIdx.x;
-    if (w >= *inCount) return;
-    const CollapseItem it = in[w];
-    uint32_t slot[kBvhWidth], first[kBvhWidth];
-    int cnt = 0;
-    if (it.node < n || counts[it.node] <= leafMax) {
-        slot[cnt] = it.node;  // only the root of a tiny scene
-        first[cnt++] = it.first;
-    } else {
-        int2 c = children[it.node - n];
-        slot[0] = (uint32_t)c.x;
-        first[0] = it.first;
-        slot[1] = (uint32_t)c.y;
-        first[1] = it.first + counts[c.x];
-        cnt = 2;
-        while (cnt < kBvhWidth) {
-            // open the largest child that has too many triangles for a leaf
-            int best = -1;
-            float bestArea = -1.0f;
-            for (int k = 0; k < cnt; k++) {
-                if (counts[slot[k]] <= leafMax) continue;
-                float a = halfArea(boxes[slot[k]]);
-                if (a > bestArea) {
-                    bestArea = a;
-                    best = k;
+    const uint32_t items = *inCount;
+    const int k = (int)(threadIdx.x & 7u);
+    // whole groups of eight lanes go round together; a wave leaves with its last group
+    for (uint32_t w = (blockIdx.x * kB + threadIdx.x) >> 3; __ballot(w < items) != 0ull; w += gridDim.x * (kB / 8)) {
+        const bool live = w < items;
+        const CollapseItem it = live ? in[w] : CollapseItem{0u, 0u, 0u, 0u};
+        uint32_t slot = it.node, first = it.first, count = 1u;  // child k, once k < cnt
+        Aabb b{};
+        int cnt = 0;
+        if (live) {
+            cnt = 1;  // a tiny scene's root may be a leaf
+            if (it.node >= n && counts[it.node] > leafMax) {
+                cnt = 2;
+                const int2 c = children[it.node - n];
+                if (k == 1) first = it.first + counts[c.x];
+                slot = (uint32_t)(k == 1 ? c.y : c.x);
+            }
+            if (k < cnt) {
+                count = counts[slot];
+                b = boxes[slot];
+            }
+        }
+        while (true) {
+            // the largest child that has too many triangles for a leaf
+            float area = k < cnt && cnt < kBvhWidth && count > leafMax ? halfArea(b) : -1.0f;
+            if (!(area == area)) area = -1.0f;  // not a number: never opened
+            int best = k;
+            float bestArea = area;
+            for (int off = 1; off < 8; off <<= 1) {
+                const float oa = __shfl_xor(bestArea, off);
+                const int ob = __shfl_xor(best, off);
+                if (oa > bestArea || (oa == bestArea && ob < best)) {
+                    bestArea = oa;
+                    best = ob;
                 }
             }
-            if (best < 0) break;
-            int2 c2 = children[slot[best] - n];
-            uint32_t f = first[best];
-            slot[best] = (uint32_t)c2.x;
-            slot[cnt] = (uint32_t)c2.y;
-            first[cnt++] = f + counts[c2.x];
+            const bool open = bestArea > -1.0f;
+            if (__ballot(open) == 0ull) break;
+            int2 c2 = make_int2(0, 0);
+            uint32_t f2 = 0u;
+            if (open && k == best) {
+                c2 = children[slot - n];
+                f2 = first + counts[c2.x];
+                slot = (uint32_t)c2.x;
+            }
+            const int lane = (int)(threadIdx.x & 63u), from = (lane & ~7) | best;
+            const int right = __shfl(c2.y, from);
+            const uint32_t rightFirst = (uint32_t)__shfl((int)f2, from);
+            if (open && k == cnt) {
+                slot = (uint32_t)right;
+                first = rightFirst;
+            }
+            if (open && (k == best || k == cnt)) {
+                count = counts[slot];
+                b = boxes[slot];
+            }
+            if (open) cnt++;
         }
-    }
-    const Aabb P = boxes[it.node];
-    BvhNode node;
-    node.ox = P.lo[0];
-    node.oy = P.lo[1];
-    node.oz = P.lo[2];
-    uint32_t e[3];
-    float step[3];
-    for (int a = 0; a < 3; a++) {
-        e[a] = nodeExponent(P.lo[a], P.hi[a]);
-        step[a] = __uint_as_float(e[a] << 23);
-    }
-    for (int k = 0; k < 6; k++) node.qlo[k] = node.qhi[k] = 0u;
-    uint32_t used = 0;
-    for (int k = 0; k < cnt; k++) {
-        const uint32_t nd = slot[k];
-        const uint32_t count = counts[nd];
-        uint32_t ref;
-        if (count <= leafMax) {
+        const bool child = k < cnt;
+        uint32_t ref = kEmptyRef;
+        if (child && count <= leafMax) {
             // the subtree's triangles, depth first, into [first, first + count)
             uint32_t stack[kLeafMaxTrisLarge];
             int sp = 0;
             uint32_t written = 0;
-            stack[sp++] = nd;
+            stack[sp++] = slot;
             while (sp > 0) {
                 uint32_t x = stack[--sp];
                 if (x < n) {
-                    writeTriangle(tris9, sortedTri[x], &triOut[first[k] + written]);
+                    writeTriangle(tris9, sortedTri[x], &triOut[first + written]);
                     written++;
                 } else {
                     int2 c = children[x - n];
@@ -312,42 +440,78 @@ __global__ __launch_bounds__(kB) void kCollapse(const CollapseItem* in, const ui
                     stack[sp++] = (uint32_t)c.x;
                 }
             }
-            ref = kLeafBit | ((count - 1u) << 27) | first[k];
-        } else {
-            uint32_t child = atomicAdd(nodeAlloc, 1u);
-            if (child >= nodeCapacity) {
+            ref = kLeafBit | ((count - 1u) << 27) | first;
+        }
+        // slots of the inner children in the node array and the next frontier, one atomic per wave
+        const bool inner = child && count > leafMax;
+        const unsigned long long mask = __ballot(inner);
+        const int lane = (int)(threadIdx.x & 63u);
+        uint32_t base = 0, outBase = 0;
+        if (mask != 0ull && lane == __ffsll(mask) - 1) {
+            base = atomicAdd(nodeAlloc, (uint32_t)__popcll(mask));
+            outBase = atomicAdd(outCount, (uint32_t)__popcll(mask));
+        }
+        if (mask != 0ull) {
+            base = (uint32_t)__shfl((int)base, __ffsll(mask) - 1);
+            outBase = (uint32_t)__shfl((int)outBase, __ffsll(mask) - 1);
+        }
+        if (inner) {
+            const uint32_t rank = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+            if (base + rank < nodeCapacity) {
+                ref = base + rank;
+                out[outBase + rank] = CollapseItem{slot, ref, first, 0u};
+            } else {
                 atomicAdd(overflow, 1u);
-                continue;
             }
-            ref = child;
-            uint32_t o = atomicAdd(outCount, 1u);
-            out[o] = CollapseItem{nd, child, first[k], 0u};
         }
-        const Aabb b = boxes[nd];
+        // the node: its own box, and lane k's plane codes in byte k of each row
+        Aabb P{};
+        if (live) P = boxes[it.node];
+        uint32_t e[3], plane[6];
         for (int a = 0; a < 3; a++) {
-            uint32_t ql, qh;
-            quantizePlanes(P.lo[a], step[a], b.lo[a], b.hi[a], ql, qh);
-            node.qlo[a * 2 + (used >> 2)] |= ql << ((used & 3u) * 8u);
-            node.qhi[a * 2 + (used >> 2)] |= qh << ((used & 3u) * 8u);
+            e[a] = nodeExponent(P.lo[a], P.hi[a]);
+            uint32_t ql = 0u, qh = 0u;
+            if (child) quantizePlanes(P.lo[a], __uint_as_float(e[a] << 23), b.lo[a], b.hi[a], ql, qh);
+            plane[a] = ql << ((k & 3) * 8);
+            plane[3 + a] = qh << ((k & 3) * 8);
         }
-        node.child[used++] = ref;
+        for (int q = 0; q < 6; q++) {
+            plane[q] |= (uint32_t)__shfl_xor((int)plane[q], 1);
+            plane[q] |= (uint32_t)__shfl_xor((int)plane[q], 2);
+        }
+        if (live) {
+            BvhNode& node = nodes[it.wide];
+            node.child[k] = ref;
+            if ((k & 3) == 0) {
+                for (int a = 0; a < 3; a++) {
+                    node.qlo[a * 2 + (k >> 2)] = plane[a];
+                    node.qhi[a * 2 + (k >> 2)] = plane[3 + a];
+                }
+            }
+            if (k == 0) {
+                node.ox = P.lo[0];
+                node.oy = P.lo[1];
+                node.oz = P.lo[2];
+                node.packed = e[0] | (e[1] << 8) | (e[2] << 16) | ((uint32_t)cnt << 24);
+            }
+        }
     }
-    for (uint32_t k = used; k < (uint32_t)kBvhWidth; k++) node.child[k] = kEmptyRef;
-    node.packed = e[0] | (e[1] << 8) | (e[2] << 16) | (used << 24);
-    nodes[it.wide] = node;
 }
 
-__global__ void kInitCollapse(CollapseItem* items, uint32_t* counts, const uint32_t* root) {
-    items[0] = CollapseItem{*root, 0u, 0u, 0u};
-    counts[0] = 1u;  // items in the current frontier
-    counts[1] = 0u;  // items in the next frontier
-    counts[2] = 1u;  // wide nodes allocated
-    counts[3] = 0u;  // overflow
+// levels[l]: nodes of level l of the collapse (level 0 is the root)
+constexpr uint32_t kMaxLevels = 4096;
+__global__ void kInitCollapse(CollapseItem* items, uint32_t* counts, uint32_t* levels, const uint32_t* root) {
+    for (uint32_t i = threadIdx.x; i < kMaxLevels + 2u; i += blockDim.x) levels[i] = i == 0u ? 1u : 0u;
+    if (threadIdx.x == 0u) {
+        items[0] = CollapseItem{*root, 0u, 0u, 0u};
+        counts[0] = 1u;  // wide nodes allocated
+        counts[1] = 0u;  // overflow
+    }
 }
 
-__global__ void kFillU32(uint32_t* p, size_t n, uint32_t v) {
-    size_t i = (size_t)blockIdx.x * kB + threadIdx.x;
-    if (i < n) p[i] = v;
+__global__ void kInitBuild(uint32_t* centroidBounds, uint32_t* nodeCounter, uint32_t n) {
+    if (threadIdx.x < 6u) centroidBounds[threadIdx.x] = threadIdx.x < 3u ? 0xffffffffu : 0u;
+    if (threadIdx.x == 0u) *nodeCounter = n;
 }
 
 static uint32_t blocks(size_t n) { return (uint32_t)((n + kB - 1) / kB); }
@@ -371,81 +535,82 @@ extern "C" int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats) {
     hipEventRecord(ctx->evStage[0], s);
     const size_t binNodes = (size_t)2 * n - 1;
     const size_t wideCap = n;  // every wide node but the root is a distinct binary node with more than one triangle
-    DeviceArray<Aabb> triBoxes, boxes;
-    DeviceArray<uint32_t> cb, vals, valsSorted, counts, nodeCounts, clusters[2], selected;
-    DeviceArray<uint64_t> keys, keysSorted;
-    DeviceArray<int2> children;
-    DeviceArray<int> nn;
-    DeviceArray<uint8_t> keep;
-    DeviceArray<CollapseItem> front[2];
-    bool ok = triBoxes.reserve(n) && boxes.reserve(binNodes) && cb.reserve(6) && vals.reserve(n) &&
-              valsSorted.reserve(n) && counts.reserve(4) && nodeCounts.reserve(binNodes) && clusters[0].reserve(n) &&
-              clusters[1].reserve(n) && selected.reserve(2) && keys.reserve(n) && keysSorted.reserve(n) &&
-              children.reserve(n) && nn.reserve(n) && keep.reserve(n) && front[0].reserve(wideCap) &&
-              front[1].reserve(wideCap) && ctx->nodes.reserve(wideCap) && ctx->tris.reserve(n);
-    void* temp = nullptr;
-    auto cleanup = [&]() {
-        if (temp) hipFree(temp);
-        temp = nullptr;
-        triBoxes.release();
-        boxes.release();
-        cb.release();
-        vals.release();
-        valsSorted.release();
-        counts.release();
-        nodeCounts.release();
-        clusters[0].release();
-        clusters[1].release();
-        selected.release();
-        keys.release();
-        keysSorted.release();
-        children.release();
-        nn.release();
-        keep.release();
-        front[0].release();
-        front[1].release();
-    };
-    if (!ok) {
-        cleanup();
-        return -3;
-    }
-    // 1-3: bounds, Morton codes, sort
-    uint32_t initCb[6] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u};
-    hipMemcpyAsync(cb.ptr, initCb, sizeof(initCb), hipMemcpyHostToDevice, s);
-    hipLaunchKernelGGL(kTriBounds, dim3(blocks(n)), dim3(kB), 0, s, ctx->worldTris.ptr, n, triBoxes.ptr, cb.ptr);
-    hipLaunchKernelGGL(kMorton, dim3(blocks(n)), dim3(kB), 0, s, triBoxes.ptr, n, cb.ptr, keys.ptr, vals.ptr);
+    if (!ctx->nodes.reserve(wideCap) || !ctx->tris.reserve(n)) return -3;
+    // everything else in one allocation, which the context keeps for the next build while
+    // it is at most kKeepScratch bytes (some 1.9M triangles)
+    constexpr size_t kKeepScratch = 256u << 20;
     size_t sortBytes = 0, selectBytes = 0;
-    rocprim::radix_sort_pairs(nullptr, sortBytes, keys.ptr, keysSorted.ptr, vals.ptr, valsSorted.ptr, n, 0, 63, s);
-    rocprim::select(nullptr, selectBytes, clusters[0].ptr, keep.ptr, clusters[1].ptr, selected.ptr, (size_t)n, s);
-    if (!check(hipMalloc(&temp, std::max<size_t>(std::max(sortBytes, selectBytes), 1)), "hipMalloc build scratch")) {
-        cleanup();
-        return -3;
-    }
-    rocprim::radix_sort_pairs(temp, sortBytes, keys.ptr, keysSorted.ptr, vals.ptr, valsSorted.ptr, n, 0, 63, s);
+    rocprim::radix_sort_pairs(nullptr, sortBytes, (uint64_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr,
+                              (uint32_t*)nullptr, n, 0, 63, s);
+    rocprim::select(nullptr, selectBytes, (uint32_t*)nullptr, (uint8_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
+                    (size_t)n, s);
+    size_t bytes = 0;
+    auto take = [&](size_t size) {
+        const size_t at = bytes;
+        bytes += (size + 255u) & ~(size_t)255u;
+        return at;
+    };
+    const size_t aBoxes = take(binNodes * sizeof(Aabb)), aNodeCounts = take(binNodes * 4u), aValsSorted = take(n * 4u),
+                 aChildren = take(n * sizeof(int2)), aClusters0 = take(n * 4u), aClusters1 = take(n * 4u),
+                 aSmall = take(64u), aLevels = take((kMaxLevels + 2u) * 4u),
+                 aTemp = take(std::max<size_t>(std::max(sortBytes, selectBytes), 1));
+    // needed until the tree stands, then the collapse's frontiers take their place
+    const size_t aShared = bytes;
+    const size_t aTriBoxes = take(n * sizeof(Aabb)), aKeys = take(n * 8u), aKeysSorted = take(n * 8u),
+                 aVals = take(n * 4u), aNn = take(n * 4u), aKeep = take(n);
+    const size_t aFront0 = aShared;
+    bytes = std::max(bytes, aShared + 2u * ((wideCap * sizeof(CollapseItem) + 255u) & ~(size_t)255u));
+    const size_t aFront1 = aShared + ((wideCap * sizeof(CollapseItem) + 255u) & ~(size_t)255u);
+    if (!ctx->buildScratch.reserve(bytes)) return -3;
+    uint8_t* base = ctx->buildScratch.ptr;
+    Aabb *boxes = (Aabb*)(base + aBoxes), *triBoxes = (Aabb*)(base + aTriBoxes);
+    uint32_t *nodeCounts = (uint32_t*)(base + aNodeCounts), *valsSorted = (uint32_t*)(base + aValsSorted),
+             *vals = (uint32_t*)(base + aVals), *small = (uint32_t*)(base + aSmall), *levels = (uint32_t*)(base + aLevels);
+    uint32_t* clusters[2] = {(uint32_t*)(base + aClusters0), (uint32_t*)(base + aClusters1)};
+    uint64_t *keys = (uint64_t*)(base + aKeys), *keysSorted = (uint64_t*)(base + aKeysSorted);
+    int2* children = (int2*)(base + aChildren);
+    int* nn = (int*)(base + aNn);
+    uint8_t* keep = base + aKeep;
+    CollapseItem* front[2] = {(CollapseItem*)(base + aFront0), (CollapseItem*)(base + aFront1)};
+    void* temp = base + aTemp;
+    uint32_t *cb = small, *nodeCounter = small + 6, *selected = small + 7, *counts = small + 8;
+    auto cleanup = [&]() {
+        if (ctx->buildScratch.capacity > kKeepScratch) ctx->buildScratch.release();
+    };
+    // 1-3: bounds, Morton codes, sort
+    hipLaunchKernelGGL(kInitBuild, dim3(1), dim3(64), 0, s, cb, nodeCounter, n);
+    hipLaunchKernelGGL(kTriBounds, dim3(std::min(blocks(n), kBoundsBlocks)), dim3(kB), 0, s, ctx->worldTris.ptr, n,
+                       triBoxes, cb);
+    hipLaunchKernelGGL(kMorton, dim3(blocks(n)), dim3(kB), 0, s, triBoxes, n, cb, keys, vals);
+    rocprim::radix_sort_pairs(temp, sortBytes, keys, keysSorted, vals, valsSorted, n, 0, 63, s);
 
     // 4: PLOC
-    hipLaunchKernelGGL(kPlocInit, dim3(blocks(n)), dim3(kB), 0, s, triBoxes.ptr, valsSorted.ptr, n, boxes.ptr,
-                       nodeCounts.ptr, clusters[0].ptr);
-    uint32_t nodeCounterInit = n;
-    hipMemcpyAsync(counts.ptr + 3, &nodeCounterInit, sizeof(uint32_t), hipMemcpyHostToDevice, s);
+    hipLaunchKernelGGL(kPlocInit, dim3(blocks(n)), dim3(kB), 0, s, triBoxes, valsSorted, n, boxes, nodeCounts,
+                       clusters[0]);
     uint32_t m = n;
     int cur = 0;
     uint32_t passes = 0;
     while (m > 1) {
-        hipLaunchKernelGGL(kPlocNearest, dim3(blocks(m)), dim3(kB), 0, s, clusters[cur].ptr, m, boxes.ptr, nn.ptr);
-        hipLaunchKernelGGL(kPlocMerge, dim3(blocks(m)), dim3(kB), 0, s, clusters[cur].ptr, m, nn.ptr, boxes.ptr,
-                           nodeCounts.ptr, children.ptr, n, counts.ptr + 3, keep.ptr);
-        size_t bytes = selectBytes;
-        rocprim::select(temp, bytes, clusters[cur].ptr, keep.ptr, clusters[1 - cur].ptr, selected.ptr, (size_t)m, s);
+        const bool last = m <= (uint32_t)kPlocSmall;
+        if (last) {
+            hipLaunchKernelGGL(kPlocFinish, dim3(1), dim3(kPlocThreads), 0, s, clusters[cur], m, boxes, nodeCounts,
+                               children, n, nodeCounter, selected);
+        } else {
+            hipLaunchKernelGGL(kPlocNearest, dim3(blocks(m)), dim3(kB), 0, s, clusters[cur], m, boxes, nn);
+            hipLaunchKernelGGL(kPlocMerge, dim3(blocks(m)), dim3(kB), 0, s, clusters[cur], m, nn, boxes, nodeCounts,
+                               children, n, nodeCounter, keep);
+            size_t tempBytes = selectBytes;
+            rocprim::select(temp, tempBytes, clusters[cur], keep, clusters[1 - cur], selected, (size_t)m, s);
+            cur = 1 - cur;
+        }
         uint32_t next = 0;
-        if (!check(hipMemcpyAsync(&next, selected.ptr, sizeof(uint32_t), hipMemcpyDeviceToHost, s), "ploc count") ||
+        if (!check(hipMemcpyAsync(&next, selected, sizeof(uint32_t), hipMemcpyDeviceToHost, s), "ploc count") ||
             !check(hipStreamSynchronize(s), "ploc sync")) {
             cleanup();
             return -4;
         }
-        cur = 1 - cur;
         passes++;
-        if (next >= m || passes > 100000u) {  // every pass merges at least one pair
+        if (next >= m || passes > 100000u || (last && next != 1u)) {  // every pass merges at least one pair
             cleanup();
             setError("BVH clustering made no progress");
             return -5;
@@ -456,12 +621,12 @@ extern "C" int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats) {
     // the root cluster's box, padded outward by 1e-5 of its size and coordinates
     // so that rounding in the rays' slab test can never reject a ray that
     // reaches a triangle
+    Aabb rb{};
     {
         uint32_t root = 0;
-        Aabb rb{};
-        if (!check(hipMemcpyAsync(&root, clusters[cur].ptr, sizeof(root), hipMemcpyDeviceToHost, s), "root") ||
+        if (!check(hipMemcpyAsync(&root, clusters[cur], sizeof(root), hipMemcpyDeviceToHost, s), "root") ||
             !check(hipStreamSynchronize(s), "root sync") ||
-            !check(hipMemcpy(&rb, boxes.ptr + root, sizeof(rb), hipMemcpyDeviceToHost), "root box")) {
+            !check(hipMemcpy(&rb, boxes + root, sizeof(rb), hipMemcpyDeviceToHost), "root box")) {
             cleanup();
             return -4;
         }
@@ -473,48 +638,74 @@ extern "C" int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats) {
         }
     }
 
-    // 5: collapse into 8-wide nodes, writing triangle records in leaf order
-    hipLaunchKernelGGL(kInitCollapse, dim3(1), dim3(1), 0, s, front[0].ptr, counts.ptr, clusters[cur].ptr);
-    uint32_t depth = 0;
+    // 5: collapse into 8-wide nodes, writing triangle records in leaf order. A level's
+    // length is read by the next level's launch; the host looks after every few levels
+    hipLaunchKernelGGL(kInitCollapse, dim3(1), dim3(kB), 0, s, front[0], counts, levels, clusters[cur]);
+    uint32_t depth = 0, launched = 0, hostCounts[2] = {1, 0}, lengths[8];
+    uint64_t bound = 1;  // of a level's length
     int fc = 0;
-    uint32_t hostCounts[4] = {1, 0, 1, 0};
-    while (true) {
-        uint32_t frontier = hostCounts[0];
-        if (frontier == 0) break;
-        depth++;
-        hipMemsetAsync(counts.ptr + 1, 0, sizeof(uint32_t), s);
-        hipLaunchKernelGGL(kCollapse, dim3(blocks(frontier)), dim3(kB), 0, s, front[fc].ptr, counts.ptr,
-                           front[1 - fc].ptr, counts.ptr + 1, counts.ptr + 2, n, children.ptr, nodeCounts.ptr,
-                           boxes.ptr, valsSorted.ptr, ctx->worldTris.ptr, ctx->tris.ptr, ctx->nodes.ptr,
-                           (uint32_t)wideCap, counts.ptr + 3, n > kLargeScene ? kLeafMaxTrisLarge : kLeafMaxTris);
-        // the next frontier becomes the current one
-        hipMemcpyAsync(counts.ptr, counts.ptr + 1, sizeof(uint32_t), hipMemcpyDeviceToDevice, s);
-        if (!check(hipMemcpyAsync(hostCounts, counts.ptr, sizeof(hostCounts), hipMemcpyDeviceToHost, s), "collapse") ||
+    while (launched < kMaxLevels) {
+        const uint32_t batch = 4;
+        for (uint32_t l = 0; l < batch; l++) {
+            const uint32_t grid = std::min(blocks((size_t)bound * 8u), 8192u);
+            hipLaunchKernelGGL(kCollapse, dim3(grid), dim3(kB), 0, s, front[fc], levels + launched, front[1 - fc],
+                               levels + launched + 1u, counts, n, children, nodeCounts, boxes, valsSorted,
+                               ctx->worldTris.ptr, ctx->tris.ptr, ctx->nodes.ptr, (uint32_t)wideCap, counts + 1,
+                               n > kLargeScene ? kLeafMaxTrisLarge : kLeafMaxTris);
+            fc = 1 - fc;
+            launched++;
+            bound = std::min<uint64_t>(bound * 8u, n);
+        }
+        if (!check(hipMemcpyAsync(lengths, levels + launched - batch, (batch + 1u) * 4u, hipMemcpyDeviceToHost, s),
+                   "collapse") ||
+            !check(hipMemcpyAsync(hostCounts, counts, sizeof(hostCounts), hipMemcpyDeviceToHost, s), "collapse") ||
             !check(hipStreamSynchronize(s), "collapse sync")) {
             cleanup();
             return -4;
         }
-        fc = 1 - fc;
-        if (depth > 4096) break;
+        for (uint32_t l = 0; l < batch; l++) depth += lengths[l] != 0u;
+        if (lengths[batch] == 0u) break;
     }
     hipEventRecord(ctx->evStage[1], s);
     hipStreamSynchronize(s);
-    if (hostCounts[3] != 0) {
-        cleanup();
+    cleanup();
+    if (hostCounts[1] != 0) {
         setError("BVH collapse exceeded node capacity");
         return -5;
     }
-    ctx->nodes.count = hostCounts[2];
+    ctx->nodes.count = hostCounts[0];
     ctx->tris.count = n;
     ctx->bvhMaxDepth = depth;
     float ms = 0.0f;
     hipEventElapsedTime(&ms, ctx->evStage[0], ctx->evStage[1]);
     if (stats) {
         stats->buildMs = ms;
-        stats->nodeCount = hostCounts[2];
+        stats->nodeCount = hostCounts[0];
         stats->leafTriangles = n;
         stats->maxDepth = depth;
+        for (int a = 0; a < 3; a++) {
+            stats->boxMin[a] = rb.lo[a];
+            stats->boxMax[a] = rb.hi[a];
+        }
     }
-    cleanup();
     return check(hipGetLastError(), "bvh build") ? 0 : -4;
+}
+
+extern "C" int mrt_place_triangles(mrt_context* ctx, const float* transforms, uint32_t meshCount) {
+    if (!ctx || (meshCount && !transforms)) return -1;
+    if (!check(hipSetDevice(ctx->device), "hipSetDevice")) return -2;
+    const uint32_t n = ctx->triCount;
+    if (meshCount != ctx->meshes.count || meshCount != ctx->meshTriBase.count) {
+        setError("mrt_place_triangles: mesh count differs from the uploaded geometry");
+        return -1;
+    }
+    if (!ctx->worldTris.reserve((size_t)n * 9u) || !ctx->meshTransforms.upload(transforms, (size_t)meshCount * 16u, ctx->stream))
+        return -3;
+    ctx->worldTris.count = (size_t)n * 9u;
+    if (n > 0)
+        hipLaunchKernelGGL(kPlaceTriangles, dim3(blocks(n)), dim3(kB), 0, ctx->stream, ctx->vertices.ptr,
+                           ctx->indices.ptr, ctx->meshes.ptr, ctx->triMesh.ptr, ctx->meshTriBase.ptr,
+                           ctx->meshTransforms.ptr, n, ctx->worldTris.ptr);
+    ctx->shadeTrisDirty = true;
+    return check(hipGetLastError(), "place triangles") && check(hipStreamSynchronize(ctx->stream), "place triangles") ? 0 : -4;
 }

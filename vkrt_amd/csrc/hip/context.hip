@@ -77,6 +77,8 @@ extern "C" void mrt_destroy(mrt_context* ctx) {
     ctx->texels.release();
     ctx->texInfo.release();
     ctx->meshTriBase.release();
+    ctx->meshTransforms.release();
+    ctx->buildScratch.release();
     ctx->tris.release();
     ctx->nodes.release();
     ctx->shadeTris.release();
@@ -165,7 +167,6 @@ extern "C" int mrt_upload_geometry(mrt_context* ctx, const mrt_geometry_desc* g)
         return -1;
     }
     bool ok = ctx->vertices.upload(g->vertices, g->vertexCount, s) && ctx->indices.upload(g->indices, g->indexCount, s) &&
-              ctx->worldTris.upload(g->worldTriangles, (size_t)g->triangleCount * 9u, s) &&
               ctx->triMesh.upload(g->triangleMesh, g->triangleCount, s) &&
               ctx->meshTriBase.upload(g->meshTriangleBase, g->meshCount, s);
     if (!ok) return -3;
@@ -182,7 +183,6 @@ extern "C" int mrt_upload_meshes(mrt_context* ctx, const MeshInfo* meshInfos, ui
     if (!ctx->meshes.upload(meshInfos, meshCount, ctx->stream)) return -3;
     ctx->shadeTrisDirty = true;
     ctx->triClassDirty = true;
-    ctx->hintPaths = 0;
     return sync(ctx, "upload meshes");
 }
 

@@ -96,6 +96,8 @@ struct mrt_context {
     mrt::DeviceArray<ShaderVertex> vertices;
     mrt::DeviceArray<uint32_t> indices;
     mrt::DeviceArray<float> worldTris;
+    mrt::DeviceArray<float> meshTransforms;  // 16 floats per mesh, column-major
+    mrt::DeviceArray<uint8_t> buildScratch;  // of the BVH build, kept while it is small
     mrt::DeviceArray<uint32_t> triMesh;
     mrt::DeviceArray<uint32_t> triAlpha;  // per-triangle alpha words, valid when alphaEnabled
     bool alphaEnabled = false;

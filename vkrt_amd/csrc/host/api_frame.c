@@ -104,6 +104,7 @@ VKRT_Result VKRT_initWithCreateInfo(VKRT* vkrt, const VKRT_CreateInfo* createInf
     }
     /* force a full upload on the first frame */
     vkrt->geometryUploaded = vkrt->geometryRevision - 1u;
+    vkrt->meshDataUploaded = vkrt->meshDataRevision - 1u;
     vkrt->materialUploaded = vkrt->materialRevision - 1u;
     vkrt->environmentUploaded = vkrt->environmentRevision - 1u;
     vkrtResetSceneData(vkrt);
@@ -130,6 +131,7 @@ static VKRT_Result deviceError(void) {
 /* Re-packs and uploads whatever changed since the last upload. */
 static VKRT_Result syncScene(VKRT* vkrt, int requireDevice) {
     int geometryDirty = vkrt->geometryUploaded != vkrt->geometryRevision;
+    int meshDataDirty = vkrt->meshDataUploaded != vkrt->meshDataRevision;
     int materialDirty = vkrt->materialUploaded != vkrt->materialRevision;
     int envDirty = vkrt->environmentUploaded != vkrt->environmentRevision;
     if (!geometryDirty && !materialDirty && !envDirty && vkrt->packed.meshInfos) return VKRT_SUCCESS;
@@ -146,9 +148,20 @@ static VKRT_Result syncScene(VKRT* vkrt, int requireDevice) {
     }
     PackedScene* p = &vkrt->packed;
     if (geometryDirty) {
-        mrt_geometry_desc g = {p->vertices, p->vertexCount, p->indices, p->indexCount, p->worldTriangles,
-                               p->triangleMesh, p->triangleCount, p->meshTriangleBase, vkrt->meshCount};
-        if (mrt_upload_geometry(vkrt->device, &g) != 0) return deviceError();
+        if (vkrt->meshDataUploaded != vkrt->meshDataRevision) {
+            mrt_geometry_desc g = {p->vertices,      p->vertexCount,      p->indices,     p->indexCount, p->triangleMesh,
+                                   p->triangleCount, p->meshTriangleBase, vkrt->meshCount};
+            if (mrt_upload_geometry(vkrt->device, &g) != 0) return deviceError();
+            vkrt->meshDataUploaded = vkrt->meshDataRevision;
+        }
+        if (mrt_upload_meshes(vkrt->device, p->meshInfos, vkrt->meshCount) != 0) return deviceError();
+        float* transforms = (float*)malloc(sizeof(float) * 16u * (vkrt->meshCount ? vkrt->meshCount : 1u));
+        if (!transforms) return VKRT_ERROR_OUT_OF_MEMORY;
+        for (uint32_t i = 0; i < vkrt->meshCount; i++)
+            memcpy(transforms + 16u * i, vkrt->meshes[i].worldTransform, sizeof(float) * 16u);
+        const int placed = mrt_place_triangles(vkrt->device, transforms, vkrt->meshCount);
+        free(transforms);
+        if (placed != 0) return deviceError();
         mrt_bvh_stats bs;
         memset(&bs, 0, sizeof(bs));
         if (mrt_build_bvh(vkrt->device, &bs) != 0) return deviceError();
@@ -159,27 +172,17 @@ static VKRT_Result syncScene(VKRT* vkrt, int requireDevice) {
         vkrt->stats.triangleCount = p->triangleCount;
         /* scene box (the neural cache's position input is normalised by it) */
         for (int a = 0; a < 3; a++) {
-            vkrt->sceneMin[a] = 0.0f;
-            vkrt->sceneMax[a] = 1.0f;
-        }
-        for (uint32_t t = 0; t < p->triangleCount; t++) {
-            for (int v = 0; v < 3; v++) {
-                const float* q = p->worldTriangles + 9u * t + 3u * v;
-                for (int a = 0; a < 3; a++) {
-                    if (t == 0 && v == 0) vkrt->sceneMin[a] = vkrt->sceneMax[a] = q[a];
-                    if (q[a] < vkrt->sceneMin[a]) vkrt->sceneMin[a] = q[a];
-                    if (q[a] > vkrt->sceneMax[a]) vkrt->sceneMax[a] = q[a];
-                }
-            }
+            vkrt->sceneMin[a] = p->triangleCount ? bs.boxMin[a] : 0.0f;
+            vkrt->sceneMax[a] = p->triangleCount ? bs.boxMax[a] : 1.0f;
         }
     }
     if (mrt_upload_materials(vkrt->device, p->materials, p->materialCount) != 0) return deviceError();
-    if ((geometryDirty || materialDirty) && mrt_upload_alpha(vkrt->device, p->triangleAlpha, p->triangleCount) != 0)
+    if ((meshDataDirty || materialDirty) && mrt_upload_alpha(vkrt->device, p->triangleAlpha, p->triangleCount) != 0)
         return deviceError();
-    if ((geometryDirty || materialDirty) &&
+    if ((meshDataDirty || materialDirty) &&
         mrt_upload_textures(vkrt->device, p->textureTexels, p->textureTexelCount, p->textureInfo, p->textureCount) != 0)
         return deviceError();
-    if (mrt_upload_meshes(vkrt->device, p->meshInfos, vkrt->meshCount) != 0) return deviceError();
+    if (!geometryDirty && mrt_upload_meshes(vkrt->device, p->meshInfos, vkrt->meshCount) != 0) return deviceError();
     mrt_light_desc l = {p->emissiveMeshes, p->emissiveMeshCount, p->emissiveTriangles, p->emissiveTriangleCount,
                         p->meshAliasQ,     p->meshAliasIdx,      p->triAliasQ,         p->triAliasIdx,
                         p->emissiveMeshMaterial};
@@ -509,6 +512,7 @@ VKRT_Result VKRT_exportSceneBuffers(VKRT* vkrt, VKRT_SceneBuffers* out) {
     VKRT_Result r = vkrtLoadRGB2SpecTable(vkrt);
     if (r != VKRT_SUCCESS) return r;
     r = syncScene(vkrt, 0);
+    if (r == VKRT_SUCCESS) r = vkrtPackWorldTriangles(vkrt);
     if (r != VKRT_SUCCESS) return r;
     const PackedScene* p = &vkrt->packed;
     memset(out, 0, sizeof(*out));

@@ -122,6 +122,7 @@ VKRT_Result VKRT_uploadMeshDataBatch(VKRT* vkrt, const VKRT_MeshUpload* uploads,
         vkrt->meshCount++;
     }
     vkrt->geometryRevision++;
+    vkrt->meshDataRevision++;
     vkrtResetSceneData(vkrt);
     return VKRT_SUCCESS;
 }
@@ -140,6 +141,7 @@ VKRT_Result VKRT_removeMesh(VKRT* vkrt, uint32_t meshIndex) {
             sizeof(HostMesh) * (vkrt->meshCount - meshIndex - 1u));
     vkrt->meshCount--;
     vkrt->geometryRevision++;
+    vkrt->meshDataRevision++;
     vkrtResetSceneData(vkrt);
     return VKRT_SUCCESS;
 }

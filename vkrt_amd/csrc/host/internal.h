@@ -62,7 +62,7 @@ typedef struct PackedScene {
     float* triAliasQ;
     uint32_t* triAliasIdx;
     uint32_t* emissiveMeshMaterial; /* material of each emissive mesh (for emission gradients) */
-    float* worldTriangles;
+    float* worldTriangles; /* built when a caller exports the scene; the device places its own */
     uint32_t* triangleMesh;
     uint32_t* meshTriangleBase;
     uint32_t triangleCount;
@@ -112,9 +112,12 @@ struct VKRT {
 
     /* revision counters, compared with the uploaded revision like the
      * reference's *ResourceRevision pairs (src/core/api/frame.c:152-163) */
-    uint32_t geometryRevision, geometryUploaded;
+    uint32_t geometryRevision, geometryUploaded; /* meshes or their transforms */
+    uint32_t meshDataRevision, meshDataUploaded; /* vertices, indices and the list of meshes alone */
     uint32_t materialRevision, materialUploaded;
     uint32_t environmentRevision, environmentUploaded;
+    /* revisions that `packed` was built from */
+    uint32_t packedMeshData, packedMaterial, packedEnvironment;
     uint8_t accumulationNeedsReset;
 
     uint32_t rngPolicy;
@@ -139,6 +142,7 @@ struct VKRT {
 
 /* scene preparation (scene_prep.c) */
 VKRT_Result vkrtPrepareScene(VKRT* vkrt);
+VKRT_Result vkrtPackWorldTriangles(VKRT* vkrt);
 void vkrtFreePackedScene(PackedScene* packed);
 int vkrtBuildAliasTable(const float* pmf, uint32_t count, float* outQ, uint32_t* outIdx);
 ShaderVertex vkrtPackShaderVertex(const Vertex* vertex);

@@ -310,6 +310,7 @@ static VKRT_Result setSceneAside(VKRT* vkrt, SceneBackup* b) {
     vkrt->textureCount = vkrt->textureCapacity = 0;
     vkrt->settings.environmentTextureIndex = VKRT_INVALID_INDEX;
     vkrt->geometryRevision++;
+    vkrt->meshDataRevision++;
     vkrt->materialRevision++;
     vkrt->environmentRevision++;
     vkrtResetSceneData(vkrt);
@@ -341,6 +342,7 @@ static void restoreScene(VKRT* vkrt, SceneBackup* b) {
     vkrt->textureCapacity = b->textureCapacity;
     vkrt->settings = b->settings;
     vkrt->geometryRevision++;
+    vkrt->meshDataRevision++;
     vkrt->materialRevision++;
     vkrt->environmentRevision++;
     vkrtWriteSceneStateUniform(vkrt);

@@ -317,7 +317,9 @@ static VKRT_Result buildLights(VKRT* vkrt, PackedScene* p) {
     return VKRT_SUCCESS;
 }
 
-static VKRT_Result buildGeometry(VKRT* vkrt, PackedScene* p) {
+/* Packed vertices, indices and the triangle tables; `keep`: those of the last
+ * packed scene, whose meshes are the same. */
+static VKRT_Result buildGeometry(VKRT* vkrt, PackedScene* p, const PackedScene* keep) {
     uint64_t vcount = 0, icount = 0;
     for (uint32_t i = 0; i < vkrt->meshCount; i++) {
         vcount += vkrt->meshes[i].info.vertexCount;
@@ -327,13 +329,18 @@ static VKRT_Result buildGeometry(VKRT* vkrt, PackedScene* p) {
     p->vertexCount = (uint32_t)vcount;
     p->indexCount = (uint32_t)icount;
     p->triangleCount = (uint32_t)(icount / 3u);
-    p->vertices = (ShaderVertex*)malloc(sizeof(ShaderVertex) * (vcount ? vcount : 1));
-    p->indices = (uint32_t*)malloc(sizeof(uint32_t) * (icount ? icount : 1));
-    p->worldTriangles = (float*)malloc(sizeof(float) * 9u * (p->triangleCount ? p->triangleCount : 1u));
-    p->triangleMesh = (uint32_t*)malloc(sizeof(uint32_t) * (p->triangleCount ? p->triangleCount : 1u));
-    p->meshTriangleBase = (uint32_t*)malloc(sizeof(uint32_t) * (vkrt->meshCount ? vkrt->meshCount : 1u));
-    if (!p->vertices || !p->indices || !p->worldTriangles || !p->triangleMesh || !p->meshTriangleBase)
-        return VKRT_ERROR_OUT_OF_MEMORY;
+    if (keep) {
+        p->vertices = keep->vertices;
+        p->indices = keep->indices;
+        p->triangleMesh = keep->triangleMesh;
+        p->meshTriangleBase = keep->meshTriangleBase;
+    } else {
+        p->vertices = (ShaderVertex*)malloc(sizeof(ShaderVertex) * (vcount ? vcount : 1));
+        p->indices = (uint32_t*)malloc(sizeof(uint32_t) * (icount ? icount : 1));
+        p->triangleMesh = (uint32_t*)malloc(sizeof(uint32_t) * (p->triangleCount ? p->triangleCount : 1u));
+        p->meshTriangleBase = (uint32_t*)malloc(sizeof(uint32_t) * (vkrt->meshCount ? vkrt->meshCount : 1u));
+        if (!p->vertices || !p->indices || !p->triangleMesh || !p->meshTriangleBase) return VKRT_ERROR_OUT_OF_MEMORY;
+    }
 
     uint32_t vbase = 0, ibase = 0, tbase = 0;
     for (uint32_t mi = 0; mi < vkrt->meshCount; mi++) {
@@ -341,18 +348,13 @@ static VKRT_Result buildGeometry(VKRT* vkrt, PackedScene* p) {
         MeshInfo* info = &p->meshInfos[mi];
         info->vertexBase = vbase;
         info->indexBase = ibase;
-        p->meshTriangleBase[mi] = tbase;
-        for (uint32_t v = 0; v < info->vertexCount; v++) p->vertices[vbase + v] = vkrtPackShaderVertex(&mesh->vertices[v]);
-        memcpy(&p->indices[ibase], mesh->indices, sizeof(uint32_t) * info->indexCount);
         uint32_t tris = info->indexCount / 3u;
-        for (uint32_t t = 0; t < tris; t++) {
-            float* dst = &p->worldTriangles[(size_t)(tbase + t) * 9u];
-            for (int c = 0; c < 3; c++) {
-                uint32_t vi = mesh->indices[t * 3u + (uint32_t)c];
-                if (vi >= info->vertexCount) vi = 0; /* out-of-range indices collapse the triangle */
-                worldPoint(mesh->worldTransform, mesh->vertices[vi].position, &dst[c * 3]);
-            }
-            p->triangleMesh[tbase + t] = mi;
+        if (!keep) {
+            p->meshTriangleBase[mi] = tbase;
+            for (uint32_t v = 0; v < info->vertexCount; v++)
+                p->vertices[vbase + v] = vkrtPackShaderVertex(&mesh->vertices[v]);
+            memcpy(&p->indices[ibase], mesh->indices, sizeof(uint32_t) * info->indexCount);
+            for (uint32_t t = 0; t < tris; t++) p->triangleMesh[tbase + t] = mi;
         }
         vbase += info->vertexCount;
         ibase += info->indexCount;
@@ -361,7 +363,35 @@ static VKRT_Result buildGeometry(VKRT* vkrt, PackedScene* p) {
     return VKRT_SUCCESS;
 }
 
-static VKRT_Result buildEnvironmentTable(VKRT* vkrt, PackedScene* p) {
+/* World-space triangles of the packed scene, for export (the device places its
+ * own from the same vertices and transforms, mrt_place_triangles). */
+VKRT_Result vkrtPackWorldTriangles(VKRT* vkrt) {
+    PackedScene* p = &vkrt->packed;
+    if (p->worldTriangles) return VKRT_SUCCESS;
+    p->worldTriangles = (float*)malloc(sizeof(float) * 9u * (p->triangleCount ? p->triangleCount : 1u));
+    if (!p->worldTriangles) return VKRT_ERROR_OUT_OF_MEMORY;
+    for (uint32_t mi = 0; mi < vkrt->meshCount; mi++) {
+        const HostMesh* mesh = &vkrt->meshes[mi];
+        const uint32_t tris = mesh->info.indexCount / 3u;
+        for (uint32_t t = 0; t < tris; t++) {
+            float* dst = &p->worldTriangles[(size_t)(p->meshTriangleBase[mi] + t) * 9u];
+            for (int c = 0; c < 3; c++) {
+                uint32_t vi = mesh->indices[t * 3u + (uint32_t)c];
+                if (vi >= mesh->info.vertexCount) vi = 0; /* out-of-range indices collapse the triangle */
+                worldPoint(mesh->worldTransform, mesh->vertices[vi].position, &dst[c * 3]);
+            }
+        }
+    }
+    return VKRT_SUCCESS;
+}
+
+static VKRT_Result buildEnvironmentTable(VKRT* vkrt, PackedScene* p, const PackedScene* keep) {
+    if (keep) {
+        p->envAliasQ = keep->envAliasQ;
+        p->envAliasIdx = keep->envAliasIdx;
+        p->envPdf = keep->envPdf;
+        return VKRT_SUCCESS;
+    }
     uint32_t ti = vkrt->settings.environmentTextureIndex;
     if (ti == VKRT_INVALID_INDEX || ti >= vkrt->textureCount) return VKRT_SUCCESS;
     const HostTexture* tex = &vkrt->textures[ti];
@@ -416,7 +446,11 @@ static int meshSamplesTextureAlpha(const Material* m) {
     return m->alphaMode != VKRT_MATERIAL_ALPHA_MODE_OPAQUE && m->baseColorTextureIndex != VKRT_INVALID_INDEX;
 }
 
-static VKRT_Result buildTriangleAlpha(VKRT* vkrt, PackedScene* p) {
+static VKRT_Result buildTriangleAlpha(VKRT* vkrt, PackedScene* p, const PackedScene* keep) {
+    if (keep) {
+        p->triangleAlpha = keep->triangleAlpha;
+        return VKRT_SUCCESS;
+    }
     int any = 0;
     for (uint32_t mi = 0; mi < vkrt->meshCount && !any; mi++)
         any = meshMayRejectHit(&p->meshInfos[mi], &p->materials[p->meshInfos[mi].materialIndex]);
@@ -443,7 +477,7 @@ static VKRT_Result buildTriangleAlpha(VKRT* vkrt, PackedScene* p) {
 /* Texture indices a material holds that name no texture are treated as
  * empty slots; the pool then holds each referenced texture once, row-major
  * from row 0 (texture coordinate v = 0), as the device samples it. */
-static VKRT_Result buildTexturePool(VKRT* vkrt, PackedScene* p) {
+static VKRT_Result buildTexturePool(VKRT* vkrt, PackedScene* p, const PackedScene* keep) {
     uint32_t tc = vkrt->textureCount;
     for (uint32_t i = 0; i < p->materialCount; i++) {
         Material* m = &p->materials[i];
@@ -451,6 +485,13 @@ static VKRT_Result buildTexturePool(VKRT* vkrt, PackedScene* p) {
                               &m->emissiveTextureIndex};
         for (int k = 0; k < 4; k++)
             if (*slots[k] >= tc) *slots[k] = VKRT_INVALID_INDEX;
+    }
+    if (keep) {
+        p->textureTexels = keep->textureTexels;
+        p->textureTexelCount = keep->textureTexelCount;
+        p->textureInfo = keep->textureInfo;
+        p->textureCount = keep->textureCount;
+        return VKRT_SUCCESS;
     }
     if (tc == 0) return VKRT_SUCCESS;
     uint8_t* used = (uint8_t*)calloc(tc, 1);
@@ -520,17 +561,37 @@ VKRT_Result vkrtPrepareScene(VKRT* vkrt) {
         next.meshInfos[i] = vkrt->meshes[i].info;
         if (next.meshInfos[i].materialIndex >= next.materialCount) next.meshInfos[i].materialIndex = 0u;
     }
-    VKRT_Result r = buildGeometry(vkrt, &next);
+    /* what the last packed scene was built from and has not changed since stays */
+    PackedScene* last = &vkrt->packed;
+    const PackedScene* meshes = last->meshInfos && vkrt->packedMeshData == vkrt->meshDataRevision ? last : NULL;
+    const PackedScene* materials = meshes && vkrt->packedMaterial == vkrt->materialRevision ? last : NULL;
+    const PackedScene* environment =
+        last->meshInfos && vkrt->packedEnvironment == vkrt->environmentRevision ? last : NULL;
+    VKRT_Result r = buildGeometry(vkrt, &next, meshes);
     if (r == VKRT_SUCCESS) r = buildLights(vkrt, &next);
-    if (r == VKRT_SUCCESS) r = buildEnvironmentTable(vkrt, &next);
-    if (r == VKRT_SUCCESS) r = buildTexturePool(vkrt, &next);
-    if (r == VKRT_SUCCESS) r = buildTriangleAlpha(vkrt, &next);
-    if (r != VKRT_SUCCESS) {
-        vkrtFreePackedScene(&next);
-        return r;
+    if (r == VKRT_SUCCESS) r = buildEnvironmentTable(vkrt, &next, environment);
+    if (r == VKRT_SUCCESS) r = buildTexturePool(vkrt, &next, materials);
+    if (r == VKRT_SUCCESS) r = buildTriangleAlpha(vkrt, &next, materials);
+    /* the arrays that both hold belong to the one that stays */
+    PackedScene* gone = r == VKRT_SUCCESS ? last : &next;
+    if (meshes) {
+        gone->vertices = NULL;
+        gone->indices = gone->triangleMesh = gone->meshTriangleBase = NULL;
     }
-    vkrtFreePackedScene(&vkrt->packed);
+    if (environment) {
+        gone->envAliasQ = gone->envPdf = NULL;
+        gone->envAliasIdx = NULL;
+    }
+    if (materials) {
+        gone->textureTexels = NULL;
+        gone->textureInfo = gone->triangleAlpha = NULL;
+    }
+    vkrtFreePackedScene(gone);
+    if (r != VKRT_SUCCESS) return r;
     vkrt->packed = next;
+    vkrt->packedMeshData = vkrt->meshDataRevision;
+    vkrt->packedMaterial = vkrt->materialRevision;
+    vkrt->packedEnvironment = vkrt->environmentRevision;
     for (uint32_t i = 0; i < vkrt->meshCount; i++) vkrt->meshes[i].info.lightPdfArea = next.meshInfos[i].lightPdfArea;
     vkrt->sceneData.emissiveMeshCount = next.emissiveMeshCount;
     vkrt->sceneData.emissiveTriangleCount = next.emissiveTriangleCount;

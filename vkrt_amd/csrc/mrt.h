@@ -35,7 +35,6 @@ typedef struct mrt_geometry_desc {
     uint32_t vertexCount;
     const uint32_t* indices;
     uint32_t indexCount;
-    const float* worldTriangles; /* 9 floats per global triangle */
     const uint32_t* triangleMesh;
     uint32_t triangleCount;
     const uint32_t* meshTriangleBase; /* first global triangle of each mesh */
@@ -48,7 +47,11 @@ typedef struct mrt_bvh_stats {
     uint32_t nodeCount;
     uint32_t leafTriangles;
     uint32_t maxDepth;
+    float boxMin[3], boxMax[3]; /* of all triangles */
 } mrt_bvh_stats;
+/* World-space triangles of the uploaded geometry and meshes under `transforms`
+ * (16 floats per mesh, column-major), which the build reads. */
+int mrt_place_triangles(mrt_context* ctx, const float* transforms, uint32_t meshCount);
 int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats);
 
 int mrt_upload_meshes(mrt_context* ctx, const MeshInfo* meshInfos, uint32_t meshCount);
