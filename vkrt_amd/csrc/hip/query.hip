@@ -23,12 +23,8 @@ struct QueryOut {
 template <bool ANY, bool ALPHA>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? 4 : 6))) void kQuery(
     SceneView sv, const float4* rays, uint32_t n, uint32_t keyBase, QueryOut out, uint32_t* gstack, uint32_t* dropped) {
-    __shared__ uint32_t lds[kLdsStackWords];
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
-    st.sp = 0;
+    __shared__ uint2 lds[kLdsStackEntries];
+    TraversalStack st(lds, gstack);
     const uint32_t lane = threadIdx.x & 63u, stride = gridDim.x * kTraceBlock;
     const uint64_t lanesBelow = (1ull << lane) - 1ull;
     uint32_t run = (blockIdx.x * kTraceBlock + threadIdx.x) & ~63u, next = run, end = min(run + 64u, n);

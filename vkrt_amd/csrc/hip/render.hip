@@ -564,12 +564,8 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(TEX
                                                       float4 camO) {
     // camO.w != 0: the queue holds primary rays without stored origins; camO.xyz is theirs
     uint32_t nodeVisits = 0, triTests = 0;
-    __shared__ uint32_t lds[kLdsStackWords];
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
-    st.sp = 0;
+    __shared__ uint2 lds[kLdsStackEntries];
+    TraversalStack st(lds, gstack);
     const uint32_t n = queueTotal(count);
     if (n == 0u || sv.nodeCount == 0u) {
         // empty queue, or no geometry: every ray misses
@@ -668,12 +664,8 @@ template <int MODE, bool ALPHA>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? 4 : 6))) void kShadow(
     SceneView sv, PathView pv, ShadowView sh, uint32_t* counters, int fetchSlot, uint32_t envPass, uint32_t* gstack,
     uint32_t alphaSalt, uint32_t pathBase) {
-    __shared__ uint32_t lds[kLdsStackWords];
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
-    st.sp = 0;
+    __shared__ uint2 lds[kLdsStackEntries];
+    TraversalStack st(lds, gstack);
     const uint32_t n = queueTotal(sh.count);
     // wavefronts beyond one per 64 rays leave at once (see kExtend)
     if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
@@ -1261,12 +1253,8 @@ template <int MODE, bool NEE>
 __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneView sv, PathView pv, QueueView in,
                                                         ShadowView sh, ShadowView she, uint32_t* counters,
                                                         uint32_t startDepth, uint32_t* gstack) {
-    __shared__ uint32_t lds[kLdsStackWords];
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
-    st.sp = 0;
+    __shared__ uint2 lds[kLdsStackEntries];
+    TraversalStack st(lds, gstack);
     const uint32_t n = queueTotal(in.count);
     // wavefronts beyond one per 64 queued paths leave at once
     if ((blockIdx.x * (kTraceBlock / 64u) + (threadIdx.x >> 6)) * 64ull >= n) return;
@@ -1769,11 +1757,8 @@ __global__ void kFill4(float4* p, size_t n, float4 v) {
 __global__ __launch_bounds__(kTraceBlock) void kPrimary(SceneView sv, SceneData sd, uint32_t rngPolicy,
                                                        uint64_t rngSeed, uint32_t sampleIndex, uint32_t* outMesh,
                                                        uint32_t* outPrim, uint32_t* gstack) {
-    __shared__ uint32_t lds[kLdsStackWords];
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
+    __shared__ uint2 lds[kLdsStackEntries];
+    TraversalStack st(lds, gstack);
     uint32_t vw = sd.viewportRect[2], vh = sd.viewportRect[3];
     uint32_t n = vw * vh;
     for (uint32_t i = blockIdx.x * kTraceBlock + threadIdx.x; i < n; i += gridDim.x * kTraceBlock) {
@@ -1919,18 +1904,14 @@ __global__ __launch_bounds__(kBlock) void kAdjointInit(uint32_t count, PathView 
 __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, SceneView sv, PathView pv, QueueView in,
                                                             const float4* hits, QueueView out, uint32_t* counters,
                                                             uint32_t* gstack, AdjointView av) {
-    __shared__ uint32_t lds[kLdsStackWords];
+    __shared__ uint2 lds[kLdsStackEntries];
     extern __shared__ float gradLds[];
     GradSink sink{av.ldsMaterials ? gradLds : nullptr, &av};
     if (av.ldsMaterials) {
         for (uint32_t k = threadIdx.x; k < av.materialCount * 7u; k += kTraceBlock) gradLds[k] = 0.0f;
         __syncthreads();
     }
-    TraversalStack st;
-    st.lds = lds + threadIdx.x;
-    st.glob = gstack + (size_t)(blockIdx.x * kTraceBlock + threadIdx.x) * kGlobalStackWords;
-    st.dropped = 0;
-    st.sp = 0;
+    TraversalStack st(lds, gstack);
     // the grid is a multiple of kQueueParts blocks: a block stays in the part of its XCD
     const uint32_t part = blockIdx.x % kQueueParts, partLen = in.count[part * kPartStride];
     const uint32_t stride = gridDim.x / kQueueParts * kTraceBlock;
