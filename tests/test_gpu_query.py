@@ -91,3 +91,59 @@ def test_queries_without_geometry_miss():
         assert np.all(r.trace_shadow_rays(rays) == 1)
     finally:
         r.close()
+
+
+@pytest.mark.parametrize("axes", [(0,), (1,), (2,), (0, 1), (1, 2), (0, 2)])
+def test_rays_parallel_to_axis_planes_find_every_hit(axes):
+    """Directions with components of exactly (plus or minus) zero, from origins
+    between the triangles, on their vertices' coordinates and on the scene's
+    box: the closest hits of a brute-force search in 64 bits over the same 32-bit
+    coordinates, and an occlusion query that agrees."""
+    rng = np.random.default_rng(17)
+    n = 3000
+    pos = (rng.random((n, 1, 3)) + rng.normal(size=(n, 3, 3)) * 0.04).reshape(-1, 3).astype(np.float32)
+    count = 600
+    rays = np.zeros((count, 8), np.float32)
+    d = rng.normal(size=(count, 3))
+    d[:, list(axes)] = 0.0
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    d[::2, list(axes)] = -0.0
+    rays[:, 4:7] = d
+    rays[:, :3] = rng.uniform(0.1, 0.9, (count, 3)) - 3.0 * d
+    # a third of the origins lie exactly at a vertex's coordinate, a few at the box's faces
+    for a in axes:
+        rays[: count // 3, a] = pos[rng.integers(0, len(pos), count // 3), a]
+        rays[count // 3: count // 3 + 5, a] = pos[:, a].min()
+        rays[count // 3 + 5: count // 3 + 10, a] = pos[:, a].max()
+    rays[:, 3], rays[:, 7] = 1e-3, 1e4
+    s = scenes.Scene()
+    s.materials = [scenes.lambert((0.5, 0.5, 0.5))]
+    s.meshes.append(scenes.MeshData(V.make_vertices(pos, np.tile([[0.0, 0.0, 1.0]], (len(pos), 1))),
+                                    np.arange(3 * n, dtype=np.uint32).reshape(-1, 3), 0))
+    r = renderer(s)
+    try:
+        mesh, prim, t, _ = r.trace_rays(rays)
+        vis = r.trace_shadow_rays(rays)
+        v = pos.astype(np.float64).reshape(-1, 3, 3)
+        e1, e2 = v[:, 1] - v[:, 0], v[:, 2] - v[:, 0]
+        nrm = np.cross(e1, e2)
+        want = np.full(count, np.inf)
+        for i, ray in enumerate(rays.astype(np.float64)):
+            o, dd = ray[:3], ray[4:7]
+            ao = o - v[:, 0]
+            dao = np.cross(ao, dd)
+            with np.errstate(divide="ignore", invalid="ignore"):
+                det = -(nrm @ dd)
+                tt = (nrm * ao).sum(1) / det
+                u, w = (e2 * dao).sum(1) / det, -(e1 * dao).sum(1) / det
+                ok = (u >= 0) & (w >= 0) & (u + w <= 1) & (tt > ray[3]) & (tt < ray[7])
+            if ok.any():
+                want[i] = tt[ok].min()
+        hit = mesh != V.VKRT_INVALID_INDEX
+        # edges within 32-bit rounding may go either way, as for any ray (see test_gpu_build)
+        assert np.mean(hit != np.isfinite(want)) <= 5e-3
+        both = hit & np.isfinite(want)
+        assert both.mean() > 0.5 and np.mean(np.abs(t[both] - want[both]) > 1e-4) <= 5e-3
+        assert np.array_equal(vis == 1, ~hit)
+    finally:
+        r.close()

@@ -159,6 +159,7 @@ struct TraversalRay {
     F3 inv;      // 1/d
     F3 oInv;     // o/d, so entry distances are plane*inv - oInv
     bool negX, negY, negZ;
+    bool parallel;  // parallel to an axis plane: some component of inv is infinite
     RayPre pre;
 };
 
@@ -171,6 +172,7 @@ DEV TraversalRay makeTraversalRay(F3 o, F3 d) {
     r.negX = d.x < 0.0f;
     r.negY = d.y < 0.0f;
     r.negZ = d.z < 0.0f;
+    r.parallel = __builtin_isinf(r.inv.x) || __builtin_isinf(r.inv.y) || __builtin_isinf(r.inv.z);
     r.pre = rayPrecompute(d);
     return r;
 }
@@ -188,6 +190,7 @@ struct Children {
     uint32_t mask;  // children whose box the ray overlaps
 };
 
+DEV float comp4(const float4& v, int i) { return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w)); }
 DEV void setComp(float4& v, int i, float x) {
     if (i == 0) v.x = x;
     else if (i == 1) v.y = x;
@@ -242,6 +245,42 @@ DEV Children boxes8(const BvhNode* node, const TraversalRay& r, float tmin, floa
             setComp(c.dHi, i - 4, hit ? tnear : INFINITY);
     }
     return c;
+}
+
+// Children of a node that a ray parallel to an axis plane can meet: those whose
+// interval on that axis holds the ray's coordinate. The slab distances of that
+// axis are NaN (0 x inf) and constrain nothing in boxes8, so without this such a
+// ray visits every box that overlaps it on the other two axes, tens of
+// thousands in a large scene: one of them in a frame of 7.4M primary rays took
+// 7 of its launch's 8.4 ms, alone. The planes contain the child, and are widened here by
+// more than the rounding of their decoding.
+DEV uint32_t parallelMask(const BvhNode* node, const TraversalRay& r) {
+    uint32_t mask = 0xFFu;
+#pragma unroll 1
+    for (int a = 0; a < 3; a++) {
+        if (!__builtin_isinf(comp(r.inv, a))) continue;
+        const float org = a == 0 ? node->ox : (a == 1 ? node->oy : node->oz), o = comp(r.o, a);
+        const float step = __uint_as_float(((node->packed >> (8 * a)) & 0xFFu) << 23);
+        const float wide = 1e-6f * (fabsf(org) + fabsf(o) + 255.0f * step);
+        const uint32_t l0 = node->qlo[2 * a], l1 = node->qlo[2 * a + 1], h0 = node->qhi[2 * a], h1 = node->qhi[2 * a + 1];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float lo = fmaf(planeByte(l0, l1, i), step, org), hi = fmaf(planeByte(h0, h1, i), step, org);
+            if (lo > o + wide || hi < o - wide) mask &= ~(1u << i);
+        }
+    }
+    return mask;
+}
+
+DEV void dropChildren(Children& c, uint32_t keep) {
+    c.mask &= keep;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        if (i < 4)
+            setComp(c.dLo, i, keep & (1u << i) ? comp4(c.dLo, i) : INFINITY);
+        else
+            setComp(c.dHi, i - 4, keep & (1u << i) ? comp4(c.dHi, i - 4) : INFINITY);
+    }
 }
 
 // Sorts the children by entry distance (misses last) with a 19-comparator
@@ -348,6 +387,7 @@ DEV bool closestStep(const SceneView& s, const TraversalRay& r, float tmin, Clos
     if (!(cs.ref & kLeafBit)) {
         if (nodeVisits) (*nodeVisits)++;
         Children c = boxes8(s.nodes + cs.ref, r, tmin, cs.h.t);
+        if (r.parallel) dropChildren(c, parallelMask(s.nodes + cs.ref, r));
         const int hits = __popc(c.mask);
         if (hits > 0) {
             sortChildren(c);
@@ -418,31 +458,22 @@ DEV Hit traceClosest(const SceneView& s, const TraversalRay& r, float tmin, floa
     return cs.h;
 }
 
-// Any-hit traversal state of one ray.
-struct AnyState {
-    uint32_t ref, steps;
-    uint32_t tri;  // the hit, once the traversal has finished: a global triangle id or kNoHit
-};
-DEV void anyBegin(AnyState& as, TraversalStack& st) {
-    as.ref = 0;
-    as.steps = 0;
-    as.tri = kNoHit;
-    st.sp = 0;
-}
-
-// One node or leaf visit of an any-hit traversal in (tmin, tmax): the first
-// accepted intersection ends the search, as
+// One node or leaf visit of an any-hit traversal in (tmin, h.t) begun with
+// closestBegin: the first accepted intersection ends the search, as
 // RAY_FLAG_ACCEPT_FIRST_HIT_AND_END_SEARCH. Returns false once the traversal
-// has finished. ALPHA = false compiles the alpha test out.
+// has finished, h.tri then being a hit's triangle or kNoHit (h.t stays tmax).
+// ALPHA = false compiles the alpha test out.
 template <bool ALPHA = true>
-DEV bool anyStep(const SceneView& s, const TraversalRay& r, float tmin, float tmax, AnyState& as, TraversalStack& st,
+DEV bool anyStep(const SceneView& s, const TraversalRay& r, float tmin, ClosestState& as, TraversalStack& st,
                  uint32_t alphaKey) {
+    const float tmax = as.h.t;
     if (as.steps++ >= kMaxTraversalSteps) {
         st.dropped++;
         return false;
     }
     if (!(as.ref & kLeafBit)) {
-        const Children c = boxes8(s.nodes + as.ref, r, tmin, tmax);
+        Children c = boxes8(s.nodes + as.ref, r, tmin, tmax);
+        if (r.parallel) c.mask &= parallelMask(s.nodes + as.ref, r);
         if (c.mask != 0u) {
             // visit the lowest overlapping slot next, push the others
             const uint32_t m = c.mask;
@@ -467,7 +498,7 @@ DEV bool anyStep(const SceneView& s, const TraversalRay& r, float tmin, float tm
             if (intersectTriangle(tr, r.o, r.pre, tmin, tmax, t, u, v)) {
                 const uint32_t tri = __float_as_uint(tr.v0.w);
                 if (!ALPHA || !s.triAlpha || alphaAccept(s, tri, u, v, alphaKey)) {
-                    as.tri = tri;
+                    as.h.tri = tri;
                     return false;
                 }
             }
@@ -483,11 +514,11 @@ DEV bool anyStep(const SceneView& s, const TraversalRay& r, float tmin, float tm
 DEV uint32_t traceAny(const SceneView& s, const TraversalRay& r, float tmin, float tmax, TraversalStack& st,
                       uint32_t alphaKey) {
     if (s.nodeCount == 0) return kNoHit;
-    AnyState as;
-    anyBegin(as, st);
-    while (anyStep<true>(s, r, tmin, tmax, as, st, alphaKey)) {
+    ClosestState as;
+    closestBegin(as, st, tmax);
+    while (anyStep<true>(s, r, tmin, as, st, alphaKey)) {
     }
-    return as.tri;
+    return as.h.tri;
 }
 
 constexpr uint32_t kVisOccluded = 0u, kVisVisible = 1u, kVisUnsupported = 2u;

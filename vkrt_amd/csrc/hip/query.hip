@@ -29,12 +29,10 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
     const uint64_t lanesBelow = (1ull << lane) - 1ull;
     uint32_t run = (blockIdx.x * kTraceBlock + threadIdx.x) & ~63u, next = run, end = min(run + 64u, n);
     uint32_t rayId = kNoRay, alphaKey = 0u;
-    float tmin = 0.0f, tmax = 0.0f;
+    float tmin = 0.0f;
     TraversalRay r;
     ClosestState cs;
-    AnyState as;
     closestBegin(cs, st, 0.0f);
-    anyBegin(as, st);
     auto finish = [&](uint32_t i, const Hit& h) {
         if (ANY) {
             out.visibility[i] = classifyOccluder(sv, h.tri);
@@ -58,16 +56,12 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
             if (rayId == kNoRay && i < end) {
                 const float4 a = rays[2 * (size_t)i], b = rays[2 * (size_t)i + 1];
                 tmin = a.w;
-                tmax = b.w;
                 r = makeTraversalRay(xyz(a), xyz(b));
                 // no tree, or the ray misses the scene's box: a miss at once
-                if (sv.nodeCount != 0u && reachesSceneBox(sv, r, tmin, tmax)) {
+                if (sv.nodeCount != 0u && reachesSceneBox(sv, r, tmin, b.w)) {
                     // a query ray has no path: its index is its key
                     if (ALPHA) alphaKey = alphaRayKey(alphaSalt(0u, 0ull, 0u, 3u), keyBase + i);
-                    if (ANY)
-                        anyBegin(as, st);
-                    else
-                        closestBegin(cs, st, tmax);
+                    closestBegin(cs, st, b.w);
                     rayId = i;
                 } else {
                     finish(i, Hit{0.0f, kNoHit, 0.0f, 0.0f});
@@ -81,10 +75,10 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
             }
         }
         if (rayId != kNoRay) {
-            const bool more = ANY ? anyStep<ALPHA>(sv, r, tmin, tmax, as, st, alphaKey)
+            const bool more = ANY ? anyStep<ALPHA>(sv, r, tmin, cs, st, alphaKey)
                                   : closestStep<ALPHA, ALPHA>(sv, r, tmin, cs, st, alphaKey);
             if (!more) {
-                finish(rayId, ANY ? Hit{0.0f, as.tri, 0.0f, 0.0f} : cs.h);
+                finish(rayId, cs.h);
                 rayId = kNoRay;
             }
         }

@@ -673,10 +673,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
     const uint64_t lanesBelow = (1ull << lane) - 1ull;
     RayClaims claims(n);
     uint32_t rayId = kNoRay, path = 0u, alphaKey = 0u;
-    float tmax = 0.0f;
     TraversalRay r;
-    AnyState as;
-    anyBegin(as, st);
+    ClosestState cs;
+    closestBegin(cs, st, 0.0f);
     while (true) {
         const uint64_t idleMask = __ballot(rayId == kNoRay);
         const uint32_t idle = (uint32_t)__popcll(idleMask);
@@ -688,16 +687,15 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
                     rayId = queueSlot(claims.from, j);
                     const float4 o = sh.o[rayId], d = sh.d[rayId];
                     path = __float_as_uint(o.w);
-                    tmax = d.w;
                     r = makeTraversalRay(xyz(o), xyz(d));
                     if (ALPHA) alphaKey = alphaRayKey(alphaSalt, pathBase + path);
-                    anyBegin(as, st);
+                    closestBegin(cs, st, d.w);
                 }
             }
         }
-        if (rayId != kNoRay && !anyStep<ALPHA>(sv, r, kRayTMin, tmax, as, st, alphaKey)) {
+        if (rayId != kNoRay && !anyStep<ALPHA>(sv, r, kRayTMin, cs, st, alphaKey)) {
             const uint32_t vis =
-                envPass ? (as.tri == kNoHit ? kVisVisible : kVisOccluded) : classifyOccluder(sv, as.tri);
+                envPass ? (cs.h.tri == kNoHit ? kVisVisible : kVisOccluded) : classifyOccluder(sv, cs.h.tri);
             if (vis == kVisVisible || !envPass)  // b is zero for environment rays
                 addShadowed<MODE>(pv, path, vis, ld4(vis == kVisVisible ? sh.a[rayId] : sh.b[rayId]));
             rayId = kNoRay;
@@ -1265,12 +1263,9 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
     RayClaims claims(n);
     float4 ro = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rd = ro;
     bool cont = false, shadowEmit = false, envEmit = false;
-    float shadowT = 0.0f;
     TraversalRay r;
-    ClosestState cs;
-    AnyState as;
+    ClosestState cs;  // of the lane's ray, closest hit or any hit
     closestBegin(cs, st, 0.0f);
-    anyBegin(as, st);
     // start the traversal of the lane's ray (ro, rd): a ray that misses the
     // scene's box (or a scene without geometry) has its miss at once
     auto beginRay = [&]() {
@@ -1296,9 +1291,8 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
             envEmit = envEmit && light;
             shadowEmit = false;
             r = makeTraversalRay(xyz(o), xyz(d));
-            shadowT = d.w;
             shadowed++;
-            anyBegin(as, st);
+            closestBegin(cs, st, d.w);
         } else if (cont) {
             depth++;
             traced++;
@@ -1328,10 +1322,11 @@ __global__ __launch_bounds__(kTraceBlock, 2) void kTail(FrameParams fp, SceneVie
             }
         }
         if (state == kTrace && !closestStep<false, false>(sv, r, kRayTMin, cs, st, 0u)) state = kReady;
-        if (NEE && state >= kLight && !anyStep<false>(sv, r, kRayTMin, shadowT, as, st, 0u)) {
+        if (NEE && state >= kLight && !anyStep<false>(sv, r, kRayTMin, cs, st, 0u)) {
             const uint32_t q = __float_as_uint(ro.w);
             const bool light = state == kLight;
-            const uint32_t vis = light ? classifyOccluder(sv, as.tri) : (as.tri == kNoHit ? kVisVisible : kVisOccluded);
+            const uint32_t vis =
+                light ? classifyOccluder(sv, cs.h.tri) : (cs.h.tri == kNoHit ? kVisVisible : kVisOccluded);
             if (light || vis == kVisVisible)  // an occluded environment ray adds nothing
                 addShadowed<MODE>(pv, q, vis, ld4(light ? (vis == kVisVisible ? sh.a[q] : sh.b[q]) : she.a[q]));
             beginNext();
