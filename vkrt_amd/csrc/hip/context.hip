@@ -82,6 +82,7 @@ extern "C" void mrt_destroy(mrt_context* ctx) {
     ctx->tris.release();
     ctx->nodes.release();
     ctx->shadeTris.release();
+    ctx->meshFrames.release();
     ctx->triClass.release();
     ctx->meshes.release();
     ctx->materials.release();

@@ -45,7 +45,19 @@ DEV F4 operator/(F4 a, float s) { return F4{a.x / s, a.y / s, a.z / s, a.w / s};
 
 DEV float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 DEV F3 cross(F3 a, F3 b) { return F3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
-DEV float rsq(float x) { return 1.0f / sqrtf(x); }
+// 1 / sqrtf(x), root and reciprocal each correctly rounded as the compiler's
+// are: the same bits for all 2^32 arguments (compared on the device). Inside
+// [2^-100, 2^100) by the hardware's estimates with one correction from the exact
+// remainder each, 8 operations for about 30, without the scaling and fix-ups
+// that only the ends of the range need. A hit takes some sixteen of these.
+DEV float rsq(float x) {
+    if (__float_as_uint(x) - 0x0d800000u >= 0x71800000u - 0x0d800000u) return 1.0f / sqrtf(x);
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s0 = x * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0);
+    const float r = __builtin_amdgcn_rcpf(s);
+    return __builtin_fmaf(__builtin_fmaf(-s, r, 1.0f), r, r);
+}
 DEV F3 normalize(F3 a) { return a * rsq(dot(a, a)); }
 DEV float sat(float x) { return fminf(fmaxf(x, 0.0f), 1.0f); }
 DEV F3 sat(F3 a) { return F3{sat(a.x), sat(a.y), sat(a.z)}; }
@@ -136,6 +148,19 @@ struct alignas(16) ShadeTri {
 };
 static_assert(sizeof(ShadeTri) == 64, "ShadeTri layout");
 
+// What a hit reads of its mesh, 64 bytes, built with the shading records: the
+// sines and cosines of the Euler rotation, the scale and its reciprocals are
+// the same for every hit of a mesh and cost six trigonometric functions and
+// three divisions each time otherwise.
+struct alignas(16) MeshFrame {
+    float sinX, cosX, sinY, cosY;
+    float sinZ, cosZ, scaleX, scaleY;
+    float scaleZ, invX, invY, invZ;  // reciprocal scale, bounded (safeSignedRcp)
+    uint32_t materialIndex;
+    uint32_t pad[3];
+};
+static_assert(sizeof(MeshFrame) == 64, "MeshFrame layout");
+
 // What the kernels read of the scene. Passed by value as a kernel argument.
 struct SceneView {
     const BvhNode* nodes;
@@ -164,6 +189,7 @@ struct SceneView {
     const float* envPdf;
     const float* rgb2spec;
     const ShadeTri* shadeTris;
+    const MeshFrame* meshFrames;
     const uint32_t* triAlpha;  // per-triangle alpha words; nullptr when every mesh is opaque
     const float4* texels;      // material texture pool; nullptr when no material has a texture
     const uint4* texInfo;      // per texture: first texel, width, height

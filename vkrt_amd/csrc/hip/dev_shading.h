@@ -112,6 +112,16 @@ DEV F3 safeNormalize(F3 v) {
 
 // -------------------------------------------------------------- packing --
 // src/shaders/geometry/packing.slang:13-56
+// v / N, correctly rounded, for a whole number v of 16 bits: the product with
+// the rounded reciprocal and one correction from the exact remainder give the
+// quotient of a full division for each of these v (three operations for about
+// eleven; a hit unpacks twelve such numbers).
+template <int N>
+DEV float divConst(float v) {
+    constexpr float r = 1.0f / (float)N;
+    const float q = v * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, (float)N, v), r, q);
+}
 DEV F3 decodeOct(float px, float py) {
     float z = 1.0f - fabsf(px) - fabsf(py);
     if (z < 0.0f) {
@@ -124,12 +134,12 @@ DEV F3 decodeOct(float px, float py) {
 DEV F3 unpackOctNormal(uint32_t p) {
     int32_t x = (int32_t)(p << 16) >> 16;
     int32_t y = (int32_t)p >> 16;
-    return decodeOct((float)x / 32767.0f, (float)y / 32767.0f);
+    return decodeOct(divConst<32767>((float)x), divConst<32767>((float)y));
 }
 DEV float unpackSnorm15(uint32_t v) {
     int32_t s = (int32_t)(v & 0x7fffu);
     if (s & 0x4000) s |= ~(int32_t)0x7fff;
-    return clampf((float)s / 16383.0f, -1.0f, 1.0f);
+    return clampf(divConst<16383>((float)s), -1.0f, 1.0f);
 }
 DEV F4 unpackOctTangent(uint32_t p) {
     F3 d = decodeOct(unpackSnorm15(p), unpackSnorm15(p >> 15u));
@@ -143,27 +153,37 @@ DEV F4 unpackColor(uint32_t p) {
 
 // ----------------------------------------------------------- transforms --
 // src/shaders/geometry/surface/transform.slang:9-55
-DEV F3 rotateMesh(F3 v, const MeshInfo& m) {
-    const float d2r = 0.01745329251994329577f;
-    float ax = m.rotation[0] * d2r, ay = m.rotation[1] * d2r, az = m.rotation[2] * d2r;
-    float s = sinf(ax), c = cosf(ax);
-    v = F3{v.x, c * v.y - s * v.z, s * v.y + c * v.z};
-    s = sinf(ay);
-    c = cosf(ay);
-    v = F3{c * v.x + s * v.z, v.y, -s * v.x + c * v.z};
-    s = sinf(az);
-    c = cosf(az);
-    return F3{c * v.x - s * v.y, s * v.x + c * v.y, v.z};
-}
 DEV float safeSignedRcp(float v) {
     if (fabsf(v) > 1e-6f) return 1.0f / v;
     return v < 0.0f ? -1.0f / 1e-6f : 1.0f / 1e-6f;
 }
-DEV F3 meshVector(const MeshInfo& m, F3 v) { return rotateMesh(v * F3{m.scale[0], m.scale[1], m.scale[2]}, m); }
-DEV F3 meshNormal(const MeshInfo& m, F3 n) {
-    F3 inv = F3{safeSignedRcp(m.scale[0]), safeSignedRcp(m.scale[1]), safeSignedRcp(m.scale[2])};
-    return safeNormalize(rotateMesh(n * inv, m));
+DEV MeshFrame buildMeshFrame(const MeshInfo& m) {
+    const float d2r = 0.01745329251994329577f;
+    const float ax = m.rotation[0] * d2r, ay = m.rotation[1] * d2r, az = m.rotation[2] * d2r;
+    MeshFrame f;
+    f.sinX = sinf(ax);
+    f.cosX = cosf(ax);
+    f.sinY = sinf(ay);
+    f.cosY = cosf(ay);
+    f.sinZ = sinf(az);
+    f.cosZ = cosf(az);
+    f.scaleX = m.scale[0];
+    f.scaleY = m.scale[1];
+    f.scaleZ = m.scale[2];
+    f.invX = safeSignedRcp(m.scale[0]);
+    f.invY = safeSignedRcp(m.scale[1]);
+    f.invZ = safeSignedRcp(m.scale[2]);
+    f.materialIndex = m.materialIndex;
+    f.pad[0] = f.pad[1] = f.pad[2] = 0u;
+    return f;
 }
+DEV F3 rotateMesh(F3 v, const MeshFrame& f) {
+    v = F3{v.x, f.cosX * v.y - f.sinX * v.z, f.sinX * v.y + f.cosX * v.z};
+    v = F3{f.cosY * v.x + f.sinY * v.z, v.y, -f.sinY * v.x + f.cosY * v.z};
+    return F3{f.cosZ * v.x - f.sinZ * v.y, f.sinZ * v.x + f.cosZ * v.y, v.z};
+}
+DEV F3 meshVector(const MeshFrame& f, F3 v) { return rotateMesh(v * F3{f.scaleX, f.scaleY, f.scaleZ}, f); }
+DEV F3 meshNormal(const MeshFrame& f, F3 n) { return safeNormalize(rotateMesh(n * F3{f.invX, f.invY, f.invZ}, f)); }
 
 // -------------------------------------------------------------- surface --
 struct Basis {
@@ -225,9 +245,10 @@ DEV ShadeTri buildShadeTri(const SceneView& s, uint32_t tri) {
     const ShaderVertex v0 = s.vertices[s.indices[tb + 0] + m.vertexBase];
     const ShaderVertex v1 = s.vertices[s.indices[tb + 1] + m.vertexBase];
     const ShaderVertex v2 = s.vertices[s.indices[tb + 2] + m.vertexBase];
+    const MeshFrame f = s.meshFrames[mesh];
     F4 p0 = ldVertexPos(v0), p1 = ldVertexPos(v1), p2 = ldVertexPos(v2);
-    F3 e1 = meshVector(m, F3{p1.x - p0.x, p1.y - p0.y, p1.z - p0.z});
-    F3 e2 = meshVector(m, F3{p2.x - p0.x, p2.y - p0.y, p2.z - p0.z});
+    F3 e1 = meshVector(f, F3{p1.x - p0.x, p1.y - p0.y, p1.z - p0.z});
+    F3 e2 = meshVector(f, F3{p2.x - p0.x, p2.y - p0.y, p2.z - p0.z});
     F3 gn = safeNormalize(cross(e1, e2));
     if (m.scale[0] * m.scale[1] * m.scale[2] < 0.0f) gn = -gn;
     r.mesh = mesh;
@@ -258,7 +279,7 @@ DEV Surface reconstruct(const SceneView& s, F3 o, F3 d, const Hit& h) {
     const uint32_t mesh = w0.x;
     const F3 gn = F3{__uint_as_float(w0.y), __uint_as_float(w0.z), __uint_as_float(w0.w)};
     // normals w1.xyz, tangents w1.w w2.xy, colours w2.zw w3.x
-    const MeshInfo m = s.meshes[mesh];
+    const MeshFrame m = s.meshFrames[mesh];
     sf.p = o + d * h.t;
     F3 objN = safeNormalize(bary3(unpackOctNormal(w1.x), unpackOctNormal(w1.y), unpackOctNormal(w1.z), h.u, h.v));
     F4 objT = bary4(unpackOctTangent(w1.w), unpackOctTangent(w2.x), unpackOctTangent(w2.y), h.u, h.v);

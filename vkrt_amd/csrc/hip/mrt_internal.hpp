@@ -109,7 +109,8 @@ struct mrt_context {
     mrt::DeviceArray<mrt::TriRecord> tris;
     mrt::DeviceArray<mrt::BvhNode> nodes;
     mrt::DeviceArray<mrt::ShadeTri> shadeTris;
-    bool shadeTrisDirty = true;  // geometry or mesh transforms changed since the records were built
+    mrt::DeviceArray<mrt::MeshFrame> meshFrames;
+    bool shadeTrisDirty = true;  // geometry or mesh transforms changed since these were built
     mrt::DeviceArray<uint8_t> triClass;  // material class per triangle (shading sort)
     bool triClassDirty = true;
     mrt::DeviceArray<MeshInfo> meshes;
@@ -191,6 +192,7 @@ struct mrt_context {
         v.envPdf = envPdf.ptr;
         v.rgb2spec = rgb2spec.ptr;
         v.shadeTris = shadeTris.ptr;
+        v.meshFrames = meshFrames.ptr;
         v.triAlpha = alphaEnabled && triAlpha.count >= triCount ? triAlpha.ptr : nullptr;
         v.texels = texturesEnabled ? texels.ptr : nullptr;
         v.texInfo = texturesEnabled ? texInfo.ptr : nullptr;

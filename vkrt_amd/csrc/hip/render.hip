@@ -485,11 +485,11 @@ __global__ __launch_bounds__(kBlock) void kGenerate(FrameParams fp, PathView pv,
         }
         pv.rng[i] = storeRng(ps.rng);
         pv.flags[i] = flags;
-        pv.thr[i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        // hero: four lanes; otherwise the throughput and, in w, the last BSDF pdf
+        pv.thr[i] = make_float4(1.0f, 1.0f, 1.0f, MODE == kModeHero ? 1.0f : 0.0f);
         pv.rad[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        // hero paths write every field of misc when they collapse to one wavelength,
-        // before anything reads it
-        if (MODE != kModeHero) pv.misc[i] = make_float4(0.0f, 1.0f, 0.0f, 0.0f);
+        // misc is hero paths' alone, which write every field of it when they collapse to
+        // one wavelength, before anything reads it
         // sigma is read only inside an absorbing medium (kFAbsorption), after a transmission wrote it
     }
     if (FULL || !fp.compactPrimary) q.o[i] = make_float4(o.x, o.y, o.z, __uint_as_float(i));
@@ -763,14 +763,17 @@ __global__ __launch_bounds__(kBlock) void kNrcTargets(const float4* record, cons
 }
 
 // One path vertex for every ray of the current queue, at three waves per SIMD
-// (at most 168 registers). Every variant must fit that budget without spilling
-// registers to scratch: a hero build that spilled about 60 registers gave wrong
+// (at most 168 registers), RGB at four (128): the kernel waits on its gathers and
+// on long chains of dependent arithmetic, so a fourth wave is worth more than the
+// registers (1024x1024 16 spp, next-event estimation, shading of a frame: 5.75 ms at 131
+// registers and three waves, 5.42 with mesh frames and shorter unpacking, 4.64 at four).
+// Every variant must fit its budget without spilling registers to scratch: a hero build that spilled about 60 registers gave wrong
 // NEE results while the same source at two waves matched the oracle bit for
 // bit. What keeps the hero variant inside the budget: the rgb2spec resolution is
 // a compile-time constant, medium coefficients and the scalar-wavelength state
 // are read only where used, and shadow rays are queued before BSDF sampling.
-// Materials with sheen take SHEEN variants at two waves per SIMD: the sheen
-// layer does not fit the three-wave budget of the hero kernel.
+// Materials with sheen take SHEEN variants, hero at two waves per SIMD and the
+// others at three: the sheen layer does not fit the budgets above.
 // One path vertex: the ray (ro, rdir) of path q = bits of ro.w, at `depth`,
 // and its hit h. Leaves the continuation ray in nextO / nextD with cont set, or
 // cont false when the path ends here. Shadow records go to the part `part` (one
@@ -819,8 +822,16 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
         const bool heroActive = MODE == kModeHero && (flags & kFHeroActive) != 0u;
         F4 thr = first ? f4(1.0f) : ld4(pv.thr[q]);
         // prevBsdfPdf, scalar throughput, scalar wavelength, scalar 1/pdf; unused while
-        // all four hero wavelengths are alive
-        F4 misc = heroActive ? f4(0.0f) : (first ? F4{0.0f, 1.0f, 0.0f, 0.0f} : ld4(pv.misc[q]));
+        // all four hero wavelengths are alive. The other modes use the first alone and
+        // keep it in the lane of thr they have free: a record less to move per vertex,
+        // and three registers less through it
+        F4 misc = f4(0.0f);
+        if (MODE == kModeHero) {
+            if (!heroActive) misc = ld4(pv.misc[q]);
+        } else {
+            misc.x = first ? 0.0f : thr.w;
+            thr = MODE == kModeRgb ? F4{thr.x, thr.y, thr.z, 0.0f} : F4{thr.x, 0.0f, 0.0f, 0.0f};
+        }
 
         if (h.tri == kNoHit) {
             if (!fp.neeOnly && !(refractive || absorbing)) {
@@ -1191,8 +1202,8 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
         nextD = wi;
         cont = true;
         pv.rng[q] = storeRng(rng);
-        pv.thr[q] = st4(thr);
-        if (!nowHero) pv.misc[q] = st4(misc);
+        pv.thr[q] = MODE == kModeHero ? st4(thr) : make_float4(thr.x, thr.y, thr.z, misc.x);
+        if (MODE == kModeHero && !nowHero) pv.misc[q] = st4(misc);
         pv.flags[q] = newFlags;
         if (newFlags & kFAbsorption) pv.sigma[q] = st4(sigma);
         if (MODE == kModeHero) pv.tpp[q] = st4(tpp);
@@ -1200,7 +1211,8 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
 }
 
 template <int MODE, bool NRC = false, bool TEX = false, bool SHEEN = false>
-__global__ __launch_bounds__(kBlock, SHEEN ? 2 : 3) void kShade(FrameParams fp, SceneView sv, PathView pv, QueueView in,
+__global__ __launch_bounds__(kBlock, MODE == kModeHero ? (SHEEN ? 2 : 3)
+                                                              : (MODE == kModeRgb && !SHEEN ? 4 : 3)) void kShade(FrameParams fp, SceneView sv, PathView pv, QueueView in,
                                                  const float4* hits, QueueView out, ShadowView sh, ShadowView she,
                                                  uint32_t* counters, NrcView nv, const uint32_t* __restrict__ order) {
     const uint32_t part = blockIdx.x % kQueueParts;
@@ -1565,7 +1577,7 @@ __global__ __launch_bounds__(kBlock) void kFeatures(FrameParams fp, SceneView sv
     const uint32_t flags = first ? (MODE == kModeHero ? kFHeroActive : 0u) : pv.flags[q];
     const bool heroActive = MODE == kModeHero && (flags & kFHeroActive) != 0u;
     F4 thr = first ? f4(1.0f) : ld4(pv.thr[q]);
-    F4 misc = heroActive ? f4(0.0f) : (first ? F4{0.0f, 1.0f, 0.0f, 0.0f} : ld4(pv.misc[q]));
+    F4 misc = MODE == kModeHero && !heroActive ? ld4(pv.misc[q]) : f4(0.0f);
     if (flags & kFAbsorption) {
         const F4 sigma = ld4(pv.sigma[q]);
         if (MODE == kModeRgb) {
@@ -1927,7 +1939,7 @@ __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, Sce
             const bool absorbing = (flags & kFAbsorption) != 0u;
             const bool refractive = (flags & kFRefractive) != 0u;
             F4 thr = ld4(pv.thr[q]);
-            F4 misc = ld4(pv.misc[q]);
+            F4 misc = F4{thr.w, 0.0f, 0.0f, 0.0f};
             F4 lr = ld4(pv.rad[q]);
             F3 lrem = F3{lr.x, lr.y, lr.z};
             // dLoss/d(sample radiance) of this path's pixel
@@ -2110,8 +2122,7 @@ __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, Sce
             nextD = wi;
             cont = true;
             pv.rng[q] = storeRng(rng);
-            pv.thr[q] = st4(thr);
-            pv.misc[q] = st4(misc);
+            pv.thr[q] = make_float4(thr.x, thr.y, thr.z, misc.x);
             pv.flags[q] = newFlags;
             if (newFlags & kFAbsorption) pv.sigma[q] = st4(sigma);
             pv.rad[q] = make_float4(lrem.x, lrem.y, lrem.z, 0.0f);
@@ -2137,6 +2148,11 @@ __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, Sce
                 atomicAdd(&av.gEmission[m * 3u + (slot - 4u)], v);
         }
     }
+}
+
+__global__ __launch_bounds__(kBlock) void kBuildMeshFrames(SceneView sv, MeshFrame* out) {
+    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < sv.meshCount) out[i] = buildMeshFrame(sv.meshes[i]);
 }
 
 __global__ __launch_bounds__(kBlock) void kBuildShadeTris(SceneView sv, uint32_t n, ShadeTri* out) {
@@ -2200,13 +2216,18 @@ __global__ __launch_bounds__(kBlock) void kClassScatter(QueueView in, const uint
 // ------------------------------------------------------------- host side --
 static uint32_t blocksFor(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
 
-// Per-triangle shading records, rebuilt after a geometry or mesh upload.
+// Mesh frames and per-triangle shading records, rebuilt after a geometry or mesh upload.
 bool ensureShadeTris(mrt_context* ctx) {
     if (!ctx->shadeTrisDirty) return true;
     uint32_t n = ctx->triCount;
     if (n > 0) {
-        if (!ctx->shadeTris.reserve(n)) return false;
+        const size_t meshes = ctx->meshes.count;
+        if (!ctx->shadeTris.reserve(n) || !ctx->meshFrames.reserve(meshes)) return false;
         ctx->shadeTris.count = n;
+        ctx->meshFrames.count = meshes;
+        hipLaunchKernelGGL(kBuildMeshFrames, dim3(blocksFor(meshes)), dim3(kBlock), 0, ctx->stream, ctx->view(),
+                           ctx->meshFrames.ptr);
+        if (!check(hipGetLastError(), "mesh frames")) return false;
         hipLaunchKernelGGL(kBuildShadeTris, dim3(blocksFor(n)), dim3(kBlock), 0, ctx->stream, ctx->view(), n,
                            ctx->shadeTris.ptr);
         if (!check(hipGetLastError(), "shading records")) return false;
