@@ -79,6 +79,8 @@ struct FrameParams {
     uint32_t count;
     uint32_t numPixels;
     uint32_t vpW;
+    // pathBegin = sampleBase * numPixels + pixelBase, and 2^32 - 1 over the two divisors
+    uint32_t sampleBase, pixelBase, pixelMagic, widthMagic;
     uint32_t accumWidth;
     uint32_t rngPolicy;
     uint64_t rngSeed;
@@ -429,12 +431,35 @@ struct PathStart {
     float jx, jy;
     int px, py;
 };
+// n / d and the remainder for magic = (2^32 - 1) / d: the high product is the
+// quotient or one less
+DEV uint32_t divRem(uint32_t n, uint32_t d, uint32_t magic, uint32_t& rem) {
+    uint32_t q = __umulhi(n, magic);
+    rem = n - q * d;
+    if (rem >= d) {
+        rem -= d;
+        q++;
+    }
+    return q;
+}
+// Sample s and pixel k of path i of the chunk. Images of up to 2^30 pixels (a chunk
+// holds 2^27 paths, so the sum stays in 32 bits) take a 32-bit product for
+// the two 64-bit divisions, some 150 operations that every primary ray pays twice.
+constexpr uint32_t kNarrowPixels = 1u << 30;
+DEV void pathPixel(const FrameParams& fp, uint32_t i, uint32_t& s, uint32_t& k) {
+    if (fp.numPixels <= kNarrowPixels) {
+        s = fp.sampleBase + divRem(fp.pixelBase + i, fp.numPixels, fp.pixelMagic, k);
+    } else {
+        const uint64_t p = fp.pathBegin + i;
+        s = (uint32_t)(p / fp.numPixels);
+        k = (uint32_t)(p % fp.numPixels);
+    }
+}
 template <int MODE>
 DEV PathStart pathStart(const FrameParams& fp, uint32_t i) {
     PathStart ps;
-    uint64_t p = fp.pathBegin + i;
-    uint32_t s = (uint32_t)(p / fp.numPixels);
-    uint32_t k = (uint32_t)(p % fp.numPixels);
+    uint32_t s, k;
+    pathPixel(fp, i, s, k);
     const bool training = fp.nrc && i >= fp.nrcRenderPaths;
     if (training) {
         uint32_t h = (i - fp.nrcRenderPaths) * 0x9E3779B9u ^ (fp.sd.frameNumber * 0x85EBCA6Bu + 0x165667B1u);
@@ -445,8 +470,9 @@ DEV PathStart pathStart(const FrameParams& fp, uint32_t i) {
         h ^= h >> 16;
         k = h % fp.numPixels;
     }
-    ps.px = (int)(fp.sd.viewportRect[0] + k % fp.vpW);
-    ps.py = (int)(fp.sd.viewportRect[1] + k / fp.vpW);
+    uint32_t x, y = divRem(k, fp.vpW, fp.widthMagic, x);
+    ps.px = (int)(fp.sd.viewportRect[0] + x);
+    ps.py = (int)(fp.sd.viewportRect[1] + y);
     float4 prev = fp.accum[(size_t)ps.py * fp.accumWidth + ps.px];
     uint32_t sampleAbs = training ? 0x80000000u + (i - fp.nrcRenderPaths) : (uint32_t)(prev.w + 0.5f) + s;
     ps.rng = rngInit(fp.rngPolicy, fp.rngSeed, ps.px, ps.py, fp.sd.frameNumber, sampleAbs);
@@ -478,7 +504,6 @@ __global__ __launch_bounds__(kBlock) void kGenerate(FrameParams fp, PathView pv,
         uint32_t flags = 0u;
         if (MODE != kModeRgb) pv.lam[i] = st4(ps.lam);
         if (MODE == kModeHero) {
-            pv.radXYZ[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             pv.tpp[i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
             // ptpp / pbtp are read only after a BSDF sample has written them
             flags |= kFHeroActive;
@@ -799,23 +824,22 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
         if (first) ps = pathStart<MODE>(fp, q);
         // first read of the accumulated radiance in this vertex (0 at depth 0 of a lean frame)
         auto radIn = [&]() { return first ? f4(0.0f) : ld4(pv.rad[q]); };
-        auto radXYZIn = [&]() { return first ? f4(0.0f) : ld4(pv.radXYZ[q]); };
         uint32_t flags = first ? (MODE == kModeHero ? kFHeroActive : 0u) : pv.flags[q];
         F4 lam = (MODE != kModeRgb) ? (first ? ps.lam : ld4(pv.lam[q])) : f4(0.0f);
         if (first) {  // what the finalisation and the shadow passes read of every path
-            pv.rad[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (MODE == kModeHero) pv.radXYZ[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (h.tri != kNoHit || fp.neeOnly) pv.rad[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // a miss writes it below
             if (MODE != kModeRgb) pv.lam[q] = st4(lam);
             pv.flags[q] = flags;
         }
         if (MODE == kModeHero && (flags & kFPendingCollapse)) {
             // collapse to the hero wavelength (src/shaders/integrator/path/spectral_hero/transport.slang:77-87),
-            // deferred from the previous vertex until its shadow rays had added their contributions
-            F4 rx = ld4(pv.radXYZ[q]);
-            F3 xyzv = F3{rx.x, rx.y, rx.z} + toXYZ4(ld4(pv.rad[q]), lam, f4(470.0f));
-            pv.radXYZ[q] = make_float4(xyzv.x, xyzv.y, xyzv.z, rx.w);
+            // deferred from the previous vertex until its shadow rays had added their
+            // contributions and the path is known to go on; radXYZ exists from here on
+            F3 xyzv = f3(0.0f) + toXYZ4(ld4(pv.rad[q]), lam, f4(470.0f));
+            pv.radXYZ[q] = make_float4(xyzv.x, xyzv.y, xyzv.z, 0.0f);
             pv.rad[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             flags &= ~kFPendingCollapse;
+            pv.flags[q] = flags;  // this vertex's own shadow rays add to the collapsed radiance
         }
         const bool absorbing = (flags & kFAbsorption) != 0u;
         const bool refractive = (flags & kFRefractive) != 0u;
@@ -857,7 +881,7 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
                     }
                     pv.rad[q] = st4(radIn() + thr * hw * spec4(fp.spec, env, lam));
                 } else {
-                    F4 rx = radXYZIn();
+                    F4 rx = ld4(pv.radXYZ[q]);
                     rx.w += misc.y * (spec1(fp.spec, env, misc.z) * w);
                     pv.radXYZ[q] = st4(rx);
                 }
@@ -1058,7 +1082,7 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
             } else if (heroActive) {
                 pv.rad[q] = st4(radIn() + add);
             } else {
-                F4 rx = radXYZIn();
+                F4 rx = ld4(pv.radXYZ[q]);
                 rx.w += add.x;
                 pv.radXYZ[q] = st4(rx);
             }
@@ -1124,8 +1148,10 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
             if (!(sp > 0.0f)) break;
             F4 weight = val * fabsf(wl.z) / sp;
             if (!anyPos(weight)) break;
-            pv.ptpp[q] = st4(tpp);
-            pv.pbtp[q] = st4(btp);
+            if (fp.neeEnabled || fp.envNee) {  // read only after next-event estimation, to weigh what it could have hit
+                pv.ptpp[q] = st4(tpp);
+                pv.pbtp[q] = st4(btp);
+            }
             tpp = tpp * btp;
             thr = thr * weight;
             if (!anyPos(thr)) break;
@@ -1137,14 +1163,7 @@ DEV void shadeVertex(const FrameParams& fp, uint32_t depth, const SceneView& sv,
                 misc.w = 470.0f;
                 misc.x = btp.x;
                 newFlags &= ~kFHeroActive;
-                if (shadowEmit || envEmit) {
-                    newFlags |= kFPendingCollapse;
-                } else {
-                    F4 rx = ld4(pv.radXYZ[q]);  // this vertex may have added to both already
-                    F3 xyzv = F3{rx.x, rx.y, rx.z} + toXYZ4(ld4(pv.rad[q]), lam, f4(470.0f));
-                    pv.radXYZ[q] = make_float4(xyzv.x, xyzv.y, xyzv.z, rx.w);
-                    pv.rad[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                }
+                newFlags |= kFPendingCollapse;
             }
         } else {
             Eval e = evalScalar<SHEEN>(fp.spec, st, wl);
@@ -1386,13 +1405,11 @@ DEV F3 pathRadiance(const PathView& pv, uint32_t i) {
         F4 l = ld4(pv.lam[i]);
         out = toXYZ1(rad.x, l.x, l.y);
     } else {
-        F4 rx = ld4(pv.radXYZ[i]);
-        out = F3{rx.x, rx.y, rx.z};
-        if (pv.flags[i] & kFHeroActive) {
-            out = out + toXYZ4(rad, ld4(pv.lam[i]), f4(470.0f));
+        if (pv.flags[i] & kFHeroActive) {  // radXYZ is written when the wavelengths collapse
+            out = f3(0.0f) + toXYZ4(rad, ld4(pv.lam[i]), f4(470.0f));
         } else {
-            F4 m = ld4(pv.misc[i]);
-            out = out + toXYZ1(rx.w, m.z, m.w);
+            const F4 rx = ld4(pv.radXYZ[i]), m = ld4(pv.misc[i]);
+            out = F3{rx.x, rx.y, rx.z} + toXYZ1(rx.w, m.z, m.w);
         }
     }
     return out;
@@ -1943,9 +1960,10 @@ __global__ __launch_bounds__(kTraceBlock) void kShadeAdjoint(FrameParams fp, Sce
             F4 lr = ld4(pv.rad[q]);
             F3 lrem = F3{lr.x, lr.y, lr.z};
             // dLoss/d(sample radiance) of this path's pixel
-            const uint64_t pg = fp.pathBegin + q;
-            const uint32_t k = (uint32_t)(pg % fp.numPixels);
-            const uint32_t px = sd.viewportRect[0] + k % fp.vpW, py = sd.viewportRect[1] + k / fp.vpW;
+            uint32_t ps, k, x;
+            pathPixel(fp, q, ps, k);
+            const uint32_t y = divRem(k, fp.vpW, fp.widthMagic, x);
+            const uint32_t px = sd.viewportRect[0] + x, py = sd.viewportRect[1] + y;
             const float* di = av.dImage + ((size_t)py * fp.accumWidth + px) * 3u;
             const F3 dI = F3{di[0], di[1], di[2]} * av.invSpp;
             const F3 t3 = F3{thr.x, thr.y, thr.z};
@@ -2214,6 +2232,14 @@ __global__ __launch_bounds__(kBlock) void kClassScatter(QueueView in, const uint
 }
 
 // ------------------------------------------------------------- host side --
+static void setPathBegin(FrameParams& fp, uint64_t begin) {
+    fp.pathBegin = begin;
+    const uint32_t pixels = std::max(fp.numPixels, 1u), width = std::max(fp.vpW, 1u);
+    fp.sampleBase = (uint32_t)(begin / pixels);
+    fp.pixelBase = (uint32_t)(begin % pixels);
+    fp.pixelMagic = 0xFFFFFFFFu / pixels;
+    fp.widthMagic = 0xFFFFFFFFu / width;
+}
 static uint32_t blocksFor(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
 
 // Mesh frames and per-triangle shading records, rebuilt after a geometry or mesh upload.
@@ -2784,7 +2810,7 @@ extern "C" int mrt_render_frame(mrt_context* ctx, const SceneData* scene, const 
             }
     }
     for (uint64_t begin = 0; begin < totalPaths; begin += chunk) {
-        fp.pathBegin = begin;
+        setPathBegin(fp, begin);
         fp.count = (uint32_t)std::min<uint64_t>(chunk, totalPaths - begin);
         if (fp.nrc) fp.count = (uint32_t)chunk;  // image paths and training paths in one chunk
         const bool sorted = fs.sortShading;
@@ -2929,7 +2955,7 @@ extern "C" int mrt_render_backward(mrt_context* ctx, const SceneData* scene, con
     StageEvents untimed;
     hipEventRecord(ctx->evBegin, s);
     for (uint64_t begin = 0; begin < fs.totalPaths; begin += fs.chunk) {
-        fp.pathBegin = begin;
+        setPathBegin(fp, begin);
         fp.count = (uint32_t)std::min<uint64_t>(fs.chunk, fs.totalPaths - begin);
         // primal: the radiance of every path of the chunk (sampleRad)
         if (!launchChunk<kModeRgb>(ctx, fp, untimed, false, nullptr, true)) return -4;
