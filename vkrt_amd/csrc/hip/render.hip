@@ -790,15 +790,17 @@ __global__ __launch_bounds__(kBlock) void kNrcTargets(const float4* record, cons
 // One path vertex for every ray of the current queue, at three waves per SIMD
 // (at most 168 registers), RGB at four (128): the kernel waits on its gathers and
 // on long chains of dependent arithmetic, so a fourth wave is worth more than the
-// registers (1024x1024 16 spp, next-event estimation, shading of a frame: 5.75 ms at 131
-// registers and three waves, 5.42 with mesh frames and shorter unpacking, 4.64 at four).
-// Every variant must fit its budget without spilling registers to scratch: a hero build that spilled about 60 registers gave wrong
-// NEE results while the same source at two waves matched the oracle bit for
-// bit. What keeps the hero variant inside the budget: the rgb2spec resolution is
-// a compile-time constant, medium coefficients and the scalar-wavelength state
-// are read only where used, and shadow rays are queued before BSDF sampling.
-// Materials with sheen take SHEEN variants, hero at two waves per SIMD and the
-// others at three: the sheen layer does not fit the budgets above.
+// registers (1024x1024 16 spp, next-event estimation, shading of a frame: 5.75 ms
+// at 131 registers and three waves, 5.42 with mesh frames and shorter unpacking,
+// 4.64 at four). Every variant must fit its budget without spilling registers to
+// scratch: a hero build that spilled about 60 registers gave wrong NEE results
+// while the same source at two waves matched the oracle bit for bit. What keeps the
+// hero variant inside the budget: the rgb2spec resolution is a compile-time
+// constant, medium coefficients and the scalar-wavelength state are read only where
+// used, and shadow rays are queued before BSDF sampling. Materials with sheen take
+// SHEEN variants, hero at two waves per SIMD and the others at three: the sheen
+// layer does not fit the budgets above.
+//
 // One path vertex: the ray (ro, rdir) of path q = bits of ro.w, at `depth`,
 // and its hit h. Leaves the continuation ray in nextO / nextD with cont set, or
 // cont false when the path ends here. Shadow records go to the part `part` (one
