@@ -142,17 +142,17 @@ static VKRT_Result syncScene(VKRT* vkrt, int requireDevice) {
         /* packed buffers stay valid until the next change; device initialisation
          * forces a full upload of whatever is prepared by then */
         vkrt->geometryUploaded = vkrt->geometryRevision;
+        vkrt->meshDataUploaded = vkrt->meshDataRevision;
         vkrt->materialUploaded = vkrt->materialRevision;
         vkrt->environmentUploaded = vkrt->environmentRevision;
         return VKRT_SUCCESS;
     }
     PackedScene* p = &vkrt->packed;
     if (geometryDirty) {
-        if (vkrt->meshDataUploaded != vkrt->meshDataRevision) {
+        if (meshDataDirty) {
             mrt_geometry_desc g = {p->vertices,      p->vertexCount,      p->indices,     p->indexCount, p->triangleMesh,
                                    p->triangleCount, p->meshTriangleBase, vkrt->meshCount};
             if (mrt_upload_geometry(vkrt->device, &g) != 0) return deviceError();
-            vkrt->meshDataUploaded = vkrt->meshDataRevision;
         }
         if (mrt_upload_meshes(vkrt->device, p->meshInfos, vkrt->meshCount) != 0) return deviceError();
         float* transforms = (float*)malloc(sizeof(float) * 16u * (vkrt->meshCount ? vkrt->meshCount : 1u));
@@ -201,7 +201,10 @@ static VKRT_Result syncScene(VKRT* vkrt, int requireDevice) {
         }
         if (mrt_upload_environment(vkrt->device, &e) != 0) return deviceError();
     }
+    /* only now, all together: after a step that failed, the next call repeats every
+     * upload that this one was to make */
     vkrt->geometryUploaded = vkrt->geometryRevision;
+    vkrt->meshDataUploaded = vkrt->meshDataRevision;
     vkrt->materialUploaded = vkrt->materialRevision;
     vkrt->environmentUploaded = vkrt->environmentRevision;
     return VKRT_SUCCESS;
