@@ -17,6 +17,13 @@ static const char* kStep[STEPS] = {"geometry", "meshes",   "place",  "build",   
                                    "alpha",    "textures", "lights", "environment"};
 static uint64_t held[STEPS]; /* fingerprint of what each step last uploaded */
 static int failing = -1;
+static long mallocsLeft = -1; /* the malloc after this many fails; negative: none */
+
+void* __real_malloc(size_t size);
+void* __wrap_malloc(size_t size) {
+    if (mallocsLeft >= 0 && mallocsLeft-- == 0) return NULL;
+    return __real_malloc(size);
+}
 
 static uint64_t mix(uint64_t h, const void* data, size_t size) {
     const uint8_t* b = (const uint8_t*)data;
@@ -138,6 +145,29 @@ static void destroy(VKRT* v) {
     VKRT_destroy(v);
 }
 
+/* A batch whose second mesh finds no memory: what the scene then holds is uploaded whole. */
+static int partialBatch(void) {
+    VKRT* v = scene();
+    upload(v);
+    Vertex vertex[3];
+    memset(vertex, 0, sizeof(vertex));
+    vertex[1].position[0] = vertex[2].position[1] = 1.0f;
+    uint32_t index[3] = {0, 1, 2}, count = 0;
+    VKRT_MeshUpload batch[2] = {{vertex, 3, index, 3}, {vertex, 3, index, 3}};
+    mallocsLeft = 2; /* the two arrays of the first mesh */
+    int bad = VKRT_uploadMeshDataBatch(v, batch, 2) != VKRT_ERROR_OUT_OF_MEMORY;
+    mallocsLeft = -1;
+    VKRT_setMeshOpacity(v, 2, 0.25f); /* packs the triangles' alpha words of every mesh again */
+    const float p[3] = {1.0f, 2.0f, 3.0f}, zero[3] = {0.0f, 0.0f, 0.0f}, one[3] = {1.0f, 1.0f, 1.0f};
+    VKRT_setMeshTransform(v, 0, p, zero, one);
+    VKRT_getMeshCount(v, &count);
+    memset(held, 0, sizeof(held));
+    bad |= upload(v) != VKRT_SUCCESS || (count != 3u && held[GEOMETRY] == 0u);
+    if (bad) printf("partial batch: %u meshes, geometry %s\n", count, held[GEOMETRY] ? "uploaded" : "not uploaded");
+    destroy(v);
+    return bad;
+}
+
 int main(void) {
     int differences = 0;
     for (int e = 0; e < EDITS; e++) {
@@ -165,5 +195,5 @@ int main(void) {
             destroy(v);
         }
     }
-    return differences;
+    return differences + partialBatch();
 }

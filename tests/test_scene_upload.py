@@ -16,7 +16,7 @@ def test_a_failed_upload_is_made_whole_by_the_next(tmp_path):
     # the device calls that an upload does not make stay unresolved and unused
     subprocess.run(["gcc", "-O1", "-std=gnu11", "-I", os.path.join(ROOT, "include"), "-I", csrc, "-I",
                     os.path.join(csrc, "host"), os.path.join(ROOT, "tests", "native", "scene_upload.c"),
-                    *sorted(glob.glob(os.path.join(csrc, "host", "*.c"))), "-o", exe,
+                    *sorted(glob.glob(os.path.join(csrc, "host", "*.c"))), "-o", exe, "-Wl,--wrap=malloc",
                     "-Wl,--unresolved-symbols=ignore-all", "-ldl", "-lm", "-lz"], check=True)
     run = subprocess.run([exe], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout + run.stderr

@@ -98,6 +98,7 @@ VKRT_Result VKRT_uploadMeshDataBatch(VKRT* vkrt, const VKRT_MeshUpload* uploads,
         vkrt->meshes = grown;
         vkrt->meshCapacity = cap;
     }
+    const uint32_t before = vkrt->meshCount;
     for (size_t i = 0; i < uploadCount; i++) {
         const VKRT_MeshUpload* u = &uploads[i];
         HostMesh* mesh = &vkrt->meshes[vkrt->meshCount];
@@ -107,7 +108,8 @@ VKRT_Result VKRT_uploadMeshDataBatch(VKRT* vkrt, const VKRT_MeshUpload* uploads,
         if (!mesh->vertices || !mesh->indices) {
             free(mesh->vertices);
             free(mesh->indices);
-            return VKRT_ERROR_OUT_OF_MEMORY;
+            r = VKRT_ERROR_OUT_OF_MEMORY;
+            break;
         }
         memcpy(mesh->vertices, u->vertices, sizeof(Vertex) * u->vertexCount);
         memcpy(mesh->indices, u->indices, sizeof(uint32_t) * u->indexCount);
@@ -121,10 +123,13 @@ VKRT_Result VKRT_uploadMeshDataBatch(VKRT* vkrt, const VKRT_MeshUpload* uploads,
         snprintf(mesh->name, VKRT_NAME_LEN, "Mesh %u", vkrt->meshCount);
         vkrt->meshCount++;
     }
+    /* the meshes before one that found no memory stay, and the packed arrays that
+     * are kept between edits have to grow with them */
+    if (r != VKRT_SUCCESS && vkrt->meshCount == before) return r;
     vkrt->geometryRevision++;
     vkrt->meshDataRevision++;
     vkrtResetSceneData(vkrt);
-    return VKRT_SUCCESS;
+    return r;
 }
 
 VKRT_Result VKRT_uploadMeshData(VKRT* vkrt, const Vertex* vertices, size_t vertexCount, const uint32_t* indices,
