@@ -147,3 +147,31 @@ def test_rays_parallel_to_axis_planes_find_every_hit(axes):
         assert np.array_equal(vis == 1, ~hit)
     finally:
         r.close()
+
+
+def triangle_scene(pos, indices=None):
+    s = scenes.Scene()
+    s.materials = [scenes.lambert((0.5, 0.5, 0.5))]
+    if indices is None:
+        indices = np.arange(len(pos), dtype=np.uint32).reshape(-1, 3)
+    s.meshes.append(scenes.MeshData(V.make_vertices(np.asarray(pos, np.float32), np.tile([[0.0, 0.0, 1.0]], (len(pos), 1))),
+                                    indices, 0))
+    return s
+
+
+def test_hits_behind_the_origin_of_a_thin_scene():
+    """A query's interval may begin before its origin. The scene is thinner than the
+    1e-5 of a distance by which a frame's rays are tested against its box."""
+    pos = [[0.0, 0.0, 0.0], [1.0, 0.0, 3e-4], [0.0, 1.0, 3e-4]]
+    rays = np.tile(np.float32([0.2, 0.2, 100.0, -1000.0, 0.0, 0.0, 1.0, 1000.0]), (70, 1))
+    rays[1::2, 2] = -100.0
+    r = renderer(triangle_scene(pos))
+    try:
+        mesh, prim, t, _ = host = r.trace_rays(rays)
+        assert np.all(mesh == 0) and np.all(prim == 0)
+        # z = 3e-4 * (u + v), rounded to the last place of 100
+        assert np.allclose(t[::2], -100.0 + 1.2e-4, rtol=0.0, atol=2e-5) and np.all(t[1::2] > 100.0)
+        same(host, device_query(r, rays))
+        assert np.all(r.trace_shadow_rays(rays) == 0)
+    finally:
+        r.close()

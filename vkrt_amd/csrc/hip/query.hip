@@ -57,8 +57,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
                 const float4 a = rays[2 * (size_t)i], b = rays[2 * (size_t)i + 1];
                 tmin = a.w;
                 r = makeTraversalRay(xyz(a), xyz(b));
-                // no tree, or the ray misses the scene's box: a miss at once
-                if (sv.nodeCount != 0u && reachesSceneBox(sv, r, tmin, b.w)) {
+                // no tree: a miss at once. The frames' test against the scene's box is left
+                // out: it is for intervals ahead of the origin and unit directions
+                if (sv.nodeCount != 0u) {
                     // a query ray has no path: its index is its key
                     if (ALPHA) alphaKey = alphaRayKey(alphaSalt(0u, 0ull, 0u, 3u), keyBase + i);
                     closestBegin(cs, st, b.w);
