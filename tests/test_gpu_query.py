@@ -175,3 +175,23 @@ def test_hits_behind_the_origin_of_a_thin_scene():
         assert np.all(r.trace_shadow_rays(rays) == 0)
     finally:
         r.close()
+
+
+def test_directions_too_short_for_a_reciprocal_still_slope():
+    """(2e-39, 4e-39, 0): 1 / 2e-39 is infinite, as for a ray parallel to the plane
+    x = 0, but the ray climbs half as fast in x as in y."""
+    pos = [[0.3, 1.0, -0.2], [0.7, 1.0, -0.2], [0.5, 1.0, 0.4]]
+    rays = np.zeros((3, 8), np.float32)
+    rays[:, 4], rays[:, 5], rays[:, 7] = 2e-39, 4e-39, 3.4e38
+    rays[1, 0] = 0.1  # ends at x = 0.6
+    rays[2, 0] = 0.25  # passes the triangle
+    r = renderer(triangle_scene(pos))
+    try:
+        mesh, _, t, _ = host = r.trace_rays(rays)
+        assert np.array_equal(mesh == 0, [True, True, False])
+        # the directions hold 21 bits
+        assert np.allclose(t[:2], np.float32(1.0) / rays[:2, 5], rtol=1e-5)
+        same(host, device_query(r, rays))
+        assert np.array_equal(r.trace_shadow_rays(rays) == 0, mesh == 0)
+    finally:
+        r.close()

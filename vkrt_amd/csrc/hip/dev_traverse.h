@@ -159,7 +159,7 @@ struct TraversalRay {
     F3 inv;      // 1/d
     F3 oInv;     // o/d, so entry distances are plane*inv - oInv
     bool negX, negY, negZ;
-    bool parallel;  // parallel to an axis plane: some component of inv is infinite
+    bool parallel;  // parallel to an axis plane: a component of d is zero wherever one of inv is infinite
     RayPre pre;
 };
 
@@ -172,7 +172,10 @@ DEV TraversalRay makeTraversalRay(F3 o, F3 d) {
     r.negX = d.x < 0.0f;
     r.negY = d.y < 0.0f;
     r.negZ = d.z < 0.0f;
-    r.parallel = __builtin_isinf(r.inv.x) || __builtin_isinf(r.inv.y) || __builtin_isinf(r.inv.z);
+    // a component below 2^-128 has an infinite reciprocal too, but such a ray may still
+    // climb (the others may be as small): it is left to the other axes, as in boxes8
+    const bool ix = __builtin_isinf(r.inv.x), iy = __builtin_isinf(r.inv.y), iz = __builtin_isinf(r.inv.z);
+    r.parallel = (ix || iy || iz) && !(ix && d.x != 0.0f) && !(iy && d.y != 0.0f) && !(iz && d.z != 0.0f);
     r.pre = rayPrecompute(d);
     return r;
 }
