@@ -195,3 +195,25 @@ def test_directions_too_short_for_a_reciprocal_still_slope():
         assert np.array_equal(r.trace_shadow_rays(rays) == 0, mesh == 0)
     finally:
         r.close()
+
+
+def test_a_device_query_cut_off_by_its_visit_limit_fails():
+    """A direction that is not a number meets every box and no triangle, here 4,205,000
+    leaves: more than the 2^22 visits a traversal may make, in a tree too shallow to
+    overflow the stack. The query has not looked everywhere, and says so."""
+    k = 1451
+    x, y = np.meshgrid(np.linspace(0.0, 1.0, k), np.linspace(0.0, 1.0, k), indexing="ij")
+    pos = np.stack([x, y, 0.1 * np.sin(9.0 * x) * np.cos(7.0 * y)], axis=-1).reshape(-1, 3)
+    i = (np.arange(k - 1, dtype=np.uint32)[:, None] * np.uint32(k) + np.arange(k - 1, dtype=np.uint32)).reshape(-1)
+    tris = np.concatenate([np.stack([i, i + 1, i + k], 1), np.stack([i + 1, i + k + 1, i + k], 1)]).astype(np.uint32)
+    rays = np.float32([[0.5, 0.5, 9.0, 1e-3, np.nan, np.nan, np.nan, 20.0], [0.3, 0.6, 9.0, 1e-3, 0.0, 0.0, -1.0, 20.0]])
+    r = renderer(triangle_scene(pos, tris))
+    try:
+        host = r.trace_rays(rays[1:])
+        assert host[0][0] == 0
+        assert r.stats().bvhMaxDepth <= 18  # 18 levels of at most 7 pushes: 128 entries hold them
+        same(host, device_query(r, rays[1:]))
+        with pytest.raises(V.VkrtError):
+            device_query(r, rays)
+    finally:
+        r.close()

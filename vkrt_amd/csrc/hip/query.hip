@@ -203,8 +203,11 @@ extern "C" int mrt_trace_rays_noalloc(mrt_context* ctx, const float* deviceRays,
     const bool own = ctx->traceGrid != 0u && ctx->traversalStack.ptr &&
                      ctx->traversalStack.capacity >= (size_t)ctx->traceGrid * kTraceBlock * kGlobalStackWords;
     uint32_t* stack = own ? ctx->traversalStack.ptr : ctx->noAllocScratch + kNoAllocHeaderWords;
-    // a tree this deep or less cannot overflow the stack, so there is no count to clear and read
-    const bool counted = ctx->bvhMaxDepth * (kBvhWidth - 1u) + 1u > (uint32_t)(kLdsStack + kGlobalStack);
+    // What the count holds: pushes beyond the stack, which a tree of few enough levels cannot
+    // make, and traversals cut off at their visit limit, which a tree of no more nodes and
+    // leaves than that cannot reach. Where neither can be there is nothing to clear and read
+    const bool counted = ctx->bvhMaxDepth * (kBvhWidth - 1u) + 1u > (uint32_t)(kLdsStack + kGlobalStack) ||
+                         ctx->nodes.count + ctx->tris.count > kMaxTraversalSteps;
     if (counted)
         hipLaunchKernelGGL(kClearWords, dim3(1), dim3((uint32_t)kNoAllocHeaderWords), 0, s, ctx->noAllocScratch,
                            (uint32_t)kNoAllocHeaderWords);
@@ -219,7 +222,7 @@ extern "C" int mrt_trace_rays_noalloc(mrt_context* ctx, const float* deviceRays,
         !check(hipMemcpy(&dropped, ctx->noAllocScratch, sizeof(dropped), hipMemcpyDeviceToHost), "read counter"))
         return -4;
     if (dropped) {
-        setError("traversal stack overflow");
+        setError("traversal stack overflow or visit limit");
         return -5;
     }
     return 0;
