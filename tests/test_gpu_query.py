@@ -217,3 +217,25 @@ def test_a_device_query_cut_off_by_its_visit_limit_fails():
             device_query(r, rays)
     finally:
         r.close()
+
+
+def test_a_tree_of_too_many_levels_is_refused():
+    """30,000 coincident triangles cluster into a chain: over 4,200 levels of eight
+    children, more than the build follows. Nothing may be traced through what is left
+    unwritten; the scene without them is traced again."""
+    pos = [[0.0, 0.0, 0.0], [1.0, 0.0, 0.0], [0.0, 1.0, 0.0]]
+    ray = np.float32([[0.2, 0.2, 1.0, 1e-3, 0.0, 0.0, -1.0, 10.0]])
+    s = triangle_scene(pos)
+    s.meshes.append(triangle_scene(pos, np.tile(np.uint32([[0, 1, 2]]), (30_000, 1))).meshes[0])
+    r = renderer(s)
+    try:
+        for trace in (lambda: r.trace_rays(ray), lambda: r.trace_shadow_rays(ray), lambda: device_query(r, ray),
+                      lambda: r.primary_hits(0), r.draw):
+            with pytest.raises(V.VkrtError):
+                trace()
+        assert r.export().triangleCount == 30_001
+        assert r.lib.VKRT_removeMesh(r.h, 1) == 0
+        mesh, prim, t, _ = r.trace_rays(ray)
+        assert (mesh[0], prim[0], t[0]) == (0, 0, 1.0)
+    finally:
+        r.close()

@@ -498,8 +498,10 @@ __global__ __launch_bounds__(kB) void kCollapse(const CollapseItem* in, const ui
     }
 }
 
-// levels[l]: nodes of level l of the collapse (level 0 is the root)
-constexpr uint32_t kMaxLevels = 4096;
+// levels[l]: nodes of level l of the collapse (level 0 is the root). A tree of more
+// levels than this is left unfinished, and nothing may traverse it (bvhComplete).
+constexpr uint32_t kMaxLevels = 4100;
+constexpr uint32_t kLevelBatch = 4;  // levels launched between two looks of the host
 __global__ void kInitCollapse(CollapseItem* items, uint32_t* counts, uint32_t* levels, const uint32_t* root) {
     for (uint32_t i = threadIdx.x; i < kMaxLevels + 2u; i += blockDim.x) levels[i] = i == 0u ? 1u : 0u;
     if (threadIdx.x == 0u) {
@@ -530,6 +532,7 @@ extern "C" int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats) {
         ctx->nodes.count = 0;
         ctx->tris.count = 0;
         ctx->bvhMaxDepth = 0;
+        ctx->bvhComplete = true;
         return 0;
     }
     hipEventRecord(ctx->evStage[0], s);
@@ -641,12 +644,12 @@ extern "C" int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats) {
     // 5: collapse into 8-wide nodes, writing triangle records in leaf order. A level's
     // length is read by the next level's launch; the host looks after every few levels
     hipLaunchKernelGGL(kInitCollapse, dim3(1), dim3(kB), 0, s, front[0], counts, levels, clusters[cur]);
-    uint32_t depth = 0, launched = 0, hostCounts[2] = {1, 0}, lengths[8];
+    uint32_t depth = 0, launched = 0, hostCounts[2] = {1, 0}, lengths[kLevelBatch + 1];
     uint64_t bound = 1;  // of a level's length
+    static_assert(kMaxLevels % kLevelBatch == 0, "levels are launched in whole batches");
     int fc = 0;
     while (launched < kMaxLevels) {
-        const uint32_t batch = 4;
-        for (uint32_t l = 0; l < batch; l++) {
+        for (uint32_t l = 0; l < kLevelBatch; l++) {
             const uint32_t grid = std::min(blocks((size_t)bound * 8u), 8192u);
             hipLaunchKernelGGL(kCollapse, dim3(grid), dim3(kB), 0, s, front[fc], levels + launched, front[1 - fc],
                                levels + launched + 1u, counts, n, children, nodeCounts, boxes, valsSorted,
@@ -656,15 +659,15 @@ extern "C" int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats) {
             launched++;
             bound = std::min<uint64_t>(bound * 8u, n);
         }
-        if (!check(hipMemcpyAsync(lengths, levels + launched - batch, (batch + 1u) * 4u, hipMemcpyDeviceToHost, s),
+        if (!check(hipMemcpyAsync(lengths, levels + launched - kLevelBatch, (kLevelBatch + 1u) * 4u, hipMemcpyDeviceToHost, s),
                    "collapse") ||
             !check(hipMemcpyAsync(hostCounts, counts, sizeof(hostCounts), hipMemcpyDeviceToHost, s), "collapse") ||
             !check(hipStreamSynchronize(s), "collapse sync")) {
             cleanup();
             return -4;
         }
-        for (uint32_t l = 0; l < batch; l++) depth += lengths[l] != 0u;
-        if (lengths[batch] == 0u) break;
+        for (uint32_t l = 0; l < kLevelBatch; l++) depth += lengths[l] != 0u;
+        if (lengths[kLevelBatch] == 0u) break;
     }
     hipEventRecord(ctx->evStage[1], s);
     hipStreamSynchronize(s);
@@ -676,6 +679,7 @@ extern "C" int mrt_build_bvh(mrt_context* ctx, mrt_bvh_stats* stats) {
     ctx->nodes.count = hostCounts[0];
     ctx->tris.count = n;
     ctx->bvhMaxDepth = depth;
+    ctx->bvhComplete = lengths[kLevelBatch] == 0u;
     float ms = 0.0f;
     hipEventElapsedTime(&ms, ctx->evStage[0], ctx->evStage[1]);
     if (stats) {

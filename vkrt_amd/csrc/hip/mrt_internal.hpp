@@ -77,6 +77,9 @@ bool nrcTrainSteps(mrt_context* ctx, const float4* in, uint32_t stride, const fl
                    uint32_t capacity, uint32_t steps, uint32_t batch, float lr);
 float nrcReadLoss(mrt_context* ctx);
 
+// whether rays may be traced at all; sets the error message if not (query.hip)
+bool traceable(const mrt_context* ctx);
+
 // allocation-free ray query (query.hip): resolves its scratch array's device address
 bool noAllocScratchInit(mrt_context* ctx);
 
@@ -127,6 +130,7 @@ struct mrt_context {
     mrt::DeviceArray<float> rgb2spec;
     uint32_t triCount = 0;
     uint32_t bvhMaxDepth = 0;
+    bool bvhComplete = true;  // every node the tree refers to is written
 
     // accumulation
     mrt::DeviceArray<float4> accum;

@@ -109,13 +109,21 @@ static void launchQuery(mrt_context* ctx, const float4* rays, uint32_t n, uint32
 
 using namespace mrt;
 
+// A tree of more levels than the build follows refers to nodes that were never
+// written. Frames refuse far shallower ones (setupFrame).
+bool mrt::traceable(const mrt_context* ctx) {
+    if (ctx->triCount == 0u || ctx->bvhComplete) return true;
+    setError("BVH deeper than the build supports");
+    return false;
+}
+
 // Host queries go through device buffers of the context in pieces of at most
 // kQueryPiece rays (32 bytes in and 20 out per ray: 54 MB), which stay for the next call.
 constexpr size_t kQueryPiece = 1u << 20;
 
 template <bool ANY>
 static int runQuery(mrt_context* ctx, const float* rays, size_t count, const QueryOut& host) {
-    if (!check(hipSetDevice(ctx->device), "hipSetDevice")) return -2;
+    if (!check(hipSetDevice(ctx->device), "hipSetDevice") || !traceable(ctx)) return -2;
     if (!ensureTraversalScratch(ctx)) return -3;
     if (count > 0xFFFFFFFFull / 2) {
         setError("too many rays");
@@ -197,7 +205,7 @@ extern "C" int mrt_trace_rays_noalloc(mrt_context* ctx, const float* deviceRays,
         setError("allocation-free ray query: no device address for its scratch array");
         return -2;
     }
-    if (!check(hipSetDevice(ctx->device), "hipSetDevice")) return -2;
+    if (!check(hipSetDevice(ctx->device), "hipSetDevice") || !traceable(ctx)) return -2;
     if (count == 0) return 0;
     hipStream_t s = ctx->stream;
     const bool own = ctx->traceGrid != 0u && ctx->traversalStack.ptr &&

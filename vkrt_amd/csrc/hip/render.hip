@@ -3036,7 +3036,7 @@ extern "C" int mrt_read_output(mrt_context* ctx, uint16_t* out, size_t count) {
 extern "C" int mrt_primary_hits(mrt_context* ctx, const SceneData* scene, const mrt_render_params* prm,
                                 uint32_t sampleIndex, uint32_t* outMesh, uint32_t* outPrim) {
     if (!ctx || !scene || !prm || !outMesh || !outPrim) return -1;
-    if (!check(hipSetDevice(ctx->device), "hipSetDevice")) return -2;
+    if (!check(hipSetDevice(ctx->device), "hipSetDevice") || !traceable(ctx)) return -2;
     if (!ensureTraversalScratch(ctx)) return -3;
     size_t n = (size_t)scene->viewportRect[2] * scene->viewportRect[3];
     if (n == 0) return 0;
