@@ -116,12 +116,13 @@ VKRT_Result VKRT_setMaterialSorting(VKRT* vkrt, uint8_t enabled);
  * launch carries every remaining path to its end, tracing and shading vertex
  * after vertex per lane, instead of a traversal and a shading launch per depth
  * that each wait for their slowest ray. It takes over at the first depth whose
- * queue held at most maxRays rays (half as many with shadow rays) in the
- * previous frame of the same size and depth, in frames of one chunk whose
- * shading needs none of the neural cache, feature images, material sorting, the
- * alpha test, material textures or sheen; other frames keep their launches per
- * depth. A small frame with shadow rays is all tail (tailStartDepth 0,
- * tailLaunches 1), up to 2^18 paths and maxRays. Results are
+ * queue held at most maxRays rays (half as many with shadow rays) when a frame of
+ * the same size and depth last counted it, in frames of one chunk whose shading
+ * needs none of the neural cache, feature images, material sorting, the alpha
+ * test, material textures or sheen; other frames keep their launches per depth,
+ * and so does a frame whose queues no frame has counted yet. A small frame with
+ * shadow rays is all tail (tailStartDepth 0, tailLaunches 1), up to 2^18 paths
+ * and maxRays. Results are
  * unchanged (every path keeps its random stream and arithmetic). 0 turns it
  * off; default 2^20 rays (about two per lane of the traversal kernel's grid). */
 VKRT_Result VKRT_setFusedTail(VKRT* vkrt, uint32_t maxRays);

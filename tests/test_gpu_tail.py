@@ -165,3 +165,31 @@ def test_fused_tail_with_shadow_rays_gives_the_same_frame(mode, spectral, env, w
         assert st.extensionRays == off.extensionRays and st.shadowRays == off.shadowRays
         assert st.raysBeforeTail + (st.tailRays if st.tailLaunches else 0) == st.extensionRays
         assert np.array_equal(img, ref)
+
+
+def test_depths_that_a_tail_carried_have_no_known_length():
+    """A frame whose tail began at depth 0 has counted no later queue: with a limit
+    below its paths the next frame starts no tail, and the ones after it start where
+    the lengths counted in between allow."""
+    w = h = 64
+    depth, limit = 9, 1600
+    r = V.Renderer(w, h)
+    scenes.load(r, scenes.cornell_box())
+    r.configure(spp=1, max_depth=depth, min_depth=4, mode=V.RENDER_MODE_RGB, rng=V.RNG_PCG32, seed=5)
+    r.start(w, h, 0)
+    stats = []
+    for rays in (1 << 20, limit, limit, limit // 4):
+        r.set_fused_tail(rays)
+        r.draw()
+        stats.append(r.stats())
+    r.close()
+    whole, unknown, known, later = stats
+    assert whole.tailLaunches == 1 and whole.tailStartDepth == 0
+    assert unknown.tailLaunches == 0
+    # shadow rays halve the limit; a tail of n paths traces at most n rays a depth, and the
+    # counts are those of the frame before (a quarter more than 5 of their deviations)
+    assert known.tailLaunches == 1 and known.tailStartDepth > 1
+    assert 0 < known.tailRays <= 1.25 * (limit // 2) * (depth - known.tailStartDepth)
+    # deeper queues keep the lengths of the frame that counted them
+    assert later.tailLaunches == 1 and later.tailStartDepth > known.tailStartDepth
+    assert 0 < later.tailRays <= 1.25 * (limit // 8) * (depth - later.tailStartDepth)

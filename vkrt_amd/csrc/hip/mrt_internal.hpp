@@ -162,8 +162,8 @@ struct mrt_context {
     mrt::DeviceArray<uint32_t> queryOut;
     uint32_t traceGrid = 0;
     uint32_t tailGrid = 0;
-    // queue length of every depth in the last single-chunk frame, with the
-    // chunk size and depth it was measured for: where the fused tail may start
+    // queue length of every depth when a single-chunk frame last counted it, with the
+    // chunk size and depth that they hold for: where the fused tail may start
     uint32_t depthHint[32] = {};
     uint64_t hintPaths = 0;
     uint32_t hintMaxDepth = 0;

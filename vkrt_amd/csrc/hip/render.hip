@@ -2411,6 +2411,7 @@ static void launchShade(hipStream_t s, bool tex, const NrcRun* nrc, const FrameP
 }
 
 constexpr uint32_t kNoTail = 0xFFFFFFFFu;
+constexpr uint32_t kUnknownLength = 0xFFFFFFFFu;  // of a queue that was not counted: no tail begins there
 // Frames with shadow rays of at most this many paths (two per lane of kTail's
 // grid) run as one kTail launch from depth 0: a 256x256 Cornell preview of 1
 // sample takes 0.36 ms so and 0.75 ms with three launches per depth, a 512x512
@@ -2788,14 +2789,16 @@ extern "C" int mrt_render_frame(mrt_context* ctx, const SceneData* scene, const 
         fview = FeatureView{b.featState.ptr, b.featAlbedo.ptr, b.featNormal.ptr, ctx->debug0.ptr, ctx->bounce0.ptr};
     }
     const FeatureView* fv = featurePass ? &fview : nullptr;
-    // The fused tail (kTail) takes over from the first depth whose queue held
-    // at most prm->tailRays rays in the previous frame of the same size: a
-    // single-chunk frame whose shading variant is the plain one (no cache,
-    // features, material sort, alpha test, textures or sheen). A vertex with a
-    // shadow ray is twice the work, so frames with them take over at half that
-    // (961x543 sky, 8 samples, both kinds of sampling: 4.85 ms without a tail, 3.37
-    // and 3.35 at 2^18 and 2^20 rays; 1024x1024 Cornell box, 16 samples: 11.23,
-    // 11.22 and 11.36), and those of at most kWholeFramePaths paths are all tail.
+    // The fused tail (kTail) takes over from the first depth whose queue held at
+    // most prm->tailRays rays when a frame of the same size and depth last counted
+    // it (moved meshes, other materials and modes keep the counts, new meshes do
+    // not; a wrong guess costs time and changes no image): a single-chunk frame
+    // whose shading variant is the plain one (no cache, features, material sort,
+    // alpha test, textures or sheen). A vertex with a shadow ray is twice the
+    // work, so frames with them take over at half that (961x543 sky, 8 samples,
+    // both kinds of sampling: 4.85 ms without a tail, 3.37 and 3.35 at 2^18 and 2^20
+    // rays; 1024x1024 Cornell box, 16 samples: 11.23, 11.22 and 11.36), and
+    // those of at most kWholeFramePaths paths are all tail.
     uint32_t tailDepth = kNoTail;
     const uint32_t maxDepth = scene->rrMaxDepth;
     const SceneView svNow = ctx->view();
@@ -2806,7 +2809,8 @@ extern "C" int mrt_render_frame(mrt_context* ctx, const SceneData* scene, const 
         tailDepth = 0u;
     } else if (tailAllowed && ctx->hintPaths == chunk && ctx->hintMaxDepth == maxDepth) {
         for (uint32_t d = 1; d < std::min<uint32_t>(maxDepth, kDepthHist); d++)
-            if (ctx->depthHint[d] <= (nee ? prm->tailRays / 2u : prm->tailRays)) {
+            if (ctx->depthHint[d] != kUnknownLength &&
+                ctx->depthHint[d] <= (nee ? prm->tailRays / 2u : prm->tailRays)) {
                 tailDepth = d;
                 break;
             }
@@ -2846,9 +2850,17 @@ extern "C" int mrt_render_frame(mrt_context* ctx, const SceneData* scene, const 
         return -5;
     }
     if (totalPaths == chunk && !fp.nrc) {
-        // queue lengths for the next frame's choice of the tail depth (depths
-        // the fused tail carried were not recorded and read as 0)
-        for (uint32_t d = 0; d < (uint32_t)kDepthHist; d++) ctx->depthHint[d] = hostCounters[kCntDepthHist + d];
+        // queue lengths for the next frame's choice of the tail depth. A tail leaves the
+        // depths that it carried on uncounted: those keep the length that the last frame
+        // of this size and depth counted, if one did
+        const uint32_t counted = tailDepth != kNoTail && !countTraversal ? tailDepth + 1u : maxDepth;
+        const bool other = ctx->hintPaths != chunk || ctx->hintMaxDepth != maxDepth;
+        for (uint32_t d = 0; d < (uint32_t)kDepthHist; d++) {
+            if (d < counted)
+                ctx->depthHint[d] = hostCounters[kCntDepthHist + d];
+            else if (other)
+                ctx->depthHint[d] = kUnknownLength;
+        }
         ctx->hintPaths = chunk;
         ctx->hintMaxDepth = maxDepth;
     }

@@ -111,7 +111,7 @@ typedef struct mrt_render_params {
     uint32_t materialSort; /* shade each depth's hits grouped by material class */
     uint32_t features;     /* accumulate the denoiser albedo / normal feature images */
     uint32_t tailRays;     /* fused tail from the first depth whose queue held at most this many rays
-                              in the previous frame (0: every depth is its own pair of launches) */
+                              when last counted (0: every depth is its own launches) */
 } mrt_render_params;
 
 typedef struct mrt_render_stats {
