@@ -160,10 +160,13 @@ def test_fused_tail_with_shadow_rays_gives_the_same_frame(mode, spectral, env, w
             continue
         img, st = shadowed_frames(lit_glass_under_sky(), w, h, spp, mode, spectral, rays, env)
         whole = paths <= min(rays, 1 << 18)
-        assert st.tailLaunches == (1 if whole or st.tailStartDepth else 0)
-        assert (st.tailLaunches == 1 and st.tailStartDepth == 0) == whole
+        # the second frame always ends in a tail: the queue of depth 1 is below 2^19 in
+        # every case, and half of half the paths are left after a few depths
+        assert st.tailLaunches == 1
+        assert st.tailStartDepth == 0 if whole else st.tailStartDepth == 1 if rays == 1 << 20 else st.tailStartDepth > 1
+        assert st.tailRays > 0 or paths < 100
         assert st.extensionRays == off.extensionRays and st.shadowRays == off.shadowRays
-        assert st.raysBeforeTail + (st.tailRays if st.tailLaunches else 0) == st.extensionRays
+        assert st.raysBeforeTail + st.tailRays == st.extensionRays
         assert np.array_equal(img, ref)
 
 
