@@ -128,3 +128,64 @@ def test_moved_meshes_and_changed_materials_match_a_fresh_scene():
             assert np.array_equal(draw(r), want)
     finally:
         r.close()
+
+
+def placed_scene():
+    """Meshes turned, stretched, mirrored, sheared, moved far and shrunk to thin slivers."""
+    rng = np.random.default_rng(23)
+    s = scenes.Scene()
+    s.materials = [scenes.lambert((0.5, 0.5, 0.5))]
+    linear = [np.eye(3), np.diag([0.3, 2.0, 1.1]), np.diag([-1.0, 1.0, 0.7]), np.diag([1.0, 1e-3, 1.0])]
+    linear += [rng.normal(size=(3, 3)) for _ in range(4)]
+    for k, a in enumerate(linear):
+        q = np.linalg.qr(rng.normal(size=(3, 3)))[0]
+        m = np.eye(4)
+        m[:3, :3] = q @ a
+        m[:3, 3] = [2.0 * (k % 4) + (100.0 if k == 7 else 0.0), 2.0 * (k // 4), 0.3 * k]
+        count = 70 + 57 * k  # not whole blocks, and meshes that share one
+        pos = soup(count, k)
+        index = rng.permutation(3 * count).astype(np.uint32).reshape(-1, 3)
+        s.meshes.append(scenes.MeshData(V.make_vertices(pos, np.tile([[0.0, 0.0, 1.0]], (len(pos), 1))), index, 0, m))
+    return s
+
+
+def test_the_device_places_the_triangles_that_an_export_shows():
+    """The same rays through a scene of transformed meshes, whose triangles the device
+    places, and through the exported triangles themselves as meshes that are not
+    transformed: the same hits to the last bit. Corners one last place further off
+    are told apart."""
+    s = placed_scene()
+    r = renderer(s)
+    try:
+        exported = r.export()
+        n = exported.triangleCount
+        tris = np.ctypeslib.as_array(exported.worldTriangles, (n * 9,)).copy().reshape(n, 3, 3)
+        rng = np.random.default_rng(24)
+        w = rng.dirichlet([1.0, 1.0, 1.0], n)[:, :, None].astype(np.float32)
+        target = np.repeat((tris * w).sum(1), 3, axis=0)
+        d = rng.normal(size=target.shape)
+        d /= np.linalg.norm(d, axis=1, keepdims=True)
+        rays = np.zeros((len(d), 8), np.float32)
+        rays[:, :3], rays[:, 4:7], rays[:, 3], rays[:, 7] = target - 3.0 * d, d, 1e-3, 1e4
+        placed = r.trace_rays(rays)
+        assert np.mean(placed[0] != V.VKRT_INVALID_INDEX) > 0.5
+    finally:
+        r.close()
+
+    def flat(corners):
+        f, first = scenes.Scene(), 0
+        f.materials = s.materials
+        for mesh in s.meshes:
+            pos = corners[first:first + len(mesh.indices)].reshape(-1, 3)
+            first += len(mesh.indices)
+            f.meshes.append(scenes.MeshData(V.make_vertices(pos, np.tile([[0.0, 0.0, 1.0]], (len(pos), 1))),
+                                            np.arange(len(pos), dtype=np.uint32).reshape(-1, 3), 0))
+        g = renderer(f)
+        try:
+            return g.trace_rays(rays)
+        finally:
+            g.close()
+
+    for a, b in zip(placed, flat(tris)):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert np.mean(placed[2] != flat(np.nextafter(tris, np.float32(np.inf)))[2]) > 0.1
