@@ -10,6 +10,8 @@ from vkrt_amd import scenes
 
 pytestmark = pytest.mark.gpu
 
+torch = pytest.importorskip("torch")
+
 
 def same_seed(scene, w, h, spp, mode, depth=6):
     r = V.Renderer(w, h)
@@ -46,3 +48,27 @@ def test_lights_seen_past_a_collapse_count():
     gpu, ref = same_seed(s, 64, 64, 16, V.RENDER_MODE_SPECTRAL, depth=3)
     # the bound of the same-seed parity tests (a lost contribution shows in 3 of 12,288 values)
     assert np.mean(np.abs(gpu - ref) <= 1e-4 * (1.0 + np.abs(ref))) > 0.9999
+
+
+@pytest.mark.parametrize("mode,spectral,nee,size", [
+    # random state, flags, throughput, radiance, medium, hit, sample, two queues of two 16-byte records
+    (V.RENDER_MODE_RGB, V.SPECTRAL_HERO, False, 164),
+    (V.RENDER_MODE_SPECTRAL, V.SPECTRAL_SINGLE, False, 180),  # and the wavelength
+    (V.RENDER_MODE_SPECTRAL, V.SPECTRAL_HERO, False, 228),  # and collapsed state and radiance, pdfs
+    (V.RENDER_MODE_SPECTRAL, V.SPECTRAL_HERO, True, 324),  # and the last vertex's pdfs, shadow rays
+])
+def test_a_path_takes_the_memory_that_its_mode_uses(mode, spectral, nee, size):
+    r = V.Renderer(256, 256)
+    try:
+        scenes.load(r, scenes.cornell_box())
+        r.configure(spp=1, max_depth=3, min_depth=2, mode=mode, spectral=spectral, rng=V.RNG_PCG32, seed=4, nee=nee)
+        r.start(256, 256, 0)
+        r.draw()
+        before = torch.cuda.mem_get_info()[0]
+        r.configure(spp=65)
+        r.draw()
+        grown = before - torch.cuda.mem_get_info()[0]
+        # some twenty allocations, of whole pages; a record of 16 bytes per path is 65 MiB
+        assert abs(grown - 65 * 256 * 256 * size) < 16 << 20
+    finally:
+        r.close()

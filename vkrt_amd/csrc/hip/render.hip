@@ -2295,7 +2295,7 @@ bool ensureTraversalScratch(mrt_context* ctx) {
 static bool ensurePaths(mrt_context* ctx, size_t n, int mode, bool lightShadows, bool envShadows) {
     PathBuffers& b = ctx->paths;
     const size_t slots = (size_t)queueBlocks(n) * kBlock;  // of a queue of up to n paths
-    bool ok = b.rng.reserve(n) && b.flags.reserve(n) && b.thr.reserve(n) && b.rad.reserve(n) && b.misc.reserve(n) &&
+    bool ok = b.rng.reserve(n) && b.flags.reserve(n) && b.thr.reserve(n) && b.rad.reserve(n) &&
               b.sigma.reserve(n) && b.hits.reserve(slots) && b.sampleRad.reserve(n);
     for (int qi = 0; qi < 2; qi++)
         for (int j = 0; j < 2; j++) ok = ok && b.rays[qi][j].reserve(slots);
@@ -2304,8 +2304,9 @@ static bool ensurePaths(mrt_context* ctx, size_t n, int mode, bool lightShadows,
     if (envShadows)
         for (int j = 0; j < 3; j++) ok = ok && b.shadowEnv[j].reserve(slots);
     if (mode != kModeRgb) ok = ok && b.lam.reserve(n);
-    if (mode == kModeHero)
-        ok = ok && b.radXYZ.reserve(n) && b.tpp.reserve(n) && b.ptpp.reserve(n) && b.pbtp.reserve(n);
+    if (mode == kModeHero) ok = ok && b.misc.reserve(n) && b.radXYZ.reserve(n) && b.tpp.reserve(n);
+    // touched only where next-event estimation is on, of lights or of the environment
+    if (mode == kModeHero && (lightShadows || envShadows)) ok = ok && b.ptpp.reserve(n) && b.pbtp.reserve(n);
     return ok;
 }
 
