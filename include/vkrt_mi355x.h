@@ -61,7 +61,7 @@ typedef struct VKRT_TraceStats {
     float backwardMs;       /* device time of the last VKRT_renderBackward (primal + replay) */
     float extendMsDepth0;   /* the part of extendMs spent on the primary rays (depth 0) */
     float shadeMsDepth0;    /* the part of shadeMs spent on the primary hits and misses (depth 0) */
-    uint32_t tailStartDepth; /* depth from which the fused tail carried the paths (0: none) */
+    uint32_t tailStartDepth; /* depth from which the fused tail carried the paths; 0: none, or with tailLaunches all */
     uint32_t tailLaunches;
     float tailMs;            /* fused tail kernel time; not part of extendMs or shadeMs */
     uint64_t tailRays;       /* extension rays the fused tail traced (part of extensionRays) */
@@ -265,10 +265,12 @@ VKRT_Result VKRT_traceShadowRays(VKRT* vkrt, const float* rays, size_t count, ui
  * deviceT / deviceBarycentrics are device pointers on the context's GPU,
  * laid out as in VKRT_traceRays; results are bit-identical to it. The
  * traversal stacks are the context's own once it has drawn a frame or answered
- * a host query; until then, and for the count of a stack overflow, one fixed
+ * a host query; until then, and for the count of searches cut short, one fixed
  * device array of the library (about 61 MB per GPU, held until the process
  * ends) serves every call on that GPU: calls that overlap on one GPU race. At most 2^30
- * rays per call (VKRT_ERROR_INVALID_ARGUMENT beyond). The scene must already
+ * rays per call (VKRT_ERROR_INVALID_ARGUMENT beyond). A search cut short, by the
+ * depth of the stack or after 2^22 visits, fails the call
+ * (VKRT_ERROR_OPERATION_FAILED). The scene must already
  * be on the device (VKRT_ERROR_OPERATION_FAILED when it changed since the
  * last upload, as uploading allocates). Returns after the results are
  * written. */

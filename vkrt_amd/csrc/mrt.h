@@ -134,7 +134,7 @@ typedef struct mrt_render_stats {
     float nrcTrainMs;
     float extendMsDepth0;  /* the part of extendMs / shadeMs spent on the paths' first rays */
     float shadeMsDepth0;
-    uint32_t tailStartDepth;   /* depth from which the fused tail kernel carried the paths (0: none) */
+    uint32_t tailStartDepth;   /* depth from which the fused tail kernel carried the paths (0 and no tailLaunches: none) */
     uint32_t tailLaunches;
     float tailMs;
     uint64_t tailRays;         /* extension rays the fused tail traced */
@@ -196,9 +196,11 @@ int mrt_primary_hits(mrt_context* ctx, const SceneData* scene, const mrt_render_
                      uint32_t* outMesh, uint32_t* outPrim);
 
 /* mrt_trace_rays on device memory with no allocation: rays and outputs are
- * device pointers; the traversal stacks and the overflow counter live in a
- * fixed device array of the library. Calls that overlap on one device race
- * on that array. At most MRT_NOALLOC_MAX_RAYS rays per call. */
+ * device pointers. The traversal stacks are the context's own once a frame or a
+ * host query has made them; until then, and for the count of searches cut short
+ * (which fail the call), a fixed device array of the library serves every
+ * context. Calls that overlap on one device race on what they share. At most
+ * MRT_NOALLOC_MAX_RAYS rays per call. */
 #define MRT_NOALLOC_MAX_RAYS (1ull << 30)
 int mrt_trace_rays_noalloc(mrt_context* ctx, const float* deviceRays, size_t count, uint32_t* deviceMesh,
                            uint32_t* devicePrim, float* deviceT, float* deviceBary);
