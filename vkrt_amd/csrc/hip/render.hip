@@ -36,9 +36,9 @@ constexpr uint32_t kFPendingCollapse = 16u;
 constexpr uint32_t kFPrevEnvNee = 32u;  // the previous vertex sampled the environment for NEE
 
 // Paths in flight per chunk. Large enough that the queues of late bounces
-// (after most paths have ended) still fill the chip: 2^27 paths keep about
-// 40 GB of path state and queues resident, well inside 288 GB of HBM (a
-// 1080p frame of 64 samples is one chunk).
+// (after most paths have ended) still fill the chip: 2^27 paths keep 31 GB of
+// path state and queues resident in hero mode (50 with both kinds of shadow
+// rays), well inside 288 GB of HBM (a 1080p frame of 64 samples is one chunk).
 constexpr uint64_t kMaxChunk = 1ull << 27;
 constexpr int kBlock = 256;
 
@@ -574,10 +574,12 @@ __global__ void kTailSnapshot(uint32_t* counters) {
 // Closest-hit traversal, persistent with lane refill. Every loop iteration
 // advances each busy lane by one node or leaf visit; once kRefillLanes lanes of
 // a wavefront are idle they take new rays (RayClaims), so lanes do not wait for
-// the slowest ray of a batch. What bounds it in scenes of many triangles is the
-// latency of the node loads: letting lanes with a leaf wait until 8, 16 or 24 of
-// them could test their triangles together halved the leaf steps and still
-// took 23.2, 23.0 and 24.2 against 22.0 ms per 1080p spectral frame.
+// the slowest ray of a batch. What bounds it while its queue is long is the issue
+// of vector instructions: 1.16 per SIMD and four cycles on the primary rays of the
+// 1080p spectral frame, more than loops of multiply-adds (0.97) or of compares and
+// selects (1.03) reach, with half of the lanes off. Letting lanes with a leaf wait
+// until 8, 16 or 24 of them could test their triangles together halved the leaf steps
+// and still took 23.2, 23.0 and 24.2 against 22.0 ms per frame.
 // COUNT adds the number of BVH nodes visited and triangles tested to the frame statistics.
 
 // ALPHA: some mesh runs the alpha test (the opaque variant keeps six waves per SIMD);
